@@ -48,22 +48,32 @@ class LogprobGather(torch.autograd.Function):
 
 class GrpoFusedLoss(torch.autograd.Function):
     """Loss of the whole GRPO step from bf16 logits (forward: one streaming pass;
-    backward: d loss / d logits = g * dlp * (onehot - softmax))."""
+    backward: d loss / d logits = g * dlp * (onehot - softmax)).  With ``shift``
+    the last position's logits take no part; their gradient rows are zeros,
+    written beside the others' (a slice of the logits outside would have autograd
+    fill and copy a second ``[B, T, V]`` gradient)."""
 
     @staticmethod
-    def forward(ctx, logits, ids, old_lp, mask, rewards, prompt_ids, adv_eps, clip, reduction):
-        res = K.grpo_fused_forward(logits, ids, old_lp, mask, rewards, prompt_ids, adv_eps, clip,
-                                   reduction)
+    def forward(ctx, logits, ids, old_lp, mask, rewards, prompt_ids, adv_eps, clip, reduction,
+                shift=False):
+        res = K.grpo_fused_forward(logits[:, :-1] if shift else logits, ids, old_lp, mask, rewards,
+                                   prompt_ids, adv_eps, clip, reduction)
         ctx.save_for_backward(logits, ids, res["lse"], res["dlp"])
         ctx.mark_non_differentiable(res["lp"], res["adv"])
+        ctx.shift = shift
         return res["loss"], res["lp"], res["adv"]
 
     @staticmethod
     def backward(ctx, grad_loss, _glp, _gadv):
         logits, ids, lse, dlp = ctx.saved_tensors
         g = grad_loss.reshape(1).float().contiguous()
-        grad = K.logprob_gather_backward(logits, ids, lse, dlp, grad_scale=g)
-        return grad, None, None, None, None, None, None, None, None
+        none = (None,) * 9
+        if not ctx.shift:
+            return (K.logprob_gather_backward(logits, ids, lse, dlp, grad_scale=g), *none)
+        grad = torch.empty(logits.shape, dtype=logits.dtype, device=logits.device)
+        K.logprob_gather_backward(logits[:, :-1], ids, lse, dlp, grad_scale=g, out=grad[:, :-1])
+        grad[:, -1].zero_()
+        return (grad, *none)
 
 
 class PpoClippedLoss(torch.autograd.Function):
@@ -164,11 +174,11 @@ def grpo_fused_loss(logits, ids, old_log_probs, response_mask, rewards, prompt_i
     old_log_probs / response_mask then refer to positions 1..T-1.
     """
     if shift:
-        logits, ids = logits[:, :-1], ids[:, 1:]
+        ids = ids[:, 1:]
         old_log_probs = old_log_probs[:, 1:]
         response_mask = response_mask[:, 1:]
     return GrpoFusedLoss.apply(logits, ids, old_log_probs, response_mask, rewards, prompt_ids,
-                               adv_eps, clip_epsilon, reduction)
+                               adv_eps, clip_epsilon, reduction, shift)
 
 
 def grpo_fused_train_step(model, optimizer, input_ids, old_log_probs, response_mask, rewards,
