@@ -334,20 +334,6 @@ int qmi_silu_mul_backward(const uint16_t* gate_up, int64_t gate_up_stride, const
                           int64_t dgate_up_stride, void* stream);
 
 /*
- * Gradient of the lm_head's input: dx[n_rows, hidden] = dy[n_rows, vocab]
- * w[vocab, hidden] in bf16 with fp32 sums (the backward of lm_head,
- * qwen3_naive.py:840).  The vocabulary is split over the chip: for few rows
- * (n_rows x hidden much smaller than the vocabulary).  vocab % 64 == 0,
- * hidden % 8 == 0; rows 16-byte aligned, strides % 8 == 0.  workspace: fp32,
- * qmi_head_backward_workspace_bytes bytes, contents ignored.
- */
-int64_t qmi_head_backward_workspace_bytes(int64_t n_rows, int64_t hidden, int64_t vocab);
-int qmi_head_backward_input(const uint16_t* dy, int64_t dy_stride, const uint16_t* w,
-                            int64_t w_stride, int64_t n_rows, int64_t hidden, int64_t vocab,
-                            uint16_t* dx, int64_t dx_stride, float* workspace,
-                            int64_t workspace_bytes, void* stream);
-
-/*
  * Causal GQA attention of a training batch: batch sequences of seq_len tokens
  * each, rows token-major ([batch * seq_len] rows of num_heads * 128 bf16
  * elements, row strides in elements).  Replaces the fp32 attention core of

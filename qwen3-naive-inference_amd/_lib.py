@@ -88,9 +88,6 @@ SIGNATURES: dict[str, tuple] = {
         _c_p, _c_i64, _c_p]),                           # workspace, bytes, stream
     "qmi_silu_mul_backward": (ctypes.c_int, [_c_p, _c_i64, _c_p, _c_i64, _c_i64, _c_i64, _c_p,
                                              _c_i64, _c_p]),
-    "qmi_head_backward_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
-    "qmi_head_backward_input": (ctypes.c_int, [_c_p, _c_i64, _c_p, _c_i64, _c_i64, _c_i64, _c_i64,
-                                               _c_p, _c_i64, _c_p, _c_i64, _c_p]),
     "qmi_train_attn_forward": (ctypes.c_int, [
         _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64,       # q, k, v with strides
         _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_f32, # batch, seq_len, heads, head_dim, scale

@@ -559,23 +559,6 @@ def silu_mul_backward(gate_up: torch.Tensor, dy: torch.Tensor) -> torch.Tensor:
     return out.view(gate_up.shape)
 
 
-def head_backward_input(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """``dy @ weight`` for ``dy [M, V]``, ``weight [V, H]``: the gradient of the
-    lm_head's input, summed over the vocabulary in ranges."""
-    dy, weight = _rows2d("dy", dy), _weight16(weight)
-    n, v = dy.shape
-    h = weight.shape[1]
-    dx = torch.empty((n, h), dtype=torch.bfloat16, device=dy.device)
-    L = lib()
-    nbytes = L.qmi_head_backward_workspace_bytes(n, h, v)
-    ws = torch.empty((max(nbytes, 16) // 4,), dtype=torch.float32, device=dy.device)
-    check(L.qmi_head_backward_input(dy.data_ptr(), dy.stride(0), weight.data_ptr(),
-                                    weight.stride(0), n, h, v, dx.data_ptr(), dx.stride(0),
-                                    ws.data_ptr(), ws.numel() * 4, stream_handle(dy.device)),
-          "head_backward_input")
-    return dx
-
-
 def train_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, batch: int,
                     softmax_scale: float, need_grad: bool):
     """Causal GQA attention of ``batch`` whole sequences, fp32 probabilities:

@@ -90,11 +90,11 @@ def _decode_linear(proj: nn.Linear, x: torch.Tensor, parts: bool = False):
     return proj(x)
 
 
-def _unhooked(*modules: nn.Module, cls=None) -> bool:
-    """Whether calling these modules runs RMSNorm.forward (``cls``'s) and nothing
-    else, so that a fused kernel may compute them from their weights."""
+def _unhooked(*modules: nn.Module) -> bool:
+    """Whether calling these norms runs RMSNorm.forward and nothing else, so
+    that a fused kernel may compute them from their weights."""
     return not nn.modules.module._has_any_global_hook() and all(
-        type(m) is (cls or RMSNorm) and "forward" not in m.__dict__ and not m._forward_hooks
+        type(m) is RMSNorm and "forward" not in m.__dict__ and not m._forward_hooks
         and not m._forward_pre_hooks and not m._backward_hooks and not m._backward_pre_hooks
         for m in modules)
 
@@ -400,11 +400,7 @@ class Qwen3ForCausalLM(nn.Module):
         self._preempted: set = set()
 
     def forward(self, x):
-        h, head = self.model(x), self.lm_head
-        if (torch.is_grad_enabled() and h.requires_grad and _unhooked(head, cls=nn.Linear)
-                and head.bias is None and T.head_ok(h, head.weight)):
-            return T.HeadLinear.apply(h, head.weight)
-        return head(h)
+        return self.lm_head(self.model(x))
 
     # ---------------- KV pool (qwen3_naive.py:994-1066) ----------------
     def kv_block_bytes(self) -> int:

@@ -225,38 +225,3 @@ def attention_ok(qkv, q_weight, k_weight, cache, num_heads, num_kv_heads) -> boo
             and cache.dtype == torch.float32 and cache.is_contiguous()
             and cache.data_ptr() % 16 == 0 and cache.shape[1] == K.HEAD_DIM
             and qkv.shape[1] <= cache.shape[0] and qkv.shape[0] <= 65535)
-
-
-# ---------------------------------------------------------------------------
-# lm_head (qwen3_naive.py:840)
-# ---------------------------------------------------------------------------
-def head_ok(hidden, weight) -> bool:
-    """Whether ``HeadLinear`` takes this product: its backward kernel is for sums
-    over a vocabulary much longer than the hidden size."""
-    return (kernels_ok(hidden, weight) and weight.dim() == 2 and hidden.numel() > 0
-            and hidden.shape[-1] == weight.shape[1] and weight.shape[0] % 64 == 0
-            and weight.shape[1] % 8 == 0 and weight.shape[0] >= 8 * weight.shape[1]
-            and weight.stride(1) == 1 and weight.shape[1] <= 65536
-            and weight.shape[0] <= 1 << 22
-            and hidden.numel() // hidden.shape[-1] <= 65536)
-
-
-class HeadLinear(torch.autograd.Function):
-    """``hidden @ weight.T`` with the split-vocabulary kernel for the gradient of
-    ``hidden``."""
-
-    @staticmethod
-    def forward(ctx, hidden, weight):
-        ctx.save_for_backward(hidden, weight)
-        return torch.nn.functional.linear(hidden, weight)
-
-    @staticmethod
-    def backward(ctx, dy):
-        hidden, weight = ctx.saved_tensors
-        dh = dw = None
-        if ctx.needs_input_grad[0]:
-            dh = (dy @ weight if torch.is_grad_enabled() else
-                  K.head_backward_input(dy, weight).view(hidden.shape))
-        if ctx.needs_input_grad[1]:
-            dw = dy.reshape(-1, dy.shape[-1]).t() @ hidden.reshape(-1, hidden.shape[-1])
-        return dh, dw

@@ -104,3 +104,22 @@ def test_train_steps_update_parameters(pkg, gpu):
     l2 = pkg.grpo_fused_train_step(m, opt, ids, old, mask, rewards, pids)
     assert all(map(lambda v: v == v and abs(v) < 1e3, (l1, l2)))
     assert not torch.equal(before, m.model.layers[0].mlp.down_proj.weight)
+
+
+@pytest.mark.parametrize("t", [2, 9])
+def test_shifted_loss_gradient(pkg, gpu, t):
+    """shift=True gives the loss and gradient of the sliced logits, zeros at the last position."""
+    g = torch.Generator(device=gpu).manual_seed(t)
+    logits = torch.randn(4, t, 1000, generator=g, device=gpu).bfloat16().requires_grad_()
+    ids = torch.randint(0, 1000, (4, t), generator=g, device=gpu)
+    old = -7.0 + 0.1 * torch.randn(4, t, generator=g, device=gpu)
+    mask = (torch.rand(4, t, generator=g, device=gpu) < 0.8).float()
+    mask[:, 1] = 1
+    rewards = torch.rand(4, generator=g, device=gpu)
+    groups = torch.tensor([0, 0, 1, 1], device=gpu)
+    a = pkg.grpo_fused_loss(logits, ids, old, mask, rewards, groups, shift=True)
+    ga, = torch.autograd.grad(a[0], logits)
+    b = pkg.grpo_fused_loss(logits[:, :-1], ids[:, 1:], old[:, 1:], mask[:, 1:], rewards, groups)
+    gb, = torch.autograd.grad(b[0], logits)
+    assert all(torch.equal(x, y) for x, y in zip(a, b))
+    assert gb.abs().max() > 0 and torch.equal(ga, gb) and bool((ga[:, -1] == 0).all())

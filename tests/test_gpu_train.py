@@ -206,62 +206,3 @@ def test_layer_gradients_twice_and_sum_only(pkg, gpu):
     _, s = T.AddRmsNorm.apply(x, r, w, 1e-6)
     gx, gr = torch.autograd.grad(s, (x, r), torch.ones_like(s))
     assert bool((gx == 1).all()) and bool((gr == 1).all())
-
-
-# Rows around both tile heights, a hidden size that is not a multiple of the
-# tile's 256 columns, the fewest vocabulary chunks, and one that does not divide
-# into equal ranges.
-@pytest.mark.parametrize("rows,hidden,vocab", [
-    (1, 64, 512), (128, 1024, 8192), (129, 264, 4160), (256, 8, 64), (300, 512, 151936), (778, 1024, 64 * 131)])
-def test_head_input_gradient(pkg, gpu, rows, hidden, vocab):
-    g = torch.Generator(device=gpu).manual_seed(rows)
-    dy = torch.randn(rows, vocab, generator=g, device=gpu).bfloat16()
-    w = torch.randn(vocab, hidden, generator=g, device=gpu).bfloat16()
-    got = pkg.kernels.head_backward_input(dy, w)
-    assert _rel(got, dy.double() @ w.double()) < BF16
-    assert torch.equal(got, pkg.kernels.head_backward_input(dy, w))
-
-
-def test_head_gradients_in_the_model(pkg, gpu):
-    """The model's logits go through HeadLinear when a gradient is wanted, and a
-    hooked lm_head is called as a module; both give the library product's gradients."""
-    torch.manual_seed(0)
-    m = pkg.Qwen3ForCausalLM(pkg.Qwen3Config(
-        hidden_size=128, num_attention_heads=2, num_key_value_heads=1, intermediate_size=256,
-        num_hidden_layers=1, vocab_size=2048, max_position_embeddings=64,
-        tie_word_embeddings=False)).to(gpu).bfloat16()
-    ids = torch.randint(0, 2048, (2, 33), device=gpu)
-    res = []
-    for hook in (False, True):
-        h = m.lm_head.register_forward_hook(lambda *_: None) if hook else None
-        m.zero_grad()
-        y = m(ids)
-        assert ("HeadLinear" in type(y.grad_fn).__name__) != hook
-        y.float().square().mean().backward()
-        res.append([y.detach()] + [p.grad for p in m.parameters()])
-        if h:
-            h.remove()
-    assert torch.equal(res[0][0], res[1][0])
-    for got, want in zip(*res):
-        assert _rel(got, want.double()) < 0.01
-    with torch.no_grad():
-        assert torch.equal(m(ids), res[0][0])
-
-
-@pytest.mark.parametrize("t", [2, 9])
-def test_shifted_loss_gradient(pkg, gpu, t):
-    """shift=True gives the loss and gradient of the sliced logits, zeros at the last position."""
-    g = torch.Generator(device=gpu).manual_seed(t)
-    logits = torch.randn(4, t, 1000, generator=g, device=gpu).bfloat16().requires_grad_()
-    ids = torch.randint(0, 1000, (4, t), generator=g, device=gpu)
-    old = -7.0 + 0.1 * torch.randn(4, t, generator=g, device=gpu)
-    mask = (torch.rand(4, t, generator=g, device=gpu) < 0.8).float()
-    mask[:, 1] = 1
-    rewards = torch.rand(4, generator=g, device=gpu)
-    groups = torch.tensor([0, 0, 1, 1], device=gpu)
-    a = pkg.grpo_fused_loss(logits, ids, old, mask, rewards, groups, shift=True)
-    ga, = torch.autograd.grad(a[0], logits)
-    b = pkg.grpo_fused_loss(logits[:, :-1], ids[:, 1:], old[:, 1:], mask[:, 1:], rewards, groups)
-    gb, = torch.autograd.grad(b[0], logits)
-    assert all(torch.equal(x, y) for x, y in zip(a, b))
-    assert gb.abs().max() > 0 and torch.equal(ga, gb) and bool((ga[:, -1] == 0).all())
