@@ -16,26 +16,23 @@ namespace {
 
 using namespace qmi;
 
-// out[c] = bf16(sum_p parts[p][c]): 32 columns x 32 partial-row groups per
-// workgroup (2,048 partial rows are then 64 loads deep; 4.9 us, latency);
-// columns below n0 go to out0, the others to out1.
-constexpr int kSumGroups = 32;
-__global__ __launch_bounds__(32 * kSumGroups) void sum_columns(const float* __restrict__ parts, int n_parts, int n,
-                                                               int n0, uint16_t* __restrict__ out0,
-                                                               uint16_t* __restrict__ out1) {
-  __shared__ float sm[kSumGroups][33];
+// out[c] = bf16(sum_p parts[p][c]): 32 columns x 8 partial-row groups per
+// workgroup; columns below n0 go to out0, the others to out1.
+__global__ __launch_bounds__(256) void sum_columns(const float* __restrict__ parts, int n_parts, int n, int n0,
+                                                   uint16_t* __restrict__ out0, uint16_t* __restrict__ out1) {
+  __shared__ float sm[8][32];
   const int lane = threadIdx.x & 31, grp = threadIdx.x >> 5;
   const int c = blockIdx.x * 32 + lane;
   float s = 0.f;
   if (c < n) {
 #pragma unroll 8
-    for (int p = grp; p < n_parts; p += kSumGroups) s += parts[(int64_t)p * n + c];
+    for (int p = grp; p < n_parts; p += 8) s += parts[(int64_t)p * n + c];
   }
   sm[grp][lane] = s;
   __syncthreads();
   if (grp == 0 && c < n) {
 #pragma unroll
-    for (int i = 1; i < kSumGroups; ++i) s += sm[i][lane];
+    for (int i = 1; i < 8; ++i) s += sm[i][lane];
     if (c < n0)
       out0[c] = f32_to_bf16(s);
     else
@@ -49,9 +46,7 @@ __global__ __launch_bounds__(32 * kSumGroups) void sum_columns(const float* __re
 // (4s + i, 64 + 4s + i).  The rotation's transpose gives the normalised
 // head's gradient g; with x^ = x / rms, dw += g x^ and
 // dx = (g w - x^ mean(g w x^)) / rms (the norm's bf16 rounding passes the
-// gradient through unchanged).  Bound by the memory latency of its one-item
-// groups: 8 workgroups per CU and 32-bit index arithmetic took 5,120 tokens
-// (94 MB) from 41 us (2 per CU, 64-bit division) to 22 us, 4.2 TB/s.
+// gradient through unchanged).
 __global__ __launch_bounds__(256) void qk_norm_rope_backward_kernel(
     const uint16_t* __restrict__ dq, int64_t dq_stride, const uint16_t* __restrict__ dk, int64_t dk_stride,
     const uint16_t* __restrict__ qkv, int64_t qkv_stride, int n_q_heads, int n_kv_heads,
@@ -62,14 +57,13 @@ __global__ __launch_bounds__(256) void qk_norm_rope_backward_kernel(
   __shared__ float sm[4][2][D];
   const int sub = threadIdx.x & 15, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int heads = n_q_heads + n_kv_heads;
-  const int n_items = (int)n_tok * heads, step = gridDim.x * 16;
+  const int64_t n_items = n_tok * heads, step = (int64_t)gridDim.x * 16;
   float aw[2][8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) aw[0][i] = aw[1][i] = 0.f;
-#pragma unroll 2
-  for (int item = blockIdx.x * 16 + (threadIdx.x >> 4); item < n_items; item += step) {
-    const int itok = (int)((unsigned)item / (unsigned)heads), h = item - itok * heads;
-    const int64_t tok = itok;
+  for (int64_t item = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4); item < n_items; item += step) {
+    const int64_t tok = item / heads;
+    const int h = (int)(item - tok * heads);
     const bool is_q = h < n_q_heads;
     const uint16_t* src = qkv + tok * qkv_stride + (int64_t)h * D;
     const uint16_t* w = is_q ? q_w : k_w;
@@ -81,7 +75,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_backward_kernel(
     const uint2 gb = *reinterpret_cast<const uint2*>(go + HALF + 4 * sub);
     const uint2 wa = *reinterpret_cast<const uint2*>(w + 4 * sub);
     const uint2 wb = *reinterpret_cast<const uint2*>(w + HALF + 4 * sub);
-    const float* cs = cos_sin + (int64_t)((unsigned)itok % (unsigned)seq_len) * D;
+    const float* cs = cos_sin + (int64_t)((uint32_t)tok % (uint32_t)seq_len) * D;
     const float4 c = *reinterpret_cast<const float4*>(cs + 4 * sub);
     const float4 sn = *reinterpret_cast<const float4*>(cs + HALF + 4 * sub);
     const float x1[4] = {bf16_lo(xa.x), bf16_hi(xa.x), bf16_lo(xa.y), bf16_hi(xa.y)};
@@ -261,10 +255,9 @@ __global__ __launch_bounds__(256) void silu_mul_backward_kernel(const uint16_t* 
 
 inline bool al(const void* p, unsigned n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }
 
-// Partial rows of a launch: `per_cu` workgroups per CU, fewer when the rows run out.
-int64_t part_rows(int64_t units, int64_t per_workgroup, int per_cu) {
-  return std::max<int64_t>(1,
-                           std::min<int64_t>(per_cu * device_cu_count(), (units + per_workgroup - 1) / per_workgroup));
+// Partial rows of a launch: two workgroups per CU, fewer when the rows run out.
+int64_t part_rows(int64_t units, int64_t per_workgroup) {
+  return std::max<int64_t>(1, std::min<int64_t>(2 * device_cu_count(), (units + per_workgroup - 1) / per_workgroup));
 }
 
 }  // namespace
@@ -272,7 +265,7 @@ int64_t part_rows(int64_t units, int64_t per_workgroup, int per_cu) {
 extern "C" int64_t qmi_qk_norm_rope_backward_workspace_bytes(int64_t n_tok, int64_t num_q_heads,
                                                              int64_t num_kv_heads) {
   if (n_tok <= 0 || num_q_heads <= 0 || num_kv_heads <= 0) return 0;
-  return part_rows(n_tok * (num_q_heads + num_kv_heads), 16, 8) * 256 * 4;
+  return part_rows(n_tok * (num_q_heads + num_kv_heads), 16) * 256 * 4;
 }
 
 extern "C" int qmi_qk_norm_rope_backward(const uint16_t* dq, int64_t dq_stride, const uint16_t* dk, int64_t dk_stride,
@@ -287,7 +280,7 @@ extern "C" int qmi_qk_norm_rope_backward(const uint16_t* dq, int64_t dq_stride, 
   if (!dq || !dk || !qkv || !q_norm_weight || !k_norm_weight || !cos_sin_cache || !dqkv || !dq_norm_weight ||
       !dk_norm_weight || !workspace)
     return QMI_E_NULL_POINTER;
-  if (head_dim != 128 || n_tok * (num_q_heads + num_kv_heads) > 0x7fff0000LL || seq_len > 0x7fffffffLL || num_q_heads > 4096 || num_kv_heads > 4096)
+  if (head_dim != 128 || n_tok > 0x7fffffffLL || seq_len > 0x7fffffffLL || num_q_heads > 4096 || num_kv_heads > 4096)
     return QMI_E_UNSUPPORTED;
   const int64_t width = (num_q_heads + num_kv_heads) * 128;
   if (dq_stride % 4 || dk_stride % 4 || qkv_stride % 4 || dqkv_stride % 4 || !al(dq, 8) || !al(dk, 8) ||
@@ -295,20 +288,20 @@ extern "C" int qmi_qk_norm_rope_backward(const uint16_t* dq, int64_t dq_stride, 
       !al(workspace, 4) || qkv_stride < width || dqkv_stride < width || dq_stride < num_q_heads * 128 ||
       dk_stride < num_kv_heads * 128)
     return QMI_E_BAD_STRIDE;
-  const int64_t parts = part_rows(n_tok * (num_q_heads + num_kv_heads), 16, 8);
+  const int64_t parts = part_rows(n_tok * (num_q_heads + num_kv_heads), 16);
   if (workspace_bytes < parts * 256 * 4) return QMI_E_WORKSPACE_TOO_SMALL;
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   hipLaunchKernelGGL(qk_norm_rope_backward_kernel, dim3((unsigned)parts), dim3(256), 0, st, dq, dq_stride, dk,
                      dk_stride, qkv, qkv_stride, (int)num_q_heads, (int)num_kv_heads, q_norm_weight, k_norm_weight,
                      cos_sin_cache, (int)seq_len, n_tok, eps, dqkv, dqkv_stride, workspace);
-  hipLaunchKernelGGL(sum_columns, dim3(8), dim3(32 * kSumGroups), 0, st, workspace, (int)parts, 256, 128, dq_norm_weight,
+  hipLaunchKernelGGL(sum_columns, dim3(8), dim3(256), 0, st, workspace, (int)parts, 256, 128, dq_norm_weight,
                      dk_norm_weight);
   QMI_RETURN_LAUNCH_STATUS();
 }
 
 extern "C" int64_t qmi_rms_norm_backward_workspace_bytes(int64_t n_rows, int64_t n) {
   if (n_rows <= 0 || n <= 0) return 0;
-  return part_rows(n_rows, 4, 2) * n * 4;
+  return part_rows(n_rows, 4) * n * 4;
 }
 
 extern "C" int qmi_rms_norm_backward(const uint16_t* x, int64_t x_stride, const uint16_t* residual,
@@ -323,7 +316,7 @@ extern "C" int qmi_rms_norm_backward(const uint16_t* x, int64_t x_stride, const 
   if (x_stride % 8 || residual_stride % 8 || dy_stride % 8 || dsum_stride % 8 || dx_stride % 8 || !al(x, 16) ||
       !al(residual, 16) || !al(weight, 16) || !al(dy, 16) || !al(dsum, 16) || !al(dx, 16) || !al(workspace, 4))
     return QMI_E_BAD_STRIDE;
-  const int64_t parts = part_rows(n_rows, 4, 2);
+  const int64_t parts = part_rows(n_rows, 4);
   if (workspace_bytes < parts * n * 4) return QMI_E_WORKSPACE_TOO_SMALL;
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   auto launch = [&](auto kernel) {
@@ -338,7 +331,7 @@ extern "C" int qmi_rms_norm_backward(const uint16_t* x, int64_t x_stride, const 
     launch(rms_norm_backward_rows<4>);
   else
     launch(rms_norm_backward_rows<8>);
-  hipLaunchKernelGGL(sum_columns, dim3((unsigned)((n + 31) / 32)), dim3(32 * kSumGroups), 0, st, workspace, (int)parts, (int)n,
+  hipLaunchKernelGGL(sum_columns, dim3((unsigned)((n + 31) / 32)), dim3(256), 0, st, workspace, (int)parts, (int)n,
                      (int)n, dweight, nullptr);
   QMI_RETURN_LAUNCH_STATUS();
 }

@@ -219,7 +219,6 @@ def attention_ok(qkv, q_weight, k_weight, cache, num_heads, num_kv_heads) -> boo
     """Whether ``QkvAttention`` takes this batch."""
     return (kernels_ok(qkv, q_weight, k_weight) and qkv.dim() == 3 and qkv.numel() > 0
             and num_heads % num_kv_heads == 0 and num_heads <= 4096
-            and qkv.shape[0] * qkv.shape[1] * (num_heads + num_kv_heads) <= 0x7fff0000
             and qkv.shape[2] == (num_heads + 2 * num_kv_heads) * K.HEAD_DIM
             and q_weight.shape == k_weight.shape == (K.HEAD_DIM,)
             and cache.dtype == torch.float32 and cache.is_contiguous()
