@@ -15,8 +15,8 @@
 //     results;
 //   * the row dot products delta = dO . O use the fp32 output.
 //
-// Three kernels, all of one shape: a workgroup of W = 4 or 8 waves keeps 16 rows
-// per wave (the forward 16 J) as MFMA B operands in registers (queries, or keys for dK / dV) and
+// Three kernels, all of one shape: a workgroup of 4 waves keeps 16 rows per
+// wave (the forward 16 J) as MFMA B operands in registers (queries, or keys for dK / dV) and
 // streams 64-row tiles of the other side through LDS, double-buffered, each
 // staged once for all waves.  A tile is read two ways: rows as the A operand
 // of the first products (ds_read_b128) and, transposed by ds_read_b64_tr_b16,
@@ -35,14 +35,13 @@
 // kernel with atomic dQ would, and give the same bits on every run.
 //
 // What bounds them: the causal products are small beside the projections
-// (8 x 640 tokens, 16 heads: 20 GFLOP with the split forward, 67 backward), and
-// no unit is busy more than a third of the time: it is the chain score -> exp
-// -> split -> product of a wave, its VALU work (7 instructions per MFMA) and the
-// uneven causal blocks.  Two waves per SIMD hide part of it, which the register
-// budget is kept to (the forward at 296 registers and one wave: 64.7 us instead
-// of 48.5; dQ and dK / dV with 32 rows per wave, one wave per SIMD: 177 us
-// instead of 136).  Measured at 8 x 640: forward 48 us, dQ + dK / dV 131 us,
-// where the torch core took 2.4 ms.
+// (8 x 640 tokens, 16 heads: 20 GFLOP with the split forward, 67 backward), so
+// the chain score -> exp -> split -> product of a wave is; two waves per SIMD
+// hide it, which the register budget is kept to (the forward at 296 registers
+// and one wave: 64.7 us instead of 48.5).  With 32 rows per wave each LDS
+// operand feeds two MFMAs; in the backward kernels that takes them to one wave
+// per SIMD (8 x 640: 177 us instead of 136).  Measured at 8 x 640: forward
+// 48.5 us, dQ + dK / dV 136 us, where the torch core took 2.4 ms.
 #include <algorithm>
 
 #include "qmi_common.h"
@@ -52,46 +51,36 @@ namespace {
 using namespace qmi;
 
 constexpr int kD = 128;
+constexpr int kThreads = 256;
 constexpr int kTile = 64;
 constexpr int kTileElems = kTile * kD;
 typedef __attribute__((ext_vector_type(4))) short v4s_t;
 
-// Chunk swizzle of row r (only r % 16 matters).  Chunk pairs (swz / 2) are a
-// bijection of rows 0-7 and of rows 8-15, for the transpose reads; rows 4-7
-// and 8-11 use the same pairs, because a ds_read_b128 serves lanes 0-3, 12-15
-// and 20-27 together (rows 0-3 and 12-15 at one chunk, rows 4-11 at its
-// neighbour).  With the plain bijection half of the row reads' cycles were
-// bank conflicts.
-__device__ __forceinline__ int swz(int r) {
-  const int hi = (r >> 3) & 1;
-  return (((r & 7) ^ (hi << 2)) << 1) | hi;
-}
+// Chunk swizzle of row r (only r % 16 matters).
+__device__ __forceinline__ int swz(int r) { return ((r & 3) << 1) | ((r & 4) << 1) | ((r >> 3) & 1); }
 
-// A 64-row tile in flight: 16 / W chunks of 16 bytes per thread of W waves.
-template <int W>
+// A 64-row tile in flight: 4 chunks of 16 bytes per thread.
 struct Stage {
-  uint4 v[16 / W];
+  uint4 v[4];
 };
 
 // Rows r0 .. r0+63 of `base` (row stride in elements); rows at or past n are zeros.
-template <int W>
-__device__ __forceinline__ Stage<W> load_tile(const uint16_t* __restrict__ base, int64_t stride, int r0, int n) {
-  Stage<W> s;
+__device__ __forceinline__ Stage load_tile(const uint16_t* __restrict__ base, int64_t stride, int r0, int n) {
+  Stage s;
   const int rr = threadIdx.x >> 4, ch = threadIdx.x & 15;
 #pragma unroll
-  for (int i = 0; i < 16 / W; ++i) {
-    const int r = r0 + rr + 4 * W * i;
+  for (int i = 0; i < 4; ++i) {
+    const int r = r0 + rr + 16 * i;
     s.v[i] = r < n ? load_u4(base + (int64_t)r * stride + 8 * ch) : make_uint4(0, 0, 0, 0);
   }
   return s;
 }
 
-template <int W>
-__device__ __forceinline__ void store_tile(uint16_t* lds, const Stage<W>& s) {
+__device__ __forceinline__ void store_tile(uint16_t* lds, const Stage& s) {
   const int rr = threadIdx.x >> 4, ch = threadIdx.x & 15;
 #pragma unroll
-  for (int i = 0; i < 16 / W; ++i)
-    *reinterpret_cast<uint4*>(lds + (rr + 4 * W * i) * kD + 8 * (ch ^ swz(rr))) = s.v[i];
+  for (int i = 0; i < 4; ++i)
+    *reinterpret_cast<uint4*>(lds + (rr + 16 * i) * kD + 8 * (ch ^ swz(rr))) = s.v[i];
 }
 
 // A operand: rows 16 kb + l16, dims 32 c + 8 g4 ..+8.
@@ -116,18 +105,14 @@ __device__ __forceinline__ f32x4_t mfma(bf16x8_t a, bf16x8_t b, f32x4_t c) {
 
 // Elements of row blocks 2c, 2c+1 as hi + lo bf16 B operands.
 __device__ __forceinline__ void split_operand(const f32x4_t& a, const f32x4_t& b, bf16x8_t& hi, bf16x8_t& lo) {
-  typedef __attribute__((ext_vector_type(2))) float f32x2_t;
-  uint32_t h[4], l[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {  // two elements per conversion
-    const f32x4_t& v = i < 2 ? a : b;
-    const float x = v[2 * (i & 1)], y = v[2 * (i & 1) + 1];
-    h[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{x, y}), bf16x2_t));
-    l[i] = __builtin_bit_cast(
-        uint32_t, __builtin_convertvector((f32x2_t{x - bf16_lo(h[i]), y - bf16_hi(h[i])}), bf16x2_t));
+  for (int r = 0; r < 4; ++r) {
+    const __bf16 ha = (__bf16)a[r], hb = (__bf16)b[r];
+    hi[r] = ha;
+    hi[4 + r] = hb;
+    lo[r] = (__bf16)(a[r] - (float)ha);
+    lo[4 + r] = (__bf16)(b[r] - (float)hb);
   }
-  hi = __builtin_bit_cast(bf16x8_t, u32x4_t{h[0], h[1], h[2], h[3]});
-  lo = __builtin_bit_cast(bf16x8_t, u32x4_t{l[0], l[1], l[2], l[3]});
 }
 
 // The wave's 16 rows from r0 as B operands (rows at or past n are zeros).
@@ -149,21 +134,6 @@ __device__ __forceinline__ void store_row_bf16(uint16_t* __restrict__ dst, const
         make_uint2(pack_bf16x2(acc[db][0] * f, acc[db][1] * f), pack_bf16x2(acc[db][2] * f, acc[db][3] * f));
 }
 
-// Adds the accumulators of waves 4-7 to those of waves 0-3 through 32 KB of
-// LDS that no wave reads any more (16 bytes per lane, conflict-free).
-__device__ __forceinline__ void add_halves(float* lds, f32x4_t (&acc)[8], int wave, int lane) {
-  f32x4_t* p = reinterpret_cast<f32x4_t*>(lds) + (wave & 3) * 8 * 64 + lane;
-  if (wave >= 4) {
-#pragma unroll
-    for (int db = 0; db < 8; ++db) p[64 * db] = acc[db];
-  }
-  __syncthreads();
-  if (wave < 4) {
-#pragma unroll
-    for (int db = 0; db < 8; ++db) acc[db] += p[64 * db];
-  }
-}
-
 struct AttnArgs {
   const uint16_t *q, *k, *v;
   int64_t q_ts, k_ts, v_ts;  // token strides (elements); heads are 128 apart
@@ -183,23 +153,20 @@ struct AttnArgs {
 // Blocks: x = query head with the KV head fastest (with 8 KV heads a KV head
 // stays on one XCD and its K / V in that XCD's L2), y = sequence, z = query
 // block, the long late blocks first.
-template <int J, int W>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) void train_attn_forward(const AttnArgs a) {
-  constexpr int kParts = W / 4, NK = 4 / kParts;  // parts of a tile's keys, 16-key blocks of a part
-  __shared__ __attribute__((aligned(16))) uint16_t tiles[2][2][kTileElems];
-  uint16_t(*const sK)[kTileElems] = tiles[0];
-  uint16_t(*const sV)[kTileElems] = tiles[1];
+template <int J>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void train_attn_forward(const AttnArgs a) {
+  __shared__ __attribute__((aligned(16))) uint16_t sK[2][kTileElems], sV[2][kTileElems];
   const int lane = threadIdx.x & 63, l16 = lane & 15, g4 = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wave >> 2;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int G = a.Hq / a.Hkv, kvh = blockIdx.x % a.Hkv, h = kvh * G + blockIdx.x / a.Hkv, b = blockIdx.y;
-  const int q0 = (gridDim.z - 1 - blockIdx.z) * (64 * J), wq0 = q0 + (wave & 3) * 16 * J;
+  const int q0 = (gridDim.z - 1 - blockIdx.z) * (64 * J), wq0 = q0 + wave * 16 * J;
   const int T = a.T;
   const int64_t tok0 = (int64_t)b * T;
   const uint16_t* qb = a.q + tok0 * a.q_ts + h * kD;
   const uint16_t* kb0 = a.k + tok0 * a.k_ts + kvh * kD;
   const uint16_t* vb0 = a.v + tok0 * a.v_ts + kvh * kD;
   const int kend = min(q0 + 64 * J, T), n_tiles = (kend + kTile - 1) / kTile;
-  Stage<W> ks = load_tile<W>(kb0, a.k_ts, 0, T), vs = load_tile<W>(vb0, a.v_ts, 0, T);
+  Stage ks = load_tile(kb0, a.k_ts, 0, T), vs = load_tile(vb0, a.v_ts, 0, T);
   bf16x8_t qop[J][4];
 #pragma unroll
   for (int j = 0; j < J; ++j) load_rows(qb, a.q_ts, wq0 + 16 * j, T, l16, g4, qop[j]);
@@ -219,36 +186,36 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
     const int buf = t & 1;
     const bool more = t + 1 < n_tiles;
     if (more) {
-      ks = load_tile<W>(kb0, a.k_ts, (t + 1) * kTile, T);
-      vs = load_tile<W>(vb0, a.v_ts, (t + 1) * kTile, T);
+      ks = load_tile(kb0, a.k_ts, (t + 1) * kTile, T);
+      vs = load_tile(vb0, a.v_ts, (t + 1) * kTile, T);
     }
-    f32x4_t s[J][NK];
+    f32x4_t s[J][4];
 #pragma unroll
-    for (int kb = 0; kb < NK; ++kb) {
+    for (int kb = 0; kb < 4; ++kb) {
 #pragma unroll
       for (int j = 0; j < J; ++j) s[j][kb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const bf16x8_t op = row_operand(sK[buf], NK * half + kb, c, l16, g4);
+        const bf16x8_t op = row_operand(sK[buf], kb, c, l16, g4);
 #pragma unroll
         for (int j = 0; j < J; ++j) s[j][kb] = mfma(op, qop[j][c], s[j][kb]);
       }
     }
-    const int key0 = t * kTile + 16 * NK * half;
-    const bool full = key0 + 16 * NK - 1 <= wq0;  // every key visible to every query of the wave
-    bf16x8_t hi[J][NK / 2], lo[J][NK / 2];
+    const int key0 = t * kTile;
+    const bool full = key0 + kTile - 1 <= wq0;  // every key visible to every query of the wave
+    bf16x8_t hi[J][2], lo[J][2];
 #pragma unroll
     for (int j = 0; j < J; ++j) {
       if (!full) {
         const int lim = wq0 + 16 * j + l16 - key0 - 4 * g4;  // key 16 kb + r visible iff <= lim
 #pragma unroll
-        for (int kb = 0; kb < NK; ++kb)
+        for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
           for (int r = 0; r < 4; ++r) s[j][kb][r] = 16 * kb + r <= lim ? s[j][kb][r] : -INFINITY;
       }
       float mx = -INFINITY;
 #pragma unroll
-      for (int kb = 0; kb < NK; ++kb)
+      for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
         for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[j][kb][r]);
       mx = rows4_max(mx) * a.scale_log2;
@@ -263,25 +230,23 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
         for (int db = 0; db < 8; ++db) acc[j][db] *= alpha;
       }
-      // A part of a tile can hold no key of a query yet: exp2(-inf - 0) = 0.
-      const float neg_m = m_run[j] == -INFINITY ? 0.f : -m_run[j];
       float sum = 0.f;
 #pragma unroll
-      for (int kb = 0; kb < NK; ++kb)
+      for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          s[j][kb][r] = fast_exp2(fmaf(s[j][kb][r], a.scale_log2, neg_m));
+          s[j][kb][r] = fast_exp2(fmaf(s[j][kb][r], a.scale_log2, -m_run[j]));
           sum += s[j][kb][r];
         }
       l_run[j] += sum;
 #pragma unroll
-      for (int c = 0; c < NK / 2; ++c) split_operand(s[j][2 * c], s[j][2 * c + 1], hi[j][c], lo[j][c]);
+      for (int c = 0; c < 2; ++c) split_operand(s[j][2 * c], s[j][2 * c + 1], hi[j][c], lo[j][c]);
     }
 #pragma unroll
     for (int db = 0; db < 8; ++db)
 #pragma unroll
-      for (int c = 0; c < NK / 2; ++c) {
-        const bf16x8_t op = col_operand(sV[buf], NK / 2 * half + c, db, l16, g4);
+      for (int c = 0; c < 2; ++c) {
+        const bf16x8_t op = col_operand(sV[buf], c, db, l16, g4);
 #pragma unroll
         for (int j = 0; j < J; ++j) {
           acc[j][db] = mfma(op, lo[j][c], acc[j][db]);
@@ -294,67 +259,33 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
     }
     __syncthreads();
   }
-  float inv[J];
-#pragma unroll
-  for (int j = 0; j < J; ++j) {
-    l_run[j] = rows4_sum(l_run[j]);
-    inv[j] = 1.0f / l_run[j];
-  }
-  if constexpr (kParts == 2) {
-    // The two halves of the keys meet: common maximum, rescaled sums.  A half
-    // that saw no key of a query (its maximum still -inf) adds nothing.
-    float* sf = reinterpret_cast<float*>(tiles);
-    float2(*const s_ml)[64] = reinterpret_cast<float2(*)[64]>(sf);
-#pragma unroll
-    for (int j = 0; j < J; ++j) s_ml[wave * J + j][lane] = make_float2(m_run[j], l_run[j]);
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const float2 o = s_ml[(wave ^ 4) * J + j][lane];
-      const float m = fmaxf(m_run[j], o.x);
-      const float f = m_run[j] == -INFINITY ? 0.f : fast_exp2(m_run[j] - m);
-      const float fo = o.x == -INFINITY ? 0.f : fast_exp2(o.x - m);
-      inv[j] = 1.0f / (l_run[j] * f + o.y * fo);
-      m_run[j] = m;
-#pragma unroll
-      for (int db = 0; db < 8; ++db) acc[j][db] *= f;
-    }
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      __syncthreads();
-      add_halves(sf, acc[j], wave, lane);
-    }
-    if (half) return;
-  }
 #pragma unroll
   for (int j = 0; j < J; ++j) {
     const int qi = wq0 + 16 * j + l16;
+    const float inv = 1.0f / rows4_sum(l_run[j]);
     if (qi >= T) continue;
-    store_row_bf16(a.out + (tok0 + qi) * a.out_ts + h * kD, acc[j], inv[j], g4);
+    store_row_bf16(a.out + (tok0 + qi) * a.out_ts + h * kD, acc[j], inv, g4);
     if (a.out32) {
       float* o = a.out32 + ((tok0 + qi) * a.Hq + h) * kD + 4 * g4;
 #pragma unroll
-      for (int db = 0; db < 8; ++db) *reinterpret_cast<f32x4_t*>(o + 16 * db) = acc[j][db] * inv[j];
-      if (g4 == 0) a.stat[((int64_t)b * a.Hq + h) * T + qi] = make_float2(m_run[j], inv[j]);
+      for (int db = 0; db < 8; ++db) *reinterpret_cast<f32x4_t*>(o + 16 * db) = acc[j][db] * inv;
+      if (g4 == 0) a.stat[((int64_t)b * a.Hq + h) * T + qi] = make_float2(m_run[j], inv);
     }
   }
 }
 
-template <int W>
-__global__ __launch_bounds__(64 * W) void train_attn_dq(const AttnArgs a) {
-  __shared__ __attribute__((aligned(16))) uint16_t tiles[2][2][kTileElems];
-  uint16_t(*const sK)[kTileElems] = tiles[0];
-  uint16_t(*const sV)[kTileElems] = tiles[1];
+__global__ __launch_bounds__(kThreads) void train_attn_dq(const AttnArgs a) {
+  __shared__ __attribute__((aligned(16))) uint16_t sK[2][kTileElems], sV[2][kTileElems];
   const int lane = threadIdx.x & 63, l16 = lane & 15, g4 = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wave >> 2;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int G = a.Hq / a.Hkv, kvh = blockIdx.x % a.Hkv, h = kvh * G + blockIdx.x / a.Hkv, b = blockIdx.y;
-  const int q0 = (gridDim.z - 1 - blockIdx.z) * 64, wq0 = q0 + (wave & 3) * 16;
+  const int q0 = (gridDim.z - 1 - blockIdx.z) * 64, wq0 = q0 + wave * 16;
   const int T = a.T;
   const int64_t tok0 = (int64_t)b * T;
   const uint16_t* kb0 = a.k + tok0 * a.k_ts + kvh * kD;
   const uint16_t* vb0 = a.v + tok0 * a.v_ts + kvh * kD;
   const int kend = min(q0 + 64, T), n_tiles = (kend + kTile - 1) / kTile;
-  Stage<W> ks = load_tile<W>(kb0, a.k_ts, 0, T), vs = load_tile<W>(vb0, a.v_ts, 0, T);
+  Stage ks = load_tile(kb0, a.k_ts, 0, T), vs = load_tile(vb0, a.v_ts, 0, T);
   bf16x8_t qop[4], dop[4];
   f32x4_t acc[8];
   const int qi = wq0 + l16;
@@ -375,7 +306,7 @@ __global__ __launch_bounds__(64 * W) void train_attn_dq(const AttnArgs a) {
     }
   }
   const float delta = rows4_sum(d);
-  if (half == 0 && qi < T && g4 == 0) a.delta[si] = delta;
+  if (qi < T && g4 == 0) a.delta[si] = delta;
 #pragma unroll
   for (int db = 0; db < 8; ++db) acc[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   store_tile(sK[0], ks);
@@ -385,22 +316,23 @@ __global__ __launch_bounds__(64 * W) void train_attn_dq(const AttnArgs a) {
     const int buf = t & 1;
     const bool more = t + 1 < n_tiles;
     if (more) {
-      ks = load_tile<W>(kb0, a.k_ts, (t + 1) * kTile, T);
-      vs = load_tile<W>(vb0, a.v_ts, (t + 1) * kTile, T);
+      ks = load_tile(kb0, a.k_ts, (t + 1) * kTile, T);
+      vs = load_tile(vb0, a.v_ts, (t + 1) * kTile, T);
     }
+    const int key0 = t * kTile;
+    const bool full = key0 + kTile - 1 <= wq0;
+    bf16x8_t hi[2], lo[2];
 #pragma unroll
-    for (int i = 0; i < 8 / W; ++i) {
-      const int c2 = W == 8 ? half : i;  // 32 keys of the tile
-      const int key0 = t * kTile + 32 * c2;
-      const bool full = key0 + 31 <= wq0;
+    for (int c2 = 0; c2 < 2; ++c2) {  // 32 keys at a time
       f32x4_t s[2], dp[2];
 #pragma unroll
       for (int k2 = 0; k2 < 2; ++k2) {
+        const int kb = 2 * c2 + k2;
         s[k2] = dp[k2] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          const bf16x8_t ok = row_operand(sK[buf], 2 * c2 + k2, c, l16, g4);
-          const bf16x8_t ov = row_operand(sV[buf], 2 * c2 + k2, c, l16, g4);
+          const bf16x8_t ok = row_operand(sK[buf], kb, c, l16, g4);
+          const bf16x8_t ov = row_operand(sV[buf], kb, c, l16, g4);
           s[k2] = mfma(ok, qop[c], s[k2]);
           dp[k2] = mfma(ov, dop[c], dp[k2]);
         }
@@ -411,55 +343,47 @@ __global__ __launch_bounds__(64 * W) void train_attn_dq(const AttnArgs a) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float p = fast_exp2(fmaf(s[k2][r], a.scale_log2, -m)) * inv;
-          s[k2][r] = p * (dp[k2][r] - delta);
+          const float ds = p * (dp[k2][r] - delta);
+          s[k2][r] = full || 16 * (2 * c2 + k2) + r <= lim ? ds : 0.f;
         }
-      if (!full) {
-#pragma unroll
-        for (int k2 = 0; k2 < 2; ++k2)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) s[k2][r] = 16 * k2 + r <= lim ? s[k2][r] : 0.f;
-      }
-      bf16x8_t hi, lo;
-      split_operand(s[0], s[1], hi, lo);
-#pragma unroll
-      for (int db = 0; db < 8; ++db) {
-        const bf16x8_t op = col_operand(sK[buf], c2, db, l16, g4);
-        acc[db] = mfma(op, lo, acc[db]);
-        acc[db] = mfma(op, hi, acc[db]);
-      }
+      split_operand(s[0], s[1], hi[c2], lo[c2]);
     }
+#pragma unroll
+    for (int db = 0; db < 8; ++db)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const bf16x8_t op = col_operand(sK[buf], c, db, l16, g4);
+        acc[db] = mfma(op, lo[c], acc[db]);
+        acc[db] = mfma(op, hi[c], acc[db]);
+      }
     if (more) {
       store_tile(sK[buf ^ 1], ks);
       store_tile(sV[buf ^ 1], vs);
     }
     __syncthreads();
   }
-  if constexpr (W == 8) add_halves(reinterpret_cast<float*>(tiles), acc, wave, lane);
-  if (half == 0 && qi < T) store_row_bf16(a.dq + (tok0 + qi) * a.dq_ts + h * kD, acc, a.scale, g4);
+  if (qi < T) store_row_bf16(a.dq + (tok0 + qi) * a.dq_ts + h * kD, acc, a.scale, g4);
 }
 
 // Blocks: x = KV head, y = sequence, z = key block (the early blocks, seen by
 // the most queries, first).
-template <int W>
-__global__ __launch_bounds__(64 * W) void train_attn_dkv(const AttnArgs a) {
-  __shared__ __attribute__((aligned(16))) uint16_t tiles[2][2][kTileElems];
-  uint16_t(*const sQ)[kTileElems] = tiles[0];
-  uint16_t(*const sO)[kTileElems] = tiles[1];
+__global__ __launch_bounds__(kThreads) void train_attn_dkv(const AttnArgs a) {
+  __shared__ __attribute__((aligned(16))) uint16_t sQ[2][kTileElems], sO[2][kTileElems];
   __shared__ __attribute__((aligned(16))) float sStat[2][3][kTile];  // max, 1 / sum, delta
   const int lane = threadIdx.x & 63, l16 = lane & 15, g4 = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wave >> 2;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int G = a.Hq / a.Hkv, kvh = blockIdx.x, b = blockIdx.y;
-  const int k0 = blockIdx.z * 64, wk0 = k0 + (wave & 3) * 16;
+  const int k0 = blockIdx.z * 64, wk0 = k0 + wave * 16;
   const int T = a.T;
   const int64_t tok0 = (int64_t)b * T;
   const int t_first = k0 / kTile, per_head = (T + kTile - 1) / kTile - t_first, n_steps = G * per_head;
-  Stage<W> qs, os;
+  Stage qs, os;
   float2 st;
   float de;
   auto load_step = [&](int i) {
     const int h = kvh * G + i / per_head, r0 = (t_first + i % per_head) * kTile;
-    qs = load_tile<W>(a.q + tok0 * a.q_ts + h * kD, a.q_ts, r0, T);
-    os = load_tile<W>(a.dout + tok0 * a.dout_ts + h * kD, a.dout_ts, r0, T);
+    qs = load_tile(a.q + tok0 * a.q_ts + h * kD, a.q_ts, r0, T);
+    os = load_tile(a.dout + tok0 * a.dout_ts + h * kD, a.dout_ts, r0, T);
     const int qi = r0 + (int)threadIdx.x;
     const bool ok = threadIdx.x < kTile && qi < T;
     const int64_t si = ((int64_t)b * a.Hq + h) * T + qi;
@@ -476,7 +400,6 @@ __global__ __launch_bounds__(64 * W) void train_attn_dkv(const AttnArgs a) {
     }
   };
   load_step(0);
-  const int key = wk0 + l16;
   bf16x8_t kop[4], vop[4];
   f32x4_t acc_k[8], acc_v[8];
   load_rows(a.k + tok0 * a.k_ts + kvh * kD, a.k_ts, wk0, T, l16, g4, kop);
@@ -492,20 +415,22 @@ __global__ __launch_bounds__(64 * W) void train_attn_dkv(const AttnArgs a) {
     const int r0 = (t_first + i % per_head) * kTile;
     const bool full = wk0 + 15 <= r0 && r0 + kTile <= T;
 #pragma unroll
-    for (int ii = 0; ii < 8 / W; ++ii) {
-      const int c2 = W == 8 ? half : ii;  // 32 queries of the tile
+    for (int c2 = 0; c2 < 2; ++c2) {  // 32 queries at a time
       f32x4_t s[2], dp[2];
 #pragma unroll
       for (int k2 = 0; k2 < 2; ++k2) {
+        const int qb = 2 * c2 + k2;
         s[k2] = dp[k2] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          const bf16x8_t oq = row_operand(sQ[buf], 2 * c2 + k2, c, l16, g4);
-          const bf16x8_t oo = row_operand(sO[buf], 2 * c2 + k2, c, l16, g4);
+          const bf16x8_t oq = row_operand(sQ[buf], qb, c, l16, g4);
+          const bf16x8_t oo = row_operand(sO[buf], qb, c, l16, g4);
           s[k2] = mfma(oq, kop[c], s[k2]);
           dp[k2] = mfma(oo, vop[c], dp[k2]);
         }
       }
+      bf16x8_t phi, plo, dhi, dlo;
+      const int key = wk0 + l16;
 #pragma unroll
       for (int k2 = 0; k2 < 2; ++k2) {
         const int row = 16 * (2 * c2 + k2) + 4 * g4;
@@ -514,19 +439,13 @@ __global__ __launch_bounds__(64 * W) void train_attn_dkv(const AttnArgs a) {
         const f32x4_t d4 = *reinterpret_cast<const f32x4_t*>(&sStat[buf][2][row]);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          s[k2][r] = fast_exp2(fmaf(s[k2][r], a.scale_log2, -m4[r])) * i4[r];
-          dp[k2][r] = s[k2][r] * (dp[k2][r] - d4[r]);
-        }
-        if (!full) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const bool seen = key <= r0 + row + r && r0 + row + r < T;
-            s[k2][r] = seen ? s[k2][r] : 0.f;
-            dp[k2][r] = seen ? dp[k2][r] : 0.f;
-          }
+          const bool seen = full || (key <= r0 + row + r && r0 + row + r < T);
+          const float p = fast_exp2(fmaf(s[k2][r], a.scale_log2, -m4[r])) * i4[r];
+          const float ds = p * (dp[k2][r] - d4[r]);
+          s[k2][r] = seen ? p : 0.f;
+          dp[k2][r] = seen ? ds : 0.f;
         }
       }
-      bf16x8_t phi, plo, dhi, dlo;
       split_operand(s[0], s[1], phi, plo);
       split_operand(dp[0], dp[1], dhi, dlo);
 #pragma unroll
@@ -542,59 +461,18 @@ __global__ __launch_bounds__(64 * W) void train_attn_dkv(const AttnArgs a) {
     if (more) store_step(buf ^ 1);
     __syncthreads();
   }
-  if constexpr (W == 8) {
-    add_halves(reinterpret_cast<float*>(tiles[0]), acc_k, wave, lane);
-    add_halves(reinterpret_cast<float*>(tiles[1]), acc_v, wave, lane);
-  }
-  if (half || key >= T) return;
+  const int key = wk0 + l16;
+  if (key >= T) return;
   store_row_bf16(a.dk + (tok0 + key) * a.dk_ts + kvh * kD, acc_k, a.scale, g4);
   store_row_bf16(a.dv + (tok0 + key) * a.dv_ts + kvh * kD, acc_v, 1.f, g4);
 }
 
-// Waves per workgroup.  Up to two workgroups per CU all are resident at once and
-// the longest one's chain of tiles is the time: 8 waves, each half of a tile's
-// other side (summed through LDS at the end), shorten it (dK / dV at 1 x 1,152
-// tokens and 8 KV heads 144 workgroups, dQ + dK / dV 125 -> 95 us; 2 x 389 56
-// -> 47; 1 x 4,096 510 -> 439; forward at 1 x 1,152 36 -> 30).  Beyond that two
-// independent 4-wave workgroups per CU hide each other's barriers (8 x 640: 137
-// us against 157 with 8 waves).
-bool few(int64_t workgroups) { return workgroups <= 2 * device_cu_count(); }
+// Forward: 32 queries per wave once that still gives every CU two workgroups
+// (16 heads: 8 x 640 tokens 48.5 us against 52.1 with 16, 4 x 1,152 56.4 / 65.8,
+// 1 x 4,096 157 / 165); below, 16 spread the work wider (2 x 389 17.0 / 21.9,
+// 1 x 1,152 34 / 46).
+bool wide_forward(int64_t workgroups) { return workgroups >= 2 * device_cu_count(); }
 
-// Forward: 32 queries per wave once that still gives every CU two workgroups:
-// each LDS operand then feeds two MFMAs (16 heads, 8 x 640 tokens 48.2 us
-// against 52.8 with 16, 4 x 1,152 55.4 / 64.4); below, 16 spread the work wider
-// (2 x 389 17.6 / 22.7).
-template <int J, int W>
-void forward(const AttnArgs& a, int64_t batch, hipStream_t st) {
-  hipLaunchKernelGGL((train_attn_forward<J, W>), dim3(a.Hq, (unsigned)batch, (a.T + 64 * J - 1) / (64 * J)),
-                     dim3(64 * W), 0, st, a);
-}
-
-template <int W>
-void dq(const AttnArgs& a, int64_t batch, hipStream_t st) {
-  hipLaunchKernelGGL(train_attn_dq<W>, dim3(a.Hq, (unsigned)batch, (a.T + 63) / 64), dim3(64 * W), 0, st, a);
-}
-
-template <int W>
-void dkv(const AttnArgs& a, int64_t batch, hipStream_t st) {
-  hipLaunchKernelGGL(train_attn_dkv<W>, dim3(a.Hkv, (unsigned)batch, (a.T + 63) / 64), dim3(64 * W), 0, st, a);
-}
-
-void launch_forward(const AttnArgs& a, int64_t batch, hipStream_t st) {
-  const int64_t rows = batch * a.Hq;
-  if (rows * ((a.T + 127) / 128) >= 2 * device_cu_count())
-    forward<2, 4>(a, batch, st);
-  else if (few(rows * ((a.T + 63) / 64)))
-    forward<1, 8>(a, batch, st);
-  else
-    forward<1, 4>(a, batch, st);
-}
-
-void launch_backward(const AttnArgs& a, int64_t batch, hipStream_t st) {
-  const int64_t blocks = batch * ((a.T + 63) / 64);
-  few(blocks * a.Hq) ? dq<8>(a, batch, st) : dq<4>(a, batch, st);
-  few(blocks * a.Hkv) ? dkv<8>(a, batch, st) : dkv<4>(a, batch, st);
-}
 int check_shape(int64_t batch, int64_t T, int64_t Hq, int64_t Hkv, int64_t D) {
   if (batch < 0 || T < 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv) return QMI_E_BAD_SHAPE;
   if (D != kD || batch > 65535 || T > (1 << 22) || Hq > 4096) return QMI_E_UNSUPPORTED;
@@ -622,8 +500,15 @@ extern "C" int qmi_train_attn_forward(const uint16_t* q, int64_t q_stride, const
   a.T = (int)seq_len, a.Hq = (int)num_q_heads, a.Hkv = (int)num_kv_heads;
   a.scale = scale, a.scale_log2 = scale * kLog2e;
   a.out = out, a.out_ts = out_stride, a.out32 = out_f32, a.stat = reinterpret_cast<float2*>(stats);
+  const int64_t n128 = (seq_len + 127) / 128;
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  launch_forward(a, batch, st);
+  if (wide_forward(n128 * batch * num_q_heads))
+    hipLaunchKernelGGL(train_attn_forward<2>, dim3((unsigned)num_q_heads, (unsigned)batch, (unsigned)n128),
+                       dim3(kThreads), 0, st, a);
+  else
+    hipLaunchKernelGGL(train_attn_forward<1>,
+                       dim3((unsigned)num_q_heads, (unsigned)batch, (unsigned)((seq_len + 63) / 64)), dim3(kThreads),
+                       0, st, a);
   QMI_RETURN_LAUNCH_STATUS();
 }
 
@@ -651,7 +536,11 @@ extern "C" int qmi_train_attn_backward(const uint16_t* q, int64_t q_stride, cons
   a.out32 = const_cast<float*>(out_f32), a.stat = reinterpret_cast<float2*>(const_cast<float*>(stats));
   a.dout = dout, a.dout_ts = dout_stride, a.delta = delta;
   a.dq = dq, a.dk = dk, a.dv = dv, a.dq_ts = dq_stride, a.dk_ts = dk_stride, a.dv_ts = dv_stride;
+  const int64_t n64 = (seq_len + 63) / 64;
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  launch_backward(a, batch, st);
+  hipLaunchKernelGGL(train_attn_dq, dim3((unsigned)num_q_heads, (unsigned)batch, (unsigned)n64), dim3(kThreads), 0, st,
+                     a);
+  hipLaunchKernelGGL(train_attn_dkv, dim3((unsigned)num_kv_heads, (unsigned)batch, (unsigned)n64), dim3(kThreads), 0,
+                     st, a);
   QMI_RETURN_LAUNCH_STATUS();
 }

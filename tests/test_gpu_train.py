@@ -29,12 +29,12 @@ def _core(q, k, v, batch, scale):
     return (torch.softmax(s.masked_fill(mask, float("-inf")), -1) @ v).transpose(1, 2).reshape(n, hq, d)
 
 
-# One token, tile edges and remainders, several group sizes, and on either side
-# of 512 workgroups (two per CU) for each kernel: 8 or 4 waves, and 32 queries
-# per wave in the forward from 512 blocks of 128.
+# One token, tile edges and remainders, every group size, and batches large
+# enough for 32 rows per wave in the forward / dQ (512 blocks of 128 queries)
+# and the dK / dV kernel (512 blocks of 128 keys).
 @pytest.mark.parametrize("batch,t,hq,hkv", [
     (1, 1, 16, 8), (2, 63, 16, 8), (1, 64, 4, 4), (3, 65, 8, 2), (2, 129, 6, 2), (1, 389, 16, 8),
-    (10, 200, 16, 8), (16, 200, 16, 8), (32, 193, 16, 8), (64, 64, 8, 8)])
+    (16, 200, 16, 8), (32, 193, 16, 8), (64, 64, 8, 8)])
 def test_train_attention(pkg, gpu, batch, t, hq, hkv):
     g = torch.Generator(device=gpu).manual_seed(batch * 1000 + t)
     n, d, scale = batch * t, 128, 128 ** -0.5
