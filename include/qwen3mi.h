@@ -309,31 +309,6 @@ int qmi_qk_norm_rope_backward(const uint16_t* dq, int64_t dq_stride, const uint1
                               float* workspace, int64_t workspace_bytes, void* stream);
 
 /*
- * Gradient of qmi_rms_norm / qmi_add_rms_norm (residual NULL: none): dx is the
- * gradient of the normalised sum s = x + residual (so of both terms), given dy
- * and, when dsum is not NULL, the gradient of the s output, added before the
- * one bf16 rounding.  dweight: bf16 [n].  n % 8 == 0, n <= 4096; rows 16-byte
- * aligned, strides % 8 == 0.  workspace: fp32,
- * qmi_rms_norm_backward_workspace_bytes bytes, contents ignored.  The weight's
- * gradient is summed in a fixed order.
- */
-int64_t qmi_rms_norm_backward_workspace_bytes(int64_t n_rows, int64_t n);
-int qmi_rms_norm_backward(const uint16_t* x, int64_t x_stride, const uint16_t* residual,
-                          int64_t residual_stride, const uint16_t* weight, const uint16_t* dy,
-                          int64_t dy_stride, const uint16_t* dsum, int64_t dsum_stride,
-                          uint16_t* dx, int64_t dx_stride, uint16_t* dweight, int64_t n_rows,
-                          int64_t n, float eps, float* workspace, int64_t workspace_bytes,
-                          void* stream);
-
-/*
- * Gradient of qmi_silu_mul: dgate_up [n_rows, 2 inter] from dy [n_rows, inter]
- * and the forward's gate_up.  Same alignment rules.
- */
-int qmi_silu_mul_backward(const uint16_t* gate_up, int64_t gate_up_stride, const uint16_t* dy,
-                          int64_t dy_stride, int64_t n_rows, int64_t inter, uint16_t* dgate_up,
-                          int64_t dgate_up_stride, void* stream);
-
-/*
  * Causal GQA attention of a training batch: batch sequences of seq_len tokens
  * each, rows token-major ([batch * seq_len] rows of num_heads * 128 bf16
  * elements, row strides in elements).  Replaces the fp32 attention core of

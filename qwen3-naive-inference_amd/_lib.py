@@ -81,13 +81,6 @@ SIGNATURES: dict[str, tuple] = {
         _c_i64, _c_i64, _c_i64, _c_i64,                 # tokens, heads, kv heads, head_dim
         _c_p, _c_p, _c_p, _c_i64, _c_f32,               # norm weights, cos / sin, seq_len, eps
         _c_p, _c_i64, _c_p, _c_p, _c_p, _c_i64, _c_p]), # dqkv, dweights, workspace, stream
-    "qmi_rms_norm_backward_workspace_bytes": (_c_i64, [_c_i64, _c_i64]),
-    "qmi_rms_norm_backward": (ctypes.c_int, [
-        _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_p, _c_i64,  # x, residual, w, dy, dsum
-        _c_p, _c_i64, _c_p, _c_i64, _c_i64, _c_f32,     # dx, dweight, rows, n, eps
-        _c_p, _c_i64, _c_p]),                           # workspace, bytes, stream
-    "qmi_silu_mul_backward": (ctypes.c_int, [_c_p, _c_i64, _c_p, _c_i64, _c_i64, _c_i64, _c_p,
-                                             _c_i64, _c_p]),
     "qmi_train_attn_forward": (ctypes.c_int, [
         _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64,       # q, k, v with strides
         _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_f32, # batch, seq_len, heads, head_dim, scale

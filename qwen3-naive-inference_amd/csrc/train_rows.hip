@@ -126,133 +126,6 @@ __global__ __launch_bounds__(256) void qk_norm_rope_backward_kernel(
   parts[(int64_t)blockIdx.x * 256 + threadIdx.x] = sm[0][k][d] + sm[1][k][d] + sm[2][k][d] + sm[3][k][d];
 }
 
-// ---------------------------------------------------------------------------
-// Gradient of y = x^ w, x^ = s / rms(s), s = x (+ residual): dw += dy x^ and
-// ds = (dy w - x^ mean(dy w x^)) / rms + (gradient of the s output, if any).
-// One wave per row, NV 8-element chunks per lane (n <= 512 NV), both row sums
-// in one pass; the next row's loads are issued before the current row's
-// sums.
-template <int NV>
-__global__ __launch_bounds__(256) void rms_norm_backward_rows(
-    const uint16_t* __restrict__ x, int64_t x_stride, const uint16_t* __restrict__ res, int64_t res_stride,
-    const uint16_t* __restrict__ w, const uint16_t* __restrict__ dy, int64_t dy_stride,
-    const uint16_t* __restrict__ ds, int64_t ds_stride, uint16_t* __restrict__ dx, int64_t dx_stride,
-    float* __restrict__ parts, int64_t n_rows, int n, float eps) {
-  __shared__ __attribute__((aligned(16))) float sm[4][512];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nvec = n >> 3;
-  float aw[NV][8];
-  uint4 wv[NV], xv[NV], rv[NV], yv[NV], sv[NV];
-#pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    const int c = lane + 64 * k;
-    wv[k] = c < nvec ? load_u4(w + 8 * c) : make_uint4(0, 0, 0, 0);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) aw[k][e] = 0.f;
-  }
-  auto load_row = [&](int64_t row) {
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      const int c = lane + 64 * k;
-      const bool ok = c < nvec;
-      xv[k] = ok ? load_u4(x + row * x_stride + 8 * c) : make_uint4(0, 0, 0, 0);
-      yv[k] = ok ? load_u4(dy + row * dy_stride + 8 * c) : make_uint4(0, 0, 0, 0);
-      rv[k] = ok && res ? load_u4(res + row * res_stride + 8 * c) : make_uint4(0, 0, 0, 0);
-      sv[k] = ok && ds ? load_u4(ds + row * ds_stride + 8 * c) : make_uint4(0, 0, 0, 0);
-    }
-  };
-  const int64_t step = (int64_t)gridDim.x * 4;
-  int64_t row = (int64_t)blockIdx.x * 4 + wave;
-  if (row < n_rows) load_row(row);
-  for (; row < n_rows; row += step) {
-    float xs[NV][8], g[NV][8];
-    uint4 add[NV];
-    float ss = 0.f, dot = 0.f;
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      const uint32_t xw[4] = {xv[k].x, xv[k].y, xv[k].z, xv[k].w}, rw[4] = {rv[k].x, rv[k].y, rv[k].z, rv[k].w};
-      const uint32_t yw[4] = {yv[k].x, yv[k].y, yv[k].z, yv[k].w}, ww[4] = {wv[k].x, wv[k].y, wv[k].z, wv[k].w};
-      add[k] = sv[k];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int i = e >> 1;
-        xs[k][e] = e & 1 ? bf16_hi(xw[i]) : bf16_lo(xw[i]);
-        if (res) xs[k][e] += e & 1 ? bf16_hi(rw[i]) : bf16_lo(rw[i]);
-        g[k][e] = e & 1 ? bf16_hi(yw[i]) : bf16_lo(yw[i]);
-        ss += xs[k][e] * xs[k][e];
-        dot += g[k][e] * (e & 1 ? bf16_hi(ww[i]) : bf16_lo(ww[i])) * xs[k][e];
-      }
-    }
-    if (row + step < n_rows) load_row(row + step);
-    ss = wave_sum(ss);
-    dot = wave_sum(dot);
-    const float inv = rsqrtf(ss / (float)n + eps);
-    const float mean = dot * inv / (float)n;
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      const int c = lane + 64 * k;
-      const uint32_t ww[4] = {wv[k].x, wv[k].y, wv[k].z, wv[k].w}, aw4[4] = {add[k].x, add[k].y, add[k].z, add[k].w};
-      float o[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int i = e >> 1;
-        const float xh = xs[k][e] * inv;
-        aw[k][e] += g[k][e] * xh;
-        o[e] = inv * (g[k][e] * (e & 1 ? bf16_hi(ww[i]) : bf16_lo(ww[i])) - xh * mean) +
-               (e & 1 ? bf16_hi(aw4[i]) : bf16_lo(aw4[i]));
-      }
-      if (c < nvec)
-        *reinterpret_cast<uint4*>(dx + row * dx_stride + 8 * c) =
-            make_uint4(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]), pack_bf16x2(o[4], o[5]),
-                       pack_bf16x2(o[6], o[7]));
-    }
-  }
-  // The four waves' sums, 512 columns at a time.
-#pragma unroll
-  for (int k = 0; k < NV; ++k) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) sm[wave][8 * lane + e] = aw[k][e];
-    __syncthreads();
-    for (int i = threadIdx.x; i < 512; i += 256)
-      if (512 * k + i < n)
-        parts[(int64_t)blockIdx.x * n + 512 * k + i] = sm[0][i] + sm[1][i] + sm[2][i] + sm[3][i];
-    __syncthreads();
-  }
-}
-
-// Gradient of silu(g) * u on a packed [g | u] row, 8 elements per lane:
-// d g = dy u s (1 + g (1 - s)), d u = dy g s with s = 1 / (1 + exp(-g)).
-__global__ __launch_bounds__(256) void silu_mul_backward_kernel(const uint16_t* __restrict__ gu, int64_t gu_stride,
-                                                                const uint16_t* __restrict__ dy, int64_t dy_stride,
-                                                                int inter, uint16_t* __restrict__ dgu,
-                                                                int64_t dgu_stride, int64_t n_rows) {
-  const int nvec = inter >> 3;
-  const int64_t total = n_rows * nvec;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-    const int64_t r = i / nvec;
-    const int c = (int)(i - r * nvec);
-    const uint4 g = load_u4(gu + r * gu_stride + 8 * c);
-    const uint4 u = load_u4(gu + r * gu_stride + inter + 8 * c);
-    const uint4 y = load_u4(dy + r * dy_stride + 8 * c);
-    const uint32_t gw[4] = {g.x, g.y, g.z, g.w}, uw[4] = {u.x, u.y, u.z, u.w}, yw[4] = {y.x, y.y, y.z, y.w};
-    float dg[8], du[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int k = e >> 1;
-      const float gf = e & 1 ? bf16_hi(gw[k]) : bf16_lo(gw[k]), uf = e & 1 ? bf16_hi(uw[k]) : bf16_lo(uw[k]);
-      const float yf = e & 1 ? bf16_hi(yw[k]) : bf16_lo(yw[k]);
-      const float s = 1.0f / (1.0f + __expf(-gf));
-      dg[e] = yf * uf * s * (1.0f + gf * (1.0f - s));
-      du[e] = yf * gf * s;
-    }
-    uint16_t* out = dgu + r * dgu_stride + 8 * c;
-    *reinterpret_cast<uint4*>(out) = make_uint4(pack_bf16x2(dg[0], dg[1]), pack_bf16x2(dg[2], dg[3]),
-                                                pack_bf16x2(dg[4], dg[5]), pack_bf16x2(dg[6], dg[7]));
-    *reinterpret_cast<uint4*>(out + inter) = make_uint4(pack_bf16x2(du[0], du[1]), pack_bf16x2(du[2], du[3]),
-                                                        pack_bf16x2(du[4], du[5]), pack_bf16x2(du[6], du[7]));
-  }
-}
-
 inline bool al(const void* p, unsigned n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }
 
 // Partial rows of a launch: two workgroups per CU, fewer when the rows run out.
@@ -296,59 +169,5 @@ extern "C" int qmi_qk_norm_rope_backward(const uint16_t* dq, int64_t dq_stride, 
                      cos_sin_cache, (int)seq_len, n_tok, eps, dqkv, dqkv_stride, workspace);
   hipLaunchKernelGGL(sum_columns, dim3(8), dim3(256), 0, st, workspace, (int)parts, 256, 128, dq_norm_weight,
                      dk_norm_weight);
-  QMI_RETURN_LAUNCH_STATUS();
-}
-
-extern "C" int64_t qmi_rms_norm_backward_workspace_bytes(int64_t n_rows, int64_t n) {
-  if (n_rows <= 0 || n <= 0) return 0;
-  return part_rows(n_rows, 4) * n * 4;
-}
-
-extern "C" int qmi_rms_norm_backward(const uint16_t* x, int64_t x_stride, const uint16_t* residual,
-                                     int64_t residual_stride, const uint16_t* weight, const uint16_t* dy,
-                                     int64_t dy_stride, const uint16_t* dsum, int64_t dsum_stride, uint16_t* dx,
-                                     int64_t dx_stride, uint16_t* dweight, int64_t n_rows, int64_t n, float eps,
-                                     float* workspace, int64_t workspace_bytes, void* stream) {
-  if (n_rows < 0 || n <= 0) return QMI_E_BAD_SHAPE;
-  if (n_rows == 0) return QMI_OK;
-  if (!x || !weight || !dy || !dx || !dweight || !workspace) return QMI_E_NULL_POINTER;
-  if (n % 8 || n > 4096) return QMI_E_UNSUPPORTED;
-  if (x_stride % 8 || residual_stride % 8 || dy_stride % 8 || dsum_stride % 8 || dx_stride % 8 || !al(x, 16) ||
-      !al(residual, 16) || !al(weight, 16) || !al(dy, 16) || !al(dsum, 16) || !al(dx, 16) || !al(workspace, 4))
-    return QMI_E_BAD_STRIDE;
-  const int64_t parts = part_rows(n_rows, 4);
-  if (workspace_bytes < parts * n * 4) return QMI_E_WORKSPACE_TOO_SMALL;
-  const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)parts), dim3(256), 0, st, x, x_stride, residual, residual_stride, weight,
-                       dy, dy_stride, dsum, dsum_stride, dx, dx_stride, workspace, n_rows, (int)n, eps);
-  };
-  if (n <= 512)
-    launch(rms_norm_backward_rows<1>);
-  else if (n <= 1024)
-    launch(rms_norm_backward_rows<2>);
-  else if (n <= 2048)
-    launch(rms_norm_backward_rows<4>);
-  else
-    launch(rms_norm_backward_rows<8>);
-  hipLaunchKernelGGL(sum_columns, dim3((unsigned)((n + 31) / 32)), dim3(256), 0, st, workspace, (int)parts, (int)n,
-                     (int)n, dweight, nullptr);
-  QMI_RETURN_LAUNCH_STATUS();
-}
-
-extern "C" int qmi_silu_mul_backward(const uint16_t* gate_up, int64_t gate_up_stride, const uint16_t* dy,
-                                     int64_t dy_stride, int64_t n_rows, int64_t inter, uint16_t* dgate_up,
-                                     int64_t dgate_up_stride, void* stream) {
-  if (n_rows < 0 || inter <= 0) return QMI_E_BAD_SHAPE;
-  if (n_rows == 0) return QMI_OK;
-  if (!gate_up || !dy || !dgate_up) return QMI_E_NULL_POINTER;
-  if (inter % 8 || inter > 0x3fffffffLL || gate_up_stride % 8 || dy_stride % 8 || dgate_up_stride % 8 ||
-      !al(gate_up, 16) || !al(dy, 16) || !al(dgate_up, 16) || gate_up_stride < 2 * inter || dy_stride < inter ||
-      dgate_up_stride < 2 * inter)
-    return QMI_E_BAD_STRIDE;
-  const int64_t blocks = std::min<int64_t>((n_rows * (inter / 8) + 255) / 256, 65535 * 8);
-  hipLaunchKernelGGL(silu_mul_backward_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                     reinterpret_cast<hipStream_t>(stream), gate_up, gate_up_stride, dy, dy_stride, (int)inter,
-                     dgate_up, dgate_up_stride, n_rows);
   QMI_RETURN_LAUNCH_STATUS();
 }

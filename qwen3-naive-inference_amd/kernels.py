@@ -529,36 +529,6 @@ def qk_norm_rope_backward(dq: torch.Tensor, dk: torch.Tensor, qkv: torch.Tensor,
     return dqw, dkw
 
 
-def rms_norm_backward(x: torch.Tensor, residual: torch.Tensor | None, weight: torch.Tensor,
-                      dy: torch.Tensor, dsum: torch.Tensor | None, eps: float):
-    """Gradients ``(ds, dweight)`` of ``rms_norm(s) * weight`` with ``s = x``
-    (``+ residual``), plus ``dsum``, the gradient of the ``s`` output."""
-    x2, dy2 = _rows2d("x", x), _rows2d("dy", dy)
-    r2 = None if residual is None else _rows2d("residual", residual)
-    s2 = None if dsum is None else _rows2d("dsum", dsum)
-    w = _dense16(weight)
-    dx, dw = torch.empty(x2.shape, dtype=x2.dtype, device=x2.device), torch.empty_like(w)
-    L = lib()
-    nbytes = L.qmi_rms_norm_backward_workspace_bytes(x2.shape[0], x2.shape[1])
-    ws = torch.empty((max(nbytes, 4) // 4,), dtype=torch.float32, device=x2.device)
-    check(L.qmi_rms_norm_backward(
-        x2.data_ptr(), x2.stride(0), _ptr(r2), 0 if r2 is None else r2.stride(0), w.data_ptr(),
-        dy2.data_ptr(), dy2.stride(0), _ptr(s2), 0 if s2 is None else s2.stride(0), dx.data_ptr(),
-        dx.stride(0), dw.data_ptr(), x2.shape[0], x2.shape[1], float(eps), ws.data_ptr(),
-        ws.numel() * 4, stream_handle(x2.device)), "rms_norm_backward")
-    return dx.view(x.shape), dw
-
-
-def silu_mul_backward(gate_up: torch.Tensor, dy: torch.Tensor) -> torch.Tensor:
-    """Gradient of ``silu_mul``."""
-    g2, dy2 = _rows2d("gate_up", gate_up), _rows2d("dy", dy)
-    out = torch.empty(g2.shape, dtype=torch.bfloat16, device=g2.device)
-    check(lib().qmi_silu_mul_backward(g2.data_ptr(), g2.stride(0), dy2.data_ptr(), dy2.stride(0),
-                                      g2.shape[0], g2.shape[1] // 2, out.data_ptr(), out.stride(0),
-                                      stream_handle(g2.device)), "silu_mul_backward")
-    return out.view(gate_up.shape)
-
-
 def train_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, batch: int,
                     softmax_scale: float, need_grad: bool):
     """Causal GQA attention of ``batch`` whole sequences, fp32 probabilities:

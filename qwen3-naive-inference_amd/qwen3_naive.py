@@ -12,10 +12,10 @@ in under its generator and GRPO loop:
 Inference paths (no autograd) run the HIP kernels: fused QK-RMSNorm + RoPE,
 slot-mapped KV store, paged decode / varlen prefill attention, RMSNorm /
 add+RMSNorm, SwiGLU; projections use torch GEMMs (hipBLASLt).  The batch
-``forward`` used for training runs RMSNorm, SwiGLU and QK-norm + RoPE +
-attention as autograd Functions with HIP kernels in both directions
-(train_ops.py; the reference's RoPE kernel has no backward), probabilities and
-score gradients in fp32.
+``forward`` used for training runs QK-norm, RoPE and attention as one autograd
+Function with HIP kernels in both directions (train_ops.py; the reference's
+RoPE kernel has no backward), probabilities and score gradients in fp32, and
+torch ops elsewhere.
 """
 from __future__ import annotations
 
@@ -28,6 +28,7 @@ from functools import lru_cache
 import numpy as np
 import torch
 import torch.nn as nn
+import torch.nn.functional as F
 
 from . import kernels as K
 from . import train_ops as T
@@ -108,9 +109,12 @@ class RMSNorm(nn.Module):
         self.weight = nn.Parameter(torch.ones(hidden_size))
 
     def _torch(self, x, residual):
-        if residual is None:
-            return T.rms_norm_formula(x, self.weight, self.eps)
-        return T.add_rms_norm_formula(x, residual, self.weight, self.eps)
+        dt = x.dtype
+        xf = x.float() if residual is None else x.float() + residual.float()
+        res = None if residual is None else xf.to(dt)
+        y = (xf * torch.rsqrt(xf.pow(2).mean(dim=-1, keepdim=True) + self.eps)
+             * self.weight.float()).to(dt)
+        return y if residual is None else (y, res)
 
     def forward(self, x, residual=None):
         if isinstance(x, K.RowParts):  # a decode projection's split-K partial products
@@ -118,10 +122,6 @@ class RMSNorm(nn.Module):
                 x = x.dense()
             else:
                 return K.add_rms_norm_parts(x, residual, self.weight, self.eps)
-        if not _use_kernels(x, self.weight) and T.norm_ok(x, self.weight, residual):
-            if residual is None:
-                return T.RmsNorm.apply(x, self.weight, self.eps)
-            return T.AddRmsNorm.apply(x, residual, self.weight, self.eps)
         if (x.dtype != torch.bfloat16 or x.shape[-1] > K.NORM_MAX_WIDTH
                 or not _use_kernels(x, self.weight)):
             return self._torch(x, residual)
@@ -276,9 +276,8 @@ class Qwen3MLP(nn.Module):
         gu = self.gate_up_proj(x)
         if gu.dtype == torch.bfloat16 and _use_kernels(gu):
             return self.down_proj(K.silu_mul(gu))
-        if T.silu_mul_ok(gu):
-            return self.down_proj(T.SiluMul.apply(gu))
-        return self.down_proj(T.silu_mul_formula(gu))
+        gate, up = gu.chunk(2, dim=-1)
+        return self.down_proj(F.silu(gate) * up)
 
     def forward_decode(self, x):
         """Decode step: gate_up GEMM with the SwiGLU epilogue, then down_proj as
@@ -300,9 +299,8 @@ class Qwen3DecoderLayer(nn.Module):
         self.mlp = Qwen3MLP(config)
 
     def forward(self, x):
-        h = self.self_attn(self.input_layernorm(x))
-        h, x = self.post_attention_layernorm(h, x)
-        return self.mlp(h) + x
+        x = self.self_attn(self.input_layernorm(x)) + x
+        return self.mlp(self.post_attention_layernorm(x)) + x
 
     def forward_prefill(self, x, positions, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
                         max_seqlen_k, block_mapping, block_tables=None, residual=None):

@@ -39,97 +39,6 @@ def _formula_grads(formula, inputs, needs, grads):
 
 
 # ---------------------------------------------------------------------------
-# RMSNorm, residual add + RMSNorm, SwiGLU (qwen3_naive.py:156-169, :695-702)
-# ---------------------------------------------------------------------------
-def rms_norm_formula(x, weight, eps):
-    xf = x.float()
-    return (xf * torch.rsqrt(xf.pow(2).mean(dim=-1, keepdim=True) + eps)
-            * weight.float()).to(x.dtype)
-
-
-def add_rms_norm_formula(x, residual, weight, eps):
-    xf = x.float() + residual.float()
-    y = (xf * torch.rsqrt(xf.pow(2).mean(dim=-1, keepdim=True) + eps)
-         * weight.float()).to(x.dtype)
-    return y, xf.to(x.dtype)
-
-
-def silu_mul_formula(gate_up):
-    gate, up = gate_up.chunk(2, dim=-1)
-    return torch.nn.functional.silu(gate) * up
-
-
-def norm_ok(x, weight, residual=None) -> bool:
-    """Whether ``RmsNorm`` / ``AddRmsNorm`` take these tensors."""
-    return (kernels_ok(x, weight) and (residual is None or (kernels_ok(x, residual)
-                                                            and residual.shape == x.shape))
-            and x.numel() > 0 and weight.shape == x.shape[-1:]
-            and x.shape[-1] % 8 == 0 and x.shape[-1] <= K.NORM_MAX_WIDTH)
-
-
-def silu_mul_ok(gate_up) -> bool:
-    return kernels_ok(gate_up) and gate_up.numel() > 0 and gate_up.shape[-1] % 16 == 0
-
-
-class RmsNorm(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, weight, eps):
-        ctx.save_for_backward(x, weight)
-        ctx.eps = eps
-        return K.rms_norm(x, weight, eps)
-
-    @staticmethod
-    def backward(ctx, dy):
-        x, weight = ctx.saved_tensors
-        need = ctx.needs_input_grad
-        if torch.is_grad_enabled():
-            return (*_formula_grads(lambda x, w: rms_norm_formula(x, w, ctx.eps), (x, weight),
-                                    need[:2], dy), None)
-        dx, dw = K.rms_norm_backward(x, None, weight, dy, None, ctx.eps)
-        return dx if need[0] else None, dw if need[1] else None, None
-
-
-class AddRmsNorm(torch.autograd.Function):
-    """``(rms_norm(s), s)`` of ``s = x + residual``."""
-
-    @staticmethod
-    def forward(ctx, x, residual, weight, eps):
-        ctx.save_for_backward(x, residual, weight)
-        ctx.set_materialize_grads(False)
-        ctx.eps = eps
-        return K.add_rms_norm(x, residual, weight, eps)
-
-    @staticmethod
-    def backward(ctx, dy, dsum):
-        x, residual, weight = ctx.saved_tensors
-        need = ctx.needs_input_grad
-        if dy is None:  # only the sum was used
-            return (dsum if need[0] else None, dsum if need[1] else None, None, None)
-        if torch.is_grad_enabled():
-            grads = (dy, torch.zeros_like(dy) if dsum is None else dsum)
-            return (*_formula_grads(lambda x, r, w: add_rms_norm_formula(x, r, w, ctx.eps),
-                                    (x, residual, weight), need[:3], grads), None)
-        ds, dw = K.rms_norm_backward(x, residual, weight, dy, dsum, ctx.eps)
-        return (ds if need[0] else None, ds if need[1] else None, dw if need[2] else None, None)
-
-
-class SiluMul(torch.autograd.Function):
-    """``silu(gate) * up`` of a packed ``[..., 2 * inter]`` projection."""
-
-    @staticmethod
-    def forward(ctx, gate_up):
-        ctx.save_for_backward(gate_up)
-        return K.silu_mul(gate_up)
-
-    @staticmethod
-    def backward(ctx, dy):
-        gate_up, = ctx.saved_tensors
-        if torch.is_grad_enabled():
-            return _formula_grads(silu_mul_formula, (gate_up,), ctx.needs_input_grad, dy)
-        return K.silu_mul_backward(gate_up, dy)
-
-
-# ---------------------------------------------------------------------------
 # Attention of a training batch (qwen3_naive.py:553-590)
 # ---------------------------------------------------------------------------
 def rotate(x: torch.Tensor, positions: torch.Tensor, cache: torch.Tensor) -> torch.Tensor:
@@ -167,6 +76,12 @@ def attention_formula(qkv, norm_q, norm_k, cache, num_heads, num_kv_heads, scale
     w = torch.softmax(scores, dim=-1)
     o = torch.matmul(w, vf).to(qkv.dtype)
     return o.transpose(1, 2).reshape(batch, seq_len, -1)
+
+
+def rms_norm_formula(x, weight, eps):
+    xf = x.float()
+    return (xf * torch.rsqrt(xf.pow(2).mean(dim=-1, keepdim=True) + eps)
+            * weight.float()).to(x.dtype)
 
 
 class QkvAttention(torch.autograd.Function):

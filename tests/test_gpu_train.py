@@ -145,64 +145,3 @@ def test_attention_second_derivative(pkg, gpu):
         gg, = torch.autograd.grad(g.float().square().sum(), qkv)
         res.append(gg)
     assert res[0].abs().max() > 0 and _rel(res[0], res[1].double()) < 0.05
-
-
-# Widths at each edge of the kernel's chunk counts (8 / 512 / 520 / 1,024 /
-# 2,048 / 4,096), a remainder of rows, more rows than one pass of the grid.
-@pytest.mark.parametrize("rows,n", [(1, 8), (7, 512), (3, 520), (5120, 1024), (66, 2048), (9, 2056), (5, 4096)])
-@pytest.mark.parametrize("residual", [False, True])
-def test_rms_norm_gradients(pkg, gpu, rows, n, residual):
-    g = torch.Generator(device=gpu).manual_seed(n + rows)
-    norm = pkg.RMSNorm(n, eps=1e-6).to(gpu).bfloat16()
-    with torch.no_grad():
-        norm.weight.copy_(torch.rand(n, generator=g, device=gpu) * 0.4 + 0.8)
-    x, r, dy, ds = (torch.randn(rows, n, generator=g, device=gpu).bfloat16() for _ in range(4))
-    x.requires_grad_(), r.requires_grad_()
-    a, b, w = (z.detach().double().requires_grad_() for z in (x, r, norm.weight))
-    s = a + b if residual else a
-    ref = s * torch.rsqrt(s.square().mean(-1, keepdim=True) + 1e-6) * w
-    if residual:
-        y, res = norm(x, r)
-        torch.autograd.backward([y, res], [dy, ds])
-        torch.autograd.backward([ref, s], [dy.double(), ds.double()])
-        assert _rel(res, s) < BF16 and torch.equal(x.grad, r.grad)
-    else:
-        y = norm(x)
-        y.backward(dy)
-        ref.backward(dy.double())
-    assert "RmsNorm" in type(y.grad_fn).__name__
-    assert _rel(y, ref) < BF16
-    assert _rel(x.grad, a.grad) < BF16
-    assert _rel(norm.weight.grad, w.grad) < BF16
-
-
-@pytest.mark.parametrize("rows,inter", [(1, 8), (3, 136), (130, 3072)])
-def test_silu_mul_gradient(pkg, gpu, rows, inter):
-    g = torch.Generator(device=gpu).manual_seed(inter)
-    gu = (torch.randn(rows, 2 * inter, generator=g, device=gpu) * 4).bfloat16()
-    gu[0, 0], gu[0, 1], gu[0, 2] = 200.0, -200.0, 0.0  # exp overflow on one side
-    dy = torch.randn(rows, inter, generator=g, device=gpu).bfloat16()
-    x = gu.double().requires_grad_()
-    (torch.nn.functional.silu(x[:, :inter]) * x[:, inter:]).backward(dy.double())
-    got = pkg.kernels.silu_mul_backward(gu, dy)
-    assert bool(torch.isfinite(got).all()) and _rel(got, x.grad) < BF16
-
-
-def test_layer_gradients_twice_and_sum_only(pkg, gpu):
-    """Second derivatives through the norm and SwiGLU, and a residual sum used without its norm."""
-    T = pkg.qwen3_naive.T
-    x = torch.randn(3, 64, device=gpu).bfloat16().requires_grad_()
-    r = torch.randn(3, 64, device=gpu).bfloat16().requires_grad_()
-    w = torch.rand(64, device=gpu).add(0.5).bfloat16().requires_grad_()
-    for fused, plain, args in ((T.RmsNorm.apply, T.rms_norm_formula, (x, w, 1e-6)),
-                               (lambda *a: T.AddRmsNorm.apply(*a)[0],
-                                lambda *a: T.add_rms_norm_formula(*a)[0], (x, r, w, 1e-6)),
-                               (T.SiluMul.apply, T.silu_mul_formula, (x,))):
-        res = []
-        for f in (fused, plain):
-            g, = torch.autograd.grad(f(*args).float().square().sum(), x, create_graph=True)
-            res.append(torch.autograd.grad(g.float().square().sum(), x)[0])
-        assert res[0].abs().max() > 0 and _rel(res[0], res[1].double()) < 0.05
-    _, s = T.AddRmsNorm.apply(x, r, w, 1e-6)
-    gx, gr = torch.autograd.grad(s, (x, r), torch.ones_like(s))
-    assert bool((gx == 1).all()) and bool((gr == 1).all())
