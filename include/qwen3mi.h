@@ -279,67 +279,6 @@ int qmi_qk_norm_rope(const uint16_t* qkv, int64_t qkv_stride, int64_t n_tok, int
                      void* stream);
 
 /*
- * qmi_qk_norm_rope for a batch of whole sequences of seq_len tokens: token
- * tok is at position tok % seq_len (seq_len <= max_position).  Replaces
- * q_norm / k_norm + RoPE of the batch path (qwen3_naive.py:553-570).
- */
-int qmi_qk_norm_rope_seq(const uint16_t* qkv, int64_t qkv_stride, int64_t n_tok,
-                         int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim,
-                         const uint16_t* q_norm_weight, const uint16_t* k_norm_weight,
-                         int64_t seq_len, const float* cos_sin_cache, int64_t max_position,
-                         uint16_t* q_out, int64_t q_stride, uint16_t* k_out, int64_t k_stride,
-                         float eps, void* stream);
-
-/*
- * Gradient of qmi_qk_norm_rope_seq.  dq [n_tok, Hq, 128] and dk [n_tok, Hkv,
- * 128] are the gradients of q_out and k_out; qkv is the forward's input.
- * Writes the q and k heads of dqkv (row stride dqkv_stride; the v heads are
- * left alone) and the bf16 gradients of the two norm weights.  workspace:
- * fp32, qmi_qk_norm_rope_backward_workspace_bytes bytes, contents ignored.
- */
-int64_t qmi_qk_norm_rope_backward_workspace_bytes(int64_t n_tok, int64_t num_q_heads,
-                                                  int64_t num_kv_heads);
-int qmi_qk_norm_rope_backward(const uint16_t* dq, int64_t dq_stride, const uint16_t* dk,
-                              int64_t dk_stride, const uint16_t* qkv, int64_t qkv_stride,
-                              int64_t n_tok, int64_t num_q_heads, int64_t num_kv_heads,
-                              int64_t head_dim, const uint16_t* q_norm_weight,
-                              const uint16_t* k_norm_weight, const float* cos_sin_cache,
-                              int64_t seq_len, float eps, uint16_t* dqkv, int64_t dqkv_stride,
-                              uint16_t* dq_norm_weight, uint16_t* dk_norm_weight,
-                              float* workspace, int64_t workspace_bytes, void* stream);
-
-/*
- * Causal GQA attention of a training batch: batch sequences of seq_len tokens
- * each, rows token-major ([batch * seq_len] rows of num_heads * 128 bf16
- * elements, row strides in elements).  Replaces the fp32 attention core of
- * Qwen3Attention.forward (qwen3_naive.py:572-590):
- * out = softmax(q k^T * scale, causal) v, probabilities in fp32.
- * out_f32 [batch * seq_len, Hq, 128] and stats [batch, Hq, seq_len, 2] (row
- * maximum in the log2 domain, 1 / row sum) are what the backward needs; both
- * are given or neither.  head_dim 128 only; q, k, v 16-byte aligned with
- * strides % 8 == 0, out 8-byte aligned with out_stride % 4 == 0.
- */
-int qmi_train_attn_forward(const uint16_t* q, int64_t q_stride, const uint16_t* k,
-                           int64_t k_stride, const uint16_t* v, int64_t v_stride, int64_t batch,
-                           int64_t seq_len, int64_t num_q_heads, int64_t num_kv_heads,
-                           int64_t head_dim, float scale, uint16_t* out, int64_t out_stride,
-                           float* out_f32, float* stats, void* stream);
-
-/*
- * Gradient of qmi_train_attn_forward: dout (16-byte aligned, stride % 8 == 0)
- * in, dq, dk, dv (8-byte aligned, strides % 4 == 0) out, score gradients in
- * fp32.  delta: fp32 [batch, Hq, seq_len] scratch.  Deterministic.
- */
-int qmi_train_attn_backward(const uint16_t* q, int64_t q_stride, const uint16_t* k,
-                            int64_t k_stride, const uint16_t* v, int64_t v_stride,
-                            const float* out_f32, const float* stats, const uint16_t* dout,
-                            int64_t dout_stride, int64_t batch, int64_t seq_len,
-                            int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim,
-                            float scale, float* delta, uint16_t* dq, int64_t dq_stride,
-                            uint16_t* dk, int64_t dk_stride, uint16_t* dv, int64_t dv_stride,
-                            void* stream);
-
-/*
  * qmi_qk_norm_rope with the KV store fused in: q goes to q_out as above; the
  * rotated k head and the token's v head (the last Hkv heads of the qkv row,
  * unchanged) go to row slot_mapping[tok] of k_cache / v_cache ([n_slots,

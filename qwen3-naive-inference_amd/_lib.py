@@ -73,23 +73,6 @@ SIGNATURES: dict[str, tuple] = {
     "qmi_qk_norm_rope": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p,
                                         _c_p, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_f32,
                                         _c_p]),
-    "qmi_qk_norm_rope_seq": (ctypes.c_int, [_c_p] + [_c_i64] * 5 + [_c_p, _c_p, _c_i64, _c_p,
-                             _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_f32, _c_p]),
-    "qmi_qk_norm_rope_backward_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
-    "qmi_qk_norm_rope_backward": (ctypes.c_int, [
-        _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64,       # dq, dk, qkv with strides
-        _c_i64, _c_i64, _c_i64, _c_i64,                 # tokens, heads, kv heads, head_dim
-        _c_p, _c_p, _c_p, _c_i64, _c_f32,               # norm weights, cos / sin, seq_len, eps
-        _c_p, _c_i64, _c_p, _c_p, _c_p, _c_i64, _c_p]), # dqkv, dweights, workspace, stream
-    "qmi_train_attn_forward": (ctypes.c_int, [
-        _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64,       # q, k, v with strides
-        _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_f32, # batch, seq_len, heads, head_dim, scale
-        _c_p, _c_i64, _c_p, _c_p, _c_p]),               # out, out_f32, stats, stream
-    "qmi_train_attn_backward": (ctypes.c_int, [
-        _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64,       # q, k, v with strides
-        _c_p, _c_p, _c_p, _c_i64,                       # out_f32, stats, dout
-        _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_f32, # batch, seq_len, heads, head_dim, scale
-        _c_p, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_p]),  # delta, dq, dk, dv, stream
     "qmi_qk_norm_rope_store": (ctypes.c_int, [
         _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_p,
         _c_i64, _c_p, _c_p, _c_p, _c_i64, _c_f32, _c_p]),

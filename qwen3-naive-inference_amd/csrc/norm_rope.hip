@@ -102,12 +102,11 @@ __global__ __launch_bounds__(kNormThreads) void rms_norm_rows(
 // row of 16 lanes.  k goes to k_out (when given) and, with the caches given,
 // the rotated k and the token's v head (16 bytes per lane) go straight to
 // cache row slots[tok] (slots outside [0, n_slots) are skipped, as in the KV
-// store).  Without a positions array (a training batch of whole sequences)
-// token tok is at position tok % seq_len.
+// store).
 __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
     const uint16_t* __restrict__ qkv, int64_t qkv_stride, int n_q_heads, int n_kv_heads,
     const uint16_t* __restrict__ q_w, const uint16_t* __restrict__ k_w,
-    const int64_t* __restrict__ positions, uint32_t seq_len, const float* __restrict__ cos_sin,
+    const int64_t* __restrict__ positions, const float* __restrict__ cos_sin,
     int64_t max_pos, uint16_t* __restrict__ q_out, int64_t q_stride,
     uint16_t* __restrict__ k_out, int64_t k_stride, uint16_t* __restrict__ k_cache,
     uint16_t* __restrict__ v_cache, const int32_t* __restrict__ slots, int64_t n_slots,
@@ -122,7 +121,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
   const bool is_q = h < n_q_heads;
   // Every load is issued before the reduction: position -> cos/sin is the
   // only dependent pair.
-  int64_t pos = positions ? positions[tok] : (int64_t)((uint32_t)tok % seq_len);
+  int64_t pos = positions[tok];
   const uint16_t* src = qkv + tok * qkv_stride + (int64_t)h * D;
   const uint16_t* w = is_q ? q_w : k_w;
   const uint2 xa = *reinterpret_cast<const uint2*>(src + 4 * sub);
@@ -267,38 +266,9 @@ extern "C" int qmi_qk_norm_rope(const uint16_t* qkv, int64_t qkv_stride, int64_t
   if ((items + 15) / 16 > 0x7fffffffLL) return QMI_E_UNSUPPORTED;
   hipLaunchKernelGGL(qk_norm_rope_kernel, dim3((unsigned)((items + 15) / 16)), dim3(256), 0,
                      reinterpret_cast<hipStream_t>(stream), qkv, qkv_stride, (int)num_q_heads,
-                     (int)num_kv_heads, q_norm_weight, k_norm_weight, positions, 1u, cos_sin_cache,
+                     (int)num_kv_heads, q_norm_weight, k_norm_weight, positions, cos_sin_cache,
                      max_position, q_out, q_stride, k_out, k_stride, nullptr, nullptr, nullptr,
                      (int64_t)0, n_tok, eps);
-  QMI_RETURN_LAUNCH_STATUS();
-}
-
-extern "C" int qmi_qk_norm_rope_seq(const uint16_t* qkv, int64_t qkv_stride, int64_t n_tok,
-                                    int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim,
-                                    const uint16_t* q_norm_weight, const uint16_t* k_norm_weight,
-                                    int64_t seq_len, const float* cos_sin_cache,
-                                    int64_t max_position, uint16_t* q_out, int64_t q_stride,
-                                    uint16_t* k_out, int64_t k_stride, float eps, void* stream) {
-  if (n_tok < 0 || num_q_heads <= 0 || num_kv_heads <= 0 || seq_len <= 0 || seq_len > max_position)
-    return QMI_E_BAD_SHAPE;
-  if (n_tok == 0) return QMI_OK;
-  if (!qkv || !q_norm_weight || !k_norm_weight || !cos_sin_cache || !q_out || !k_out)
-    return QMI_E_NULL_POINTER;
-  if (head_dim != 128 || n_tok > 0x7fffffffLL || num_q_heads > 4096 || num_kv_heads > 4096)
-    return QMI_E_UNSUPPORTED;
-  if (qkv_stride < (num_q_heads + 2 * num_kv_heads) * head_dim || q_stride < num_q_heads * 128 ||
-      k_stride < num_kv_heads * 128)
-    return QMI_E_BAD_STRIDE;
-  if (qkv_stride % 8 || q_stride % 4 || k_stride % 4 || !al16(qkv) || !al8(q_out) || !al8(k_out) ||
-      !al16(cos_sin_cache) || !al8(q_norm_weight) || !al8(k_norm_weight))
-    return QMI_E_BAD_STRIDE;
-  const int64_t items = n_tok * (num_q_heads + num_kv_heads);
-  if ((items + 15) / 16 > 0x7fffffffLL) return QMI_E_UNSUPPORTED;
-  hipLaunchKernelGGL(qk_norm_rope_kernel, dim3((unsigned)((items + 15) / 16)), dim3(256), 0,
-                     reinterpret_cast<hipStream_t>(stream), qkv, qkv_stride, (int)num_q_heads,
-                     (int)num_kv_heads, q_norm_weight, k_norm_weight, nullptr, (uint32_t)seq_len,
-                     cos_sin_cache, max_position, q_out, q_stride, k_out, k_stride, nullptr,
-                     nullptr, nullptr, (int64_t)0, n_tok, eps);
   QMI_RETURN_LAUNCH_STATUS();
 }
 
@@ -325,7 +295,7 @@ extern "C" int qmi_qk_norm_rope_store(
   if ((items + 15) / 16 > 0x7fffffffLL) return QMI_E_UNSUPPORTED;
   hipLaunchKernelGGL(qk_norm_rope_kernel, dim3((unsigned)((items + 15) / 16)), dim3(256), 0,
                      reinterpret_cast<hipStream_t>(stream), qkv, qkv_stride, (int)num_q_heads,
-                     (int)num_kv_heads, q_norm_weight, k_norm_weight, positions, 1u, cos_sin_cache,
+                     (int)num_kv_heads, q_norm_weight, k_norm_weight, positions, cos_sin_cache,
                      max_position, q_out, q_stride, nullptr, (int64_t)0, k_cache, v_cache,
                      slot_mapping, n_slots, n_tok, eps);
   QMI_RETURN_LAUNCH_STATUS();

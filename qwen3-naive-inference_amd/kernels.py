@@ -493,77 +493,6 @@ def qk_norm_rope_store(qkv: torch.Tensor, q_norm_weight: torch.Tensor,
     return q
 
 
-def qk_norm_rope_seq(qkv: torch.Tensor, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor,
-                     seq_len: int, cos_sin_cache: torch.Tensor, num_q_heads: int,
-                     num_kv_heads: int, eps: float):
-    """``qk_norm_rope`` of a batch of whole sequences: token ``t`` is at position
-    ``t % seq_len``.  Returns ``q [N, Hq, 128]`` and ``k [N, Hkv, 128]``."""
-    n = qkv.shape[0]
-    q = torch.empty((n, num_q_heads, HEAD_DIM), dtype=torch.bfloat16, device=qkv.device)
-    k = torch.empty((n, num_kv_heads, HEAD_DIM), dtype=torch.bfloat16, device=qkv.device)
-    check(lib().qmi_qk_norm_rope_seq(
-        qkv.data_ptr(), qkv.stride(0), n, num_q_heads, num_kv_heads, HEAD_DIM,
-        q_norm_weight.data_ptr(), k_norm_weight.data_ptr(), seq_len, cos_sin_cache.data_ptr(),
-        cos_sin_cache.shape[0], q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), float(eps),
-        stream_handle(qkv.device)), "qk_norm_rope_seq")
-    return q, k
-
-
-def qk_norm_rope_backward(dq: torch.Tensor, dk: torch.Tensor, qkv: torch.Tensor,
-                          q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, seq_len: int,
-                          cos_sin_cache: torch.Tensor, eps: float, dqkv: torch.Tensor):
-    """Gradient of ``qk_norm_rope_seq``: fills the q and k heads of ``dqkv`` and
-    returns the gradients of the two norm weights."""
-    n, hq, _ = dq.shape
-    hkv = dk.shape[1]
-    dqw, dkw = torch.empty_like(q_norm_weight), torch.empty_like(k_norm_weight)
-    L = lib()
-    nbytes = L.qmi_qk_norm_rope_backward_workspace_bytes(n, hq, hkv)
-    ws = torch.empty((max(nbytes, 4) // 4,), dtype=torch.float32, device=qkv.device)
-    check(L.qmi_qk_norm_rope_backward(
-        dq.data_ptr(), dq.stride(0), dk.data_ptr(), dk.stride(0), qkv.data_ptr(), qkv.stride(0),
-        n, hq, hkv, HEAD_DIM, q_norm_weight.data_ptr(), k_norm_weight.data_ptr(),
-        cos_sin_cache.data_ptr(), seq_len, float(eps), dqkv.data_ptr(), dqkv.stride(0),
-        dqw.data_ptr(), dkw.data_ptr(), ws.data_ptr(), ws.numel() * 4,
-        stream_handle(qkv.device)), "qk_norm_rope_backward")
-    return dqw, dkw
-
-
-def train_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, batch: int,
-                    softmax_scale: float, need_grad: bool):
-    """Causal GQA attention of ``batch`` whole sequences, fp32 probabilities:
-    ``q [N, Hq, 128]``, ``k`` / ``v [N, Hkv, 128]`` bf16 rows (unit stride along
-    heads and dims, any row stride).  Returns ``out [N, Hq, 128]`` bf16 and,
-    with ``need_grad``, the fp32 output and row statistics its backward takes."""
-    n, hq, d = q.shape
-    out = torch.empty((n, hq, d), dtype=torch.bfloat16, device=q.device)
-    out32 = stats = None
-    if need_grad:
-        out32 = torch.empty((n, hq, d), dtype=torch.float32, device=q.device)
-        stats = torch.empty((n, hq, 2), dtype=torch.float32, device=q.device)
-    check(lib().qmi_train_attn_forward(
-        q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), batch,
-        n // batch, hq, k.shape[1], d, float(softmax_scale), out.data_ptr(), out.stride(0),
-        _ptr(out32), _ptr(stats), stream_handle(q.device)), "train_attention")
-    return out, out32, stats
-
-
-def train_attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, batch: int,
-                             softmax_scale: float, out32: torch.Tensor, stats: torch.Tensor,
-                             dout: torch.Tensor, dv: torch.Tensor):
-    """Gradient of ``train_attention``: returns ``(dq, dk)`` and fills ``dv``."""
-    n, hq, d = q.shape
-    dq, dk = torch.empty_like(q), torch.empty_like(k)
-    delta = torch.empty((n, hq), dtype=torch.float32, device=q.device)
-    check(lib().qmi_train_attn_backward(
-        q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
-        out32.data_ptr(), stats.data_ptr(), dout.data_ptr(), dout.stride(0), batch, n // batch,
-        hq, k.shape[1], d, float(softmax_scale), delta.data_ptr(), dq.data_ptr(), dq.stride(0),
-        dk.data_ptr(), dk.stride(0), dv.data_ptr(), dv.stride(0), stream_handle(q.device)),
-        "train_attention_backward")
-    return dq, dk
-
-
 def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     """``silu(gate) * up`` of a fused ``[..., 2 * inter]`` projection (one bf16 rounding)."""
     g2 = _rows2d("gate_up", gate_up)

@@ -12,10 +12,9 @@ in under its generator and GRPO loop:
 Inference paths (no autograd) run the HIP kernels: fused QK-RMSNorm + RoPE,
 slot-mapped KV store, paged decode / varlen prefill attention, RMSNorm /
 add+RMSNorm, SwiGLU; projections use torch GEMMs (hipBLASLt).  The batch
-``forward`` used for training runs QK-norm, RoPE and attention as one autograd
-Function with HIP kernels in both directions (train_ops.py; the reference's
-RoPE kernel has no backward), probabilities and score gradients in fp32, and
-torch ops elsewhere.
+``forward`` used for training keeps torch ops so autograd works, with a
+differentiable RoPE (the reference's RoPE kernel has no backward) and the
+attention core in fp32.
 """
 from __future__ import annotations
 
@@ -31,7 +30,6 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import kernels as K
-from . import train_ops as T
 from .kernels import store_kvcache  # noqa: F401  (reference import surface)
 from .paged import (BLOCK_SIZE, BlockManager, Sequence, build_block_tables, fill_decode_inputs,
                     near_equal_contexts, prepare_decode, prepare_step)
@@ -91,15 +89,6 @@ def _decode_linear(proj: nn.Linear, x: torch.Tensor, parts: bool = False):
     return proj(x)
 
 
-def _unhooked(*modules: nn.Module) -> bool:
-    """Whether calling these norms runs RMSNorm.forward and nothing else, so
-    that a fused kernel may compute them from their weights."""
-    return not nn.modules.module._has_any_global_hook() and all(
-        type(m) is RMSNorm and "forward" not in m.__dict__ and not m._forward_hooks
-        and not m._forward_pre_hooks and not m._backward_hooks and not m._backward_pre_hooks
-        for m in modules)
-
-
 class RMSNorm(nn.Module):
     """RMSNorm with optional fused residual add (qwen3_naive.py:150-175)."""
 
@@ -143,7 +132,13 @@ class RotaryEmbedding(nn.Module):
     @staticmethod
     def rotate(x: torch.Tensor, positions: torch.Tensor, cache: torch.Tensor) -> torch.Tensor:
         """Differentiable half-split rotation (fp32 math, cast back)."""
-        return T.rotate(x, positions, cache)
+        half = x.shape[-1] // 2
+        cs = cache[positions]
+        while cs.dim() < x.dim():
+            cs = cs.unsqueeze(-2)
+        c, s = cs[..., :half], cs[..., half:]
+        x1, x2 = x[..., :half].float(), x[..., half:].float()
+        return torch.cat((x1 * c - x2 * s, x2 * c + x1 * s), dim=-1).to(x.dtype)
 
     def forward(self, q, k, positions):
         return (self.rotate(q, positions, self.cos_sin_cache),
@@ -217,16 +212,28 @@ class Qwen3Attention(nn.Module):
 
     # ----- batch path (training / no-cache eager forward, qwen3_naive.py:553-593) -----
     def forward(self, x):
+        batch, seq_len, _ = x.shape
         qkv = self.qkv_proj(x)
+        q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
+        q = self.q_norm(q.reshape(batch, seq_len, self.num_heads, self.head_dim))
+        k = self.k_norm(k.reshape(batch, seq_len, self.num_kv_heads, self.head_dim))
+        v = v.reshape(batch, seq_len, self.num_kv_heads, self.head_dim)
+        positions = torch.arange(seq_len, device=x.device)
         cache = self._cos_sin(x.device)
-        qw, kw = self.q_norm.weight, self.k_norm.weight
-        if (_unhooked(self.q_norm, self.k_norm) and self.q_norm.eps == self.k_norm.eps == self.eps
-                and T.attention_ok(qkv, qw, kw, cache, self.num_heads, self.num_kv_heads)):
-            o = T.QkvAttention.apply(qkv, qw, kw, cache, self.num_heads, self.num_kv_heads,
-                                     self.eps, self.scale)
-        else:
-            o = T.attention_formula(qkv, self.q_norm, self.k_norm, cache, self.num_heads,
-                                    self.num_kv_heads, self.scale)
+        q = RotaryEmbedding.rotate(q, positions[None, :].expand(batch, -1), cache)
+        k = RotaryEmbedding.rotate(k, positions[None, :].expand(batch, -1), cache)
+        rep = self.num_heads // self.num_kv_heads
+        # Attention core in fp32: batched bf16 products with transposed operands
+        # (and their autograd) are avoided on this platform.
+        qf = q.transpose(1, 2).float()
+        kf = k.transpose(1, 2).float().repeat_interleave(rep, dim=1)
+        vf = v.transpose(1, 2).float().repeat_interleave(rep, dim=1)
+        scores = torch.matmul(qf, kf.transpose(-2, -1).contiguous()) * self.scale
+        mask = torch.triu(torch.ones(seq_len, seq_len, device=x.device, dtype=torch.bool), 1)
+        scores = scores.masked_fill(mask, float("-inf"))
+        w = torch.softmax(scores, dim=-1)
+        o = torch.matmul(w, vf).to(x.dtype)
+        o = o.transpose(1, 2).reshape(batch, seq_len, -1)
         return self.o_proj(o)
 
     # ----- continuous batching (qwen3_naive.py:597-683) -----
