@@ -351,6 +351,74 @@ int qmi_add_rms_norm_parts(const float* parts, int64_t n_parts, int64_t m,
                            const uint16_t* weight, uint16_t* y, int64_t y_stride, int64_t n,
                            float eps, void* stream);
 
+/* y[m][n] = bf16(sum_s parts[s]) of qmi_linear_rows_parts' partial products (n_parts in
+ * {1, 2, 4, 8}, n % 8 == 0, y 16-byte aligned with y_stride % 8 == 0). */
+int qmi_sum_parts(const float* parts, int64_t n_parts, int64_t m, int64_t n, uint16_t* y,
+                  int64_t y_stride, void* stream);
+
+/*
+ * Prefill projection y = x W^T for up to 2^20 rows: arguments, rounding points
+ * and layout rules of qmi_linear_rows, with k % 64 == 0.  Replaces the bf16
+ * nn.Linear calls of a prefill step (qwen3_naive.py:427-428, :692-702).
+ */
+int qmi_linear_tiles(const uint16_t* x, int64_t x_stride, const uint16_t* w, int64_t w_stride,
+                     int64_t m, int64_t n, int64_t k, int32_t activation, uint16_t* y,
+                     int64_t y_stride, void* stream);
+
+/*
+ * One decoder layer over the new tokens of a prefill step
+ * (Qwen3DecoderLayer.forward_prefill, qwen3_naive.py:719-745): input norm (of
+ * x, or of x + residual), qkv projection, QK-norm + RoPE + KV store, varlen
+ * attention over the paged cache, o_proj, residual add + norm, SwiGLU MLP.
+ * Writes out [n_tok, hidden] (the MLP's output) and residual_out (the sum
+ * that it is to be added to), both contiguous.  Every member means what it
+ * means in the entry point of that step, whose limits apply; norm weights
+ * are bf16, projections [n, k] without bias.  workspace: 16-byte aligned,
+ * qmi_prefill_layer_workspace_bytes(...) bytes, any contents;
+ * attn_workspace: as qmi_varlen_prefill_attention's workspace.
+ */
+typedef struct qmi_prefill_layer_args {
+  int64_t n_tok, hidden, num_q_heads, num_kv_heads, head_dim, inter;
+  const uint16_t* x;
+  int64_t x_stride;
+  const uint16_t* residual; /* NULL: the first layer, whose residual is x */
+  int64_t residual_stride;
+  const uint16_t* input_norm;
+  const uint16_t* qkv_weight;
+  int64_t qkv_stride;
+  const uint16_t* q_norm;
+  const uint16_t* k_norm;
+  const uint16_t* o_weight;
+  int64_t o_stride;
+  const uint16_t* post_norm;
+  const uint16_t* gate_up_weight;
+  int64_t gate_up_stride;
+  const uint16_t* down_weight;
+  int64_t down_stride;
+  const int64_t* positions;
+  const float* cos_sin_cache;
+  int64_t max_position;
+  uint16_t* k_cache;
+  uint16_t* v_cache;
+  int64_t num_blocks, block_size;
+  const int32_t* slot_mapping;
+  const int32_t* cu_seqlens_q;
+  const int32_t* cu_seqlens_k;
+  const int32_t* block_table;
+  int64_t bt_stride, bt_width, batch, max_seqlen_q, max_seqlen_k;
+  uint16_t* out;
+  uint16_t* residual_out;
+  void* workspace;
+  int64_t workspace_bytes;
+  float* attn_workspace;
+  int64_t attn_workspace_bytes;
+  float eps, qk_eps, post_eps, scale;
+} qmi_prefill_layer_args;
+
+int64_t qmi_prefill_layer_workspace_bytes(int64_t n_tok, int64_t hidden, int64_t num_q_heads,
+                                          int64_t num_kv_heads, int64_t head_dim, int64_t inter);
+int qmi_prefill_layer(const qmi_prefill_layer_args* args, void* stream);
+
 /*
  * Row-wise log-softmax gathered at one token per row.
  * Replaces `F.log_softmax(logits.float(), -1).gather(-1, ids)` of

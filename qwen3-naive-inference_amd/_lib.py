@@ -84,6 +84,12 @@ SIGNATURES: dict[str, tuple] = {
                                              _c_p, _c_i64, _c_p]),
     "qmi_add_rms_norm_parts": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_p, _c_i64, _c_p, _c_i64,
                                               _c_p, _c_p, _c_i64, _c_i64, _c_f32, _c_p]),
+    "qmi_sum_parts": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_p]),
+    "qmi_linear_tiles": (ctypes.c_int, [_c_p, _c_i64, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i32,
+                                        _c_p, _c_i64, _c_p]),
+    "qmi_prefill_layer_workspace_bytes": (_c_i64, [_c_i64] * 6),
+    # The argument struct as bytes (kernels.PREFILL_LAYER_ARGS).
+    "qmi_prefill_layer": (ctypes.c_int, [ctypes.c_char_p, _c_p]),
     "qmi_logprob_gather": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_p, _c_i64, _c_i64, _c_i64,
                                           _c_i64, _c_i64, _c_p, _c_p, _c_p]),
     "qmi_grpo_advantage": (ctypes.c_int, [_c_p, _c_p, _c_i64, _c_f32, _c_p, _c_p]),

@@ -260,6 +260,30 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_parts_kernel(
   }
 }
 
+// y = bf16(sum_s part[s]), summed in part order: 8 columns per lane.
+template <int S>
+__global__ __launch_bounds__(256) void sum_parts_kernel(const float* __restrict__ part, int64_t mn,
+                                                        uint16_t* __restrict__ y, int n8,
+                                                        int64_t y_stride) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (8 * i >= mn) return;
+  f32x4_t pa[S], pb[S];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    pa[s] = *reinterpret_cast<const f32x4_t*>(part + s * mn + 8 * i);
+    pb[s] = *reinterpret_cast<const f32x4_t*>(part + s * mn + 8 * i + 4);
+  }
+  f32x4_t a = pa[0], b = pb[0];
+#pragma unroll
+  for (int s = 1; s < S; ++s) {
+    a += pa[s];
+    b += pb[s];
+  }
+  *reinterpret_cast<uint4*>(y + i / n8 * y_stride + i % n8 * 8) =
+      make_uint4(pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]), pack_bf16x2(b[0], b[1]),
+                 pack_bf16x2(b[2], b[3]));
+}
+
 inline bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 inline bool al8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; }
 
@@ -410,5 +434,31 @@ extern "C" int qmi_add_rms_norm_parts(const float* parts, int64_t n_parts, int64
     QMI_NP(8)
   }
 #undef QMI_NP
+  QMI_RETURN_LAUNCH_STATUS();
+}
+
+extern "C" int qmi_sum_parts(const float* parts, int64_t n_parts, int64_t m, int64_t n, uint16_t* y,
+                             int64_t y_stride, void* stream) {
+  if (m < 0 || n <= 0 || n_parts <= 0) return QMI_E_BAD_SHAPE;
+  if (m == 0) return QMI_OK;
+  if (!parts || !y) return QMI_E_NULL_POINTER;
+  if (n % 8 || n > (1 << 20) || m > (1 << 20) ||
+      (n_parts != 1 && n_parts != 2 && n_parts != 4 && n_parts != 8))
+    return QMI_E_UNSUPPORTED;
+  if (y_stride < n || y_stride % 8 || !al16(parts) || !al16(y)) return QMI_E_BAD_STRIDE;
+  const unsigned grid = (unsigned)((m * n / 8 + 255) / 256);
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+#define QMI_SP(SS)                                                                                \
+  case SS:                                                                                        \
+    hipLaunchKernelGGL(sum_parts_kernel<SS>, dim3(grid), dim3(256), 0, st, parts, m * n, y,       \
+                       (int)(n / 8), y_stride);                                                   \
+    break;
+  switch (n_parts) {
+    QMI_SP(1)
+    QMI_SP(2)
+    QMI_SP(4)
+    QMI_SP(8)
+  }
+#undef QMI_SP
   QMI_RETURN_LAUNCH_STATUS();
 }

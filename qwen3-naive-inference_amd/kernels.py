@@ -8,6 +8,8 @@ never allocate, synchronise or read device data on the host.
 """
 from __future__ import annotations
 
+import struct
+
 import torch
 
 from ._lib import check, lib, stream_handle
@@ -603,6 +605,118 @@ def add_rms_norm_parts(x: RowParts, residual: torch.Tensor, weight: torch.Tensor
                                        stream_handle(r2.device)),
           "add_rms_norm_parts")
     return y.view(residual.shape), r_out.view(residual.shape)
+
+
+def linear_tiles(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = False) -> torch.Tensor:
+    """``linear_rows`` for prefill batches (any number of rows, K % 64 == 0)."""
+    x2 = _rows2d("x", x)
+    _require_cuda("weight", weight)
+    _require_dtype("weight", weight, torch.bfloat16)
+    w = _weight16(weight)
+    m, k = x2.shape
+    n = w.shape[0] // 2 if swiglu else w.shape[0]
+    if w.dim() != 2 or w.shape[1] != k or (swiglu and w.shape[0] % 2):
+        raise ValueError(f"linear_tiles: x {tuple(x.shape)} / weight {tuple(weight.shape)} mismatch")
+    y = torch.empty((m, n), dtype=torch.bfloat16, device=x2.device)
+    check(lib().qmi_linear_tiles(x2.data_ptr(), x2.stride(0), w.data_ptr(), w.stride(0), m, n, k,
+                                 1 if swiglu else 0, y.data_ptr(), y.stride(0),
+                                 stream_handle(x2.device)),
+          "linear_tiles")
+    return y
+
+
+# ---------------------------------------------------------------------------
+# One decoder layer of a prefill step (qwen3_naive.py:719-745)
+# ---------------------------------------------------------------------------
+# qmi_prefill_layer_args: 44 64-bit members, then 4 floats.
+PREFILL_LAYER_ARGS = struct.Struct("@44q4f")
+# Up to this much output (rows x columns of the widest projection) the layer
+# runs on qmi_linear_tiles: at 2,048 rows of hidden 1024 / MLP 3072 its four
+# projections take 83 us against the library GEMM's 94, at 4,096 rows 154
+# against 152 and at 8,192 300 against 249, where the GPU work also hides the
+# library's host time.
+PREFILL_LAYER_ROWS = 2048
+PREFILL_LAYER_OUTPUT = 2048 * 6144
+
+
+def _plain(t: torch.Tensor, dtype: torch.dtype, device: int) -> bool:
+    return (t.dtype == dtype and t.get_device() == device and t.is_contiguous()
+            and t.data_ptr() % 16 == 0)
+
+
+def prefill_layer(x, residual, norms, mats, eps, positions, cos_sin_cache, num_q_heads, num_kv_heads,
+                  k_cache, v_cache, slot_mapping, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
+                  max_seqlen_k, softmax_scale, block_table):
+    """A whole prefill layer in one library call: ``(mlp output, residual)``, or
+    None for a call that the separate entry points have to take (or refuse).
+
+    ``norms``: input, q, k and post-attention norm weights; ``mats``: qkv, o,
+    gate_up and down weights; ``eps``: of the input, q / k and post norms.
+    """
+    if x.dim() != 2 or not x.is_cuda:
+        return None
+    t, hidden = x.shape
+    dev = x.get_device()
+    bf16, i32 = torch.bfloat16, torch.int32
+    qkv_w, o_w, gu_w, down_w = mats
+    q_n, kv_n = num_q_heads * HEAD_DIM, num_kv_heads * HEAD_DIM
+    if down_w.dim() != 2 or k_cache.dim() != 4 or cu_seqlens_q.dim() != 1 or block_table.dim() != 2:
+        return None
+    inter = down_w.shape[1]
+    if not (0 < t <= PREFILL_LAYER_ROWS and t * max(q_n + 2 * kv_n, 2 * inter) <= PREFILL_LAYER_OUTPUT
+            and hidden <= NORM_MAX_WIDTH and hidden % 64 == 0 and inter % 64 == 0
+            and num_q_heads in (num_kv_heads, 2 * num_kv_heads, 4 * num_kv_heads)
+            and qkv_w.shape == (q_n + 2 * kv_n, hidden) and o_w.shape == (hidden, q_n)
+            and gu_w.shape == (2 * inter, hidden) and down_w.shape == (hidden, inter)):
+        return None
+    nb, bs, bsz = k_cache.shape[0], k_cache.shape[1], cu_seqlens_q.shape[0] - 1
+    max_q, max_k = int(max_seqlen_q), int(max_seqlen_k)
+    if not (nb > 0 and bsz > 0 and max_q > 0 and bs == BLOCK_SIZE
+            and k_cache.shape == v_cache.shape == (nb, bs, num_kv_heads, HEAD_DIM)
+            and positions.shape == (t,) and slot_mapping.shape == (t,)
+            and cu_seqlens_k.shape == cu_seqlens_q.shape
+            and block_table.shape[0] == bsz and block_table.shape[1] > 0
+            and block_table.stride(1) == 1 and block_table.dtype == i32
+            and block_table.get_device() == dev
+            and cos_sin_cache.dim() == 2 and cos_sin_cache.shape[1] == HEAD_DIM):
+        return None
+    in_w, qn_w, kn_w, post_w = norms
+    if not (in_w.shape == post_w.shape == (hidden,) and qn_w.shape == kn_w.shape == (HEAD_DIM,)):
+        return None
+    for a in (x, in_w, qn_w, kn_w, post_w, qkv_w, o_w, gu_w, down_w, k_cache, v_cache):
+        if not _plain(a, bf16, dev):
+            return None
+    if residual is not None and not (residual.shape == x.shape and _plain(residual, bf16, dev)):
+        return None
+    if not _plain(cos_sin_cache, torch.float32, dev):
+        return None
+    for a, dtype in ((positions, torch.int64), (slot_mapping, i32), (cu_seqlens_q, i32),
+                     (cu_seqlens_k, i32)):
+        if a.dtype != dtype or a.get_device() != dev or not a.is_contiguous():
+            return None
+    L = lib()
+    device = x.device
+    need = L.qmi_prefill_layer_workspace_bytes(t, hidden, num_q_heads, num_kv_heads, HEAD_DIM, inter)
+    ws = torch.empty(need, dtype=torch.uint8, device=device)
+    attn_need = L.qmi_varlen_prefill_workspace_bytes(bsz, max_q, max_k, num_q_heads, num_kv_heads,
+                                                     block_table.shape[1], 0)
+    attn_ws = _prefill_workspace(device, attn_need) if attn_need > 0 else None
+    out = torch.empty((t, hidden), dtype=bf16, device=device)
+    r_out = torch.empty_like(out)
+    args = PREFILL_LAYER_ARGS.pack(
+        t, hidden, num_q_heads, num_kv_heads, HEAD_DIM, inter,
+        x.data_ptr(), hidden, 0 if residual is None else residual.data_ptr(), hidden,
+        in_w.data_ptr(), qkv_w.data_ptr(), hidden, qn_w.data_ptr(), kn_w.data_ptr(),
+        o_w.data_ptr(), q_n, post_w.data_ptr(), gu_w.data_ptr(), hidden, down_w.data_ptr(), inter,
+        positions.data_ptr(), cos_sin_cache.data_ptr(), cos_sin_cache.shape[0],
+        k_cache.data_ptr(), v_cache.data_ptr(), nb, bs, slot_mapping.data_ptr(),
+        cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(), block_table.data_ptr(),
+        block_table.stride(0), block_table.shape[1], bsz, max_q, max_k,
+        out.data_ptr(), r_out.data_ptr(), ws.data_ptr(), need,
+        0 if attn_ws is None else attn_ws.data_ptr(), attn_need,
+        *eps, softmax_scale)
+    check(L.qmi_prefill_layer(args, stream_handle(device)), "prefill_layer")
+    return out, r_out
 
 
 # ---------------------------------------------------------------------------

@@ -309,8 +309,43 @@ class Qwen3DecoderLayer(nn.Module):
         x = self.self_attn(self.input_layernorm(x)) + x
         return self.mlp(self.post_attention_layernorm(x)) + x
 
+    def _prefill_native(self, x, positions, cu_q, cu_k, max_q, max_k, slots, tables, residual):
+        """The layer as one library call, or None: a call whose modules are
+        hooked, replaced or tracked by autograd, or that ``K.prefill_layer``
+        does not take, goes through the modules."""
+        sub = self._modules
+        attn, mlp = sub.get("self_attn"), sub.get("mlp")
+        if (tables is None or type(attn) is not Qwen3Attention or type(mlp) is not Qwen3MLP
+                or attn.k_cache is None or nn.modules.module._has_any_global_hook()
+                or torch.is_autocast_enabled("cuda") or _prefill_methods() != _PREFILL_METHODS):
+            return None
+        a, m = attn._modules, mlp._modules
+        norms = (sub.get("input_layernorm"), a.get("q_norm"), a.get("k_norm"),
+                 sub.get("post_attention_layernorm"))
+        mats = (a.get("qkv_proj"), a.get("o_proj"), m.get("gate_up_proj"), m.get("down_proj"))
+        for group, cls in (((attn, mlp), None), (norms, RMSNorm), (mats, nn.Linear)):
+            for mod in group:
+                if ((cls is not None and type(mod) is not cls) or mod._forward_hooks
+                        or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks
+                        or "forward" in mod.__dict__ or "forward_prefill" in mod.__dict__):
+                    return None
+        if any(mod._parameters.get("bias", mod) is not None for mod in mats):
+            return None
+        norm_w = [mod._parameters.get("weight") for mod in norms]
+        mat_w = [mod._parameters.get("weight") for mod in mats]
+        if any(w is None for w in norm_w + mat_w) or not _use_kernels(x, *norm_w, *mat_w):
+            return None
+        return K.prefill_layer(
+            x, residual, norm_w, mat_w, (norms[0].eps, attn.eps, norms[3].eps), positions,
+            attn._cos_sin(x.device), attn.num_heads, attn.num_kv_heads, attn.k_cache, attn.v_cache,
+            slots, cu_q, cu_k, max_q, max_k, attn.scale, tables)
+
     def forward_prefill(self, x, positions, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
                         max_seqlen_k, block_mapping, block_tables=None, residual=None):
+        done = self._prefill_native(x, positions, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
+                                    max_seqlen_k, block_mapping, block_tables, residual)
+        if done is not None:
+            return done
         if residual is None:
             h, residual = self.input_layernorm(x), x
         else:
@@ -329,6 +364,17 @@ class Qwen3DecoderLayer(nn.Module):
         h = self.self_attn.forward_decode(h, positions, context_lens, block_tables, slot_mapping)
         h, residual = self.post_attention_layernorm(h, residual)
         return self.mlp.forward_decode(h), residual
+
+
+def _prefill_methods():
+    """What the module path of a prefill layer calls; a program may replace any
+    of them, and then the layer runs through the modules."""
+    return (Qwen3Attention.forward_prefill, Qwen3Attention._project_store, Qwen3Attention._cos_sin,
+            Qwen3MLP.forward, RMSNorm.forward, nn.Linear.forward, K.rms_norm, K.add_rms_norm,
+            K.qk_norm_rope_store, K.varlen_prefill_attention, K.silu_mul)
+
+
+_PREFILL_METHODS = _prefill_methods()
 
 
 class Qwen3Model(nn.Module):
