@@ -74,13 +74,21 @@ __device__ __forceinline__ int64_t active_wgs(int64_t total, int64_t n_wg) {
   return want < 1 ? 1 : (want < n_wg ? want : n_wg);
 }
 
+// a / b of non-negative values: the schedule's few divisions sit on the serial
+// chain before the first load, and a 64-bit division is ~150 dependent
+// instructions against ~20 of the 32-bit one that almost every call needs.
+__device__ __forceinline__ int64_t div_nn(int64_t a, int64_t b) {
+  if ((((uint64_t)a | (uint64_t)b) >> 32) == 0) return (int64_t)((uint32_t)a / (uint32_t)b);
+  return a / b;
+}
+
 __device__ __forceinline__ int64_t range_start(int64_t w, int64_t total, int64_t n_wg) {
-  return w * total / n_wg;
+  return div_nn(w * total, n_wg);
 }
 
 // Workgroup owning global step s: the largest w with range_start(w) <= s.
 __device__ __forceinline__ int64_t owner_of(int64_t s, int64_t total, int64_t n_wg) {
-  int64_t w = ((s + 1) * n_wg - 1) / total;
+  int64_t w = div_nn((s + 1) * n_wg - 1, total);
   return w < n_wg - 1 ? w : n_wg - 1;
 }
 
@@ -153,7 +161,7 @@ __device__ __forceinline__ bool use_unit_mode(int64_t total, int max_steps, int6
                                               int64_t n_wg_grid, int64_t n_bal) {
   if (total == 0 || n_units > n_wg_grid) return false;
   const int64_t n_act = active_wgs(total, n_bal);
-  const int64_t share = (total + n_act - 1) / n_act;
+  const int64_t share = div_nn(total + n_act - 1, n_act);
   return (int64_t)max_steps * 10 <= share * 11;
 }
 
@@ -301,7 +309,7 @@ void decode_streamk_split(
     while ((int64_t)NHG * off[b + 1] <= s) ++b;  // skip empty sequences
     const int64_t steps_b = off[b + 1] - off[b];
     const int64_t sq0 = (int64_t)NHG * off[b];
-    const int hgi = (int)((s - sq0) / steps_b);   // head group of the unit
+    const int hgi = NHG == 1 ? 0 : (int)div_nn(s - sq0, steps_b);   // head group of the unit
     const int64_t sb = sq0 + hgi * steps_b;       // the unit's steps: [sb, sb + steps_b)
     const int64_t seg_end = min(sb + steps_b, s_end);
     const int h = hgi * HG + hl;                  // this lane's KV head
@@ -584,24 +592,46 @@ __global__ __launch_bounds__(kThreads) void decode_streamk_merge(
   float M = kNegBig, Ls = 0.f, A[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) A[e] = 0.f;
-  for (int64_t ww = w0 + grp; ww <= w1; ww += kGroups) {
-    const int64_t r0 = range_start(ww, total, n_act);
-    if (r0 == range_start(ww + 1, total, n_act)) continue;  // empty range: owns no slot
-    const int slot = (r0 >= ub) ? 0 : 1;
-    const float* p = ws + ((ww * 2 + slot) * HQ + ql) * kSlotStride;
-    const float mw = p[kHeadDim], lw = p[kHeadDim + 1];
-    const f32x4_t a0 = *reinterpret_cast<const f32x4_t*>(p + d0);
-    const f32x4_t a1 = *reinterpret_cast<const f32x4_t*>(p + d0 + 4);
-    const float mn = fmaxf(M, mw);
-    const float s1 = fast_exp2(M - mn), s2 = fast_exp2(mw - mn);
-    Ls = Ls * s1 + lw * s2;
+  // N slots of the group in flight at once; a workgroup with an empty step
+  // range owns no slot, and w0, which owns step ub, stands in for it.
+  auto walk = [&](auto n_c) {
+    constexpr int N = decltype(n_c)::value;
+    for (int64_t wb = w0 + grp; wb <= w1; wb += N * kGroups) {
+      float mw[N], lw[N];
+      f32x4_t a0[N], a1[N];
+      bool ok[N];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      A[e] = A[e] * s1 + a0[e] * s2;
-      A[4 + e] = A[4 + e] * s1 + a1[e] * s2;
+      for (int j = 0; j < N; ++j) {
+        const int64_t ww = wb + j * kGroups;
+        const int64_t r0 = range_start(ww, total, n_act);
+        ok[j] = ww <= w1 && r0 != range_start(ww + 1, total, n_act);
+        const int64_t slot = ok[j] ? ww * 2 + (r0 >= ub ? 0 : 1)
+                                   : w0 * 2 + (range_start(w0, total, n_act) >= ub ? 0 : 1);
+        const float* p = ws + (slot * HQ + ql) * kSlotStride;
+        mw[j] = p[kHeadDim];
+        lw[j] = p[kHeadDim + 1];
+        a0[j] = *reinterpret_cast<const f32x4_t*>(p + d0);
+        a1[j] = *reinterpret_cast<const f32x4_t*>(p + d0 + 4);
+      }
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        if (!ok[j]) continue;
+        const float mn = fmaxf(M, mw[j]);
+        const float s1 = fast_exp2(M - mn), s2 = fast_exp2(mw[j] - mn);
+        Ls = Ls * s1 + lw[j] * s2;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          A[e] = A[e] * s1 + a0[j][e] * s2;
+          A[4 + e] = A[4 + e] * s1 + a1[j][e] * s2;
+        }
+        M = mn;
+      }
     }
-    M = mn;
-  }
+  };
+  if (w1 - w0 < kGroups)
+    walk(std::integral_constant<int, 1>{});
+  else
+    walk(std::integral_constant<int, 4>{});
   if (lane16 == 0) {
     s_ml[grp][0] = M;
     s_ml[grp][1] = Ls;
