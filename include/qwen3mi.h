@@ -351,6 +351,22 @@ int qmi_add_rms_norm_parts(const float* parts, int64_t n_parts, int64_t m,
                            const uint16_t* weight, uint16_t* y, int64_t y_stride, int64_t n,
                            float eps, void* stream);
 
+/*
+ * Decode projection for at most 16 rows, k in {1024, 2048, 3072, 4096}:
+ * y = x' W^T (activation as qmi_linear_rows) with x' = x, or with norm_weight
+ * [k] given x' = rms_norm(x) * norm_weight, or with residual given too
+ * residual_out = bf16(x + residual) and x' the norm of that sum
+ * (qmi_add_rms_norm and the projection after it, qwen3_naive.py:163-169,
+ * :654, :699-701, in one launch; the same rounding points).  n % 16 == 0;
+ * residual_out must overlap no input; rows 16-byte
+ * aligned with strides % 8 == 0.
+ */
+int qmi_linear_small(const uint16_t* x, int64_t x_stride, const uint16_t* residual,
+                     int64_t residual_stride, uint16_t* residual_out, int64_t residual_out_stride,
+                     const uint16_t* norm_weight, float eps, const uint16_t* w, int64_t w_stride,
+                     int64_t m, int64_t n, int64_t k, int32_t activation, uint16_t* y,
+                     int64_t y_stride, void* stream);
+
 /* y[m][n] = bf16(sum_s parts[s]) of qmi_linear_rows_parts' partial products (n_parts in
  * {1, 2, 4, 8}, n % 8 == 0, y 16-byte aligned with y_stride % 8 == 0). */
 int qmi_sum_parts(const float* parts, int64_t n_parts, int64_t m, int64_t n, uint16_t* y,

@@ -84,6 +84,8 @@ SIGNATURES: dict[str, tuple] = {
                                              _c_p, _c_i64, _c_p]),
     "qmi_add_rms_norm_parts": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_p, _c_i64, _c_p, _c_i64,
                                               _c_p, _c_p, _c_i64, _c_i64, _c_f32, _c_p]),
+    "qmi_linear_small": (ctypes.c_int, [_c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_f32, _c_p,
+                                        _c_i64, _c_i64, _c_i64, _c_i64, _c_i32, _c_p, _c_i64, _c_p]),
     "qmi_sum_parts": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_p]),
     "qmi_linear_tiles": (ctypes.c_int, [_c_p, _c_i64, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i32,
                                         _c_p, _c_i64, _c_p]),

@@ -607,6 +607,67 @@ def add_rms_norm_parts(x: RowParts, residual: torch.Tensor, weight: torch.Tensor
     return y.view(residual.shape), r_out.view(residual.shape)
 
 
+class PendingNorm:
+    """The rows ``rms_norm(x)`` or ``rms_norm(x + residual)``, not yet computed:
+    the projection that reads them (``linear_small``) computes them and leaves
+    the sum in ``sum``."""
+
+    __slots__ = ("x", "residual", "weight", "eps", "sum")
+
+    def __init__(self, x: torch.Tensor, residual: torch.Tensor | None, weight: torch.Tensor,
+                 eps: float):
+        self.x, self.residual, self.weight, self.eps = x, residual, weight, eps
+        self.sum = x if residual is None else None
+
+    def project(self, weight: torch.Tensor, swiglu: bool = False) -> torch.Tensor:
+        y, total = linear_small(self.x, weight, swiglu, self.weight, self.eps, self.residual)
+        if total is not None:
+            self.sum = total
+        return y
+
+
+LINEAR_SMALL_ROWS = 16
+LINEAR_SMALL_K = (1024, 2048, 3072, 4096)
+
+
+def linear_small_ok(x: torch.Tensor) -> bool:
+    """Whether ``linear_small`` takes a product that ``linear_rows_ok`` holds for."""
+    return x.shape[0] <= LINEAR_SMALL_ROWS and x.shape[1] in LINEAR_SMALL_K
+
+
+def linear_small(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = False,
+                 norm: torch.Tensor | None = None, eps: float = 0.0,
+                 residual: torch.Tensor | None = None):
+    """``linear_rows`` for at most 16 rows; with ``norm`` of ``rms_norm(x, norm, eps)``,
+    with ``residual`` too of ``add_rms_norm(x, residual, norm, eps)``.  Returns
+    ``(y, residual sum or None)``."""
+    if not (linear_rows_ok(x, weight, swiglu) and linear_small_ok(x)):
+        raise ValueError(f"linear_small: unsupported x {tuple(x.shape)} / weight "
+                         f"{tuple(weight.shape)}")
+    x2 = _rows2d("x", x)
+    w = _weight16(weight)
+    m, k = x2.shape
+    n = w.shape[0] // 2 if swiglu else w.shape[0]
+    nw = r2 = r_out = None
+    if norm is not None:
+        _require_cuda("norm", norm)
+        nw = _dense16(norm.to(torch.bfloat16))
+        if nw.shape != (k,):
+            raise ValueError(f"norm must be [{k}], got {tuple(norm.shape)}")
+    if residual is not None:
+        r2 = _rows2d("residual", residual)
+        if nw is None or r2.shape != x2.shape:
+            raise ValueError("residual needs norm and the shape of x")
+        r_out = torch.empty((m, k), dtype=torch.bfloat16, device=x2.device)
+    y = torch.empty((m, n), dtype=torch.bfloat16, device=x2.device)
+    check(lib().qmi_linear_small(x2.data_ptr(), x2.stride(0), _ptr(r2),
+                                 0 if r2 is None else r2.stride(0), _ptr(r_out), k, _ptr(nw),
+                                 float(eps), w.data_ptr(), w.stride(0), m, n, k,
+                                 1 if swiglu else 0, y.data_ptr(), n, stream_handle(x2.device)),
+          "linear_small")
+    return y, r_out
+
+
 def linear_tiles(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = False) -> torch.Tensor:
     """``linear_rows`` for prefill batches (any number of rows, K % 64 == 0)."""
     x2 = _rows2d("x", x)

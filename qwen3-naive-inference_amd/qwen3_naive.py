@@ -79,10 +79,14 @@ def _use_kernels(*tensors: torch.Tensor) -> bool:
 
 def _decode_linear(proj: nn.Linear, x: torch.Tensor, parts: bool = False):
     """A decode-step projection: the HIP decode-batch GEMM for bf16 inference
-    at <= 256 rows (as fp32 partial products when ``parts``: the residual add
-    + RMSNorm that follows sums them), else ``proj(x)``."""
+    at <= 256 rows (as fp32 partial products when ``parts`` and above 16 rows:
+    the residual add + RMSNorm that follows sums them), else ``proj(x)``."""
     w = proj.weight
+    if isinstance(x, K.PendingNorm):  # made for this projection by the layer
+        return x.project(w)
     if proj.bias is None and _use_kernels(x, w) and K.linear_rows_ok(x, w):
+        if K.linear_small_ok(x):
+            return K.linear_small(x, w)[0]
         if parts and w.shape[0] <= K.NORM_MAX_WIDTH:  # the norm that sums them takes the width
             return K.linear_rows_parts(x, w)
         return K.linear_rows(x, w)
@@ -207,7 +211,7 @@ class Qwen3Attention(nn.Module):
         rotated k and v land in the cache rows ``slots``."""
         qkv = _decode_linear(self.qkv_proj, x) if decode else self.qkv_proj(x)
         return K.qk_norm_rope_store(qkv, self.q_norm.weight, self.k_norm.weight, positions,
-                                    self._cos_sin(x.device), self.num_heads, self.num_kv_heads,
+                                    self._cos_sin(qkv.device), self.num_heads, self.num_kv_heads,
                                     self.eps, self.k_cache, self.v_cache, slots)
 
     # ----- batch path (training / no-cache eager forward, qwen3_naive.py:553-593) -----
@@ -250,16 +254,17 @@ class Qwen3Attention(nn.Module):
     def forward_decode(self, x, positions, context_lens, block_tables, slot_mapping=None):
         """One new token per sequence: store its K/V at ``slot_mapping`` (derived
         from the tables when None) and attend over ``context_lens + 1`` keys."""
-        batch = x.shape[0]
+        rows = x.x if isinstance(x, K.PendingNorm) else x
+        batch = rows.shape[0]
         if slot_mapping is None:
             ctx = context_lens.long()
             blk = block_tables.long().gather(1, (ctx // BLOCK_SIZE)[:, None])[:, 0]
             slot_mapping = (blk * BLOCK_SIZE + ctx % BLOCK_SIZE).to(torch.int32)
-        if (self.decode_fused_qkv and self.decode_pages_per_split <= 0 and _use_kernels(x)
+        if (self.decode_fused_qkv and self.decode_pages_per_split <= 0 and _use_kernels(rows)
                 and K.decode_qkv_ok(self.num_heads, self.num_kv_heads, self.head_dim, batch)):
             qkv = _decode_linear(self.qkv_proj, x)
             o = K.paged_decode_attention_qkv(
-                qkv, self.q_norm.weight, self.k_norm.weight, positions, self._cos_sin(x.device),
+                qkv, self.q_norm.weight, self.k_norm.weight, positions, self._cos_sin(qkv.device),
                 self.num_heads, self.num_kv_heads, self.eps, self.k_cache, self.v_cache,
                 slot_mapping, context_lens, block_tables, self.scale,
                 pages_per_split=self.decode_pages_per_split)
@@ -291,8 +296,12 @@ class Qwen3MLP(nn.Module):
         partial products for the next residual add + RMSNorm (HIP decode-batch
         GEMMs at <= 256 rows; otherwise as ``forward``)."""
         w = self.gate_up_proj.weight
+        if isinstance(x, K.PendingNorm):
+            return _decode_linear(self.down_proj, x.project(w, swiglu=True), parts=True)
         if (self.gate_up_proj.bias is None and _use_kernels(x, w)
                 and K.linear_rows_ok(x, w, swiglu=True)):
+            if K.linear_small_ok(x):
+                return _decode_linear(self.down_proj, K.linear_small(x, w, swiglu=True)[0], parts=True)
             return _decode_linear(self.down_proj, K.linear_rows(x, w, swiglu=True), parts=True)
         return self.forward(x)
 
@@ -355,8 +364,45 @@ class Qwen3DecoderLayer(nn.Module):
         h, residual = self.post_attention_layernorm(h, residual)
         return self.mlp(h), residual
 
+    def _norms_in_projections(self, x, residual) -> bool:
+        """Whether a decode step's two norms run inside the projections that
+        read them: few enough rows, and plain modules."""
+        sub = self._modules
+        attn, mlp, n1, n2 = (sub.get(k) for k in ("self_attn", "mlp", "input_layernorm",
+                                                  "post_attention_layernorm"))
+        if (type(x) is not torch.Tensor or x.dim() != 2 or type(attn) is not Qwen3Attention
+                or type(mlp) is not Qwen3MLP or nn.modules.module._has_any_global_hook()
+                or (Qwen3Attention.forward_decode, Qwen3MLP.forward_decode, RMSNorm.forward,
+                    K.rms_norm, K.add_rms_norm) != _DECODE_METHODS):
+            return False
+        for mod in (n1, n2):
+            if (type(mod) is not RMSNorm or mod._forward_hooks or mod._forward_pre_hooks
+                    or mod._backward_hooks or mod._backward_pre_hooks or "forward" in mod.__dict__
+                    or mod.weight.shape != x.shape[1:]):
+                return False
+        if "forward_decode" in attn.__dict__ or "forward_decode" in mlp.__dict__:
+            return False
+        qkv, o, gu = attn.qkv_proj, attn.o_proj, mlp.gate_up_proj
+        if not (qkv.bias is None and o.bias is None and gu.bias is None
+                and _use_kernels(x, n1.weight, n2.weight, qkv.weight, o.weight, gu.weight)):
+            return False
+        if residual is not None and not (type(residual) is torch.Tensor and residual.is_cuda
+                                         and residual.shape == x.shape
+                                         and residual.dtype == torch.bfloat16):
+            return False
+        return (K.linear_small_ok(x) and K.linear_rows_ok(x, qkv.weight)
+                and K.linear_rows_ok(x, gu.weight, swiglu=True)
+                and o.weight.dtype == torch.bfloat16 and o.weight.shape[0] == x.shape[1]
+                and o.weight.shape[1] == attn.q_size and attn.q_size in K.LINEAR_SMALL_K)
+
     def forward_decode(self, x, positions, context_lens, block_tables, slot_mapping=None,
                        residual=None):
+        if self._norms_in_projections(x, residual):
+            h = K.PendingNorm(x, residual, self.input_layernorm.weight, self.input_layernorm.eps)
+            o = self.self_attn.forward_decode(h, positions, context_lens, block_tables, slot_mapping)
+            h = K.PendingNorm(o, h.sum, self.post_attention_layernorm.weight,
+                              self.post_attention_layernorm.eps)
+            return self.mlp.forward_decode(h), h.sum
         if residual is None:
             h, residual = self.input_layernorm(x), x
         else:
@@ -375,6 +421,8 @@ def _prefill_methods():
 
 
 _PREFILL_METHODS = _prefill_methods()
+_DECODE_METHODS = (Qwen3Attention.forward_decode, Qwen3MLP.forward_decode, RMSNorm.forward,
+                   K.rms_norm, K.add_rms_norm)
 
 
 class Qwen3Model(nn.Module):

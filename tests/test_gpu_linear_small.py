@@ -1,0 +1,92 @@
+"""Decode projections of at most 16 rows (qmi_linear_small) against fp32 torch
+products, and the decode layer whose norms run inside them against its modules.
+
+Tolerances: one bf16 rounding of an fp32 sum (8 significant bits: half an ulp
+is at most 2^-8 of the value; SwiGLU rounds g, u and the result); the
+norm's rows may differ from add_rms_norm's by flipped roundings (another order
+of the sum of squares), as may SwiGLU's g and u."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(a, b):
+    return ((a.double() - b.double()).norm() / b.double().norm()).item()
+
+
+# The fewest and most rows and those around one per wave; a grid of one
+# workgroup (which writes every row of the residual sum) and larger ones.
+@pytest.mark.parametrize("m", [1, 7, 8, 9, 16])
+@pytest.mark.parametrize("n", [16, 48, 4096])
+@pytest.mark.parametrize("k", [1024, 2048, 3072, 4096])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_linear_small(pkg, gpu, m, n, k, swiglu):
+    K = pkg.kernels
+    g = torch.Generator(device=gpu).manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device=gpu).bfloat16()
+    r = torch.randn(m, k + 8, generator=g, device=gpu).bfloat16()[:, :k]
+    w = (torch.randn((2 * n if swiglu else n), k, generator=g, device=gpu) * 0.05).bfloat16()
+    nw = torch.rand(k, generator=g, device=gpu).bfloat16() + 0.5
+
+    def ref(rows):
+        y = rows.float() @ w.float().T
+        if swiglu:
+            gate, up = y.bfloat16().float().chunk(2, -1)
+            y = torch.nn.functional.silu(gate) * up
+        return y
+
+    tol = 2 ** -7 if swiglu else 2 ** -8
+    y, s = K.linear_small(x, w, swiglu)
+    assert s is None and y.shape == (m, n) and _rel(y, ref(x)) < tol
+    y, s = K.linear_small(x, w, swiglu, nw, 1e-6)
+    assert s is None and _rel(y, ref(K.rms_norm(x, nw, 1e-6))) < 2 * tol
+    y, s = K.linear_small(x, w, swiglu, nw, 1e-6, r)
+    h, total = K.add_rms_norm(x, r, nw, 1e-6)
+    assert torch.equal(s, total) and _rel(y, ref(h)) < 2 * tol
+
+
+def test_linear_small_refuses(pkg, gpu):
+    K = pkg.kernels
+    x = torch.zeros(17, 1024, device=gpu).bfloat16()
+    w = torch.zeros(32, 1024, device=gpu).bfloat16()
+    for a, b, sw in ((x, w, False), (x[:4], w[:24], False), (x[:4, :512], w[:, :512], False),
+                     (x[:4], w[:12], True)):
+        with pytest.raises(ValueError):
+            K.linear_small(a, b, sw)
+
+
+@pytest.mark.parametrize("batch", [1, 16, 17])
+@pytest.mark.parametrize("first", [False, True])
+@pytest.mark.parametrize("fused_qkv", [False, True])
+def test_decode_layer_matches_modules(pkg, gpu, batch, first, fused_qkv):
+    torch.manual_seed(0)
+    cfg = pkg.Qwen3Config(hidden_size=1024, num_attention_heads=8, num_key_value_heads=4,
+                          intermediate_size=2048, num_hidden_layers=1, max_position_embeddings=1024)
+    layer = pkg.Qwen3DecoderLayer(cfg).to(gpu).bfloat16()
+    layer.self_attn.decode_fused_qkv = fused_qkv
+    with torch.no_grad():
+        for name, p in layer.named_parameters():
+            p.uniform_(0.8, 1.2) if "norm" in name else p.normal_(0, 0.03)
+    kv = [torch.randn(batch * 2, 256, 4, 128, device=gpu).bfloat16() for _ in range(2)]
+    ctx = (torch.arange(batch, dtype=torch.int32, device=gpu) * 29) % 500
+    bt = torch.arange(batch * 2, dtype=torch.int32, device=gpu).view(batch, 2)
+    x = torch.randn(batch, 1024, device=gpu).bfloat16()
+    r = None if first else torch.randn(batch, 1024, device=gpu).bfloat16()
+    res = []
+    for hook in (False, True):
+        layer.self_attn.k_cache, layer.self_attn.v_cache = kv[0].clone(), kv[1].clone()
+        seen = []
+        h = (layer.input_layernorm.register_forward_hook(lambda *_: seen.append(1)) if hook else None)
+        with torch.no_grad():
+            assert layer._norms_in_projections(x, r) == (batch <= 16 and not hook)
+            y, s = layer.forward_decode(x, ctx.long(), ctx, bt, None, r)
+        res.append([t.dense() if isinstance(t, pkg.kernels.RowParts) else t
+                    for t in (y, s, layer.self_attn.k_cache, layer.self_attn.v_cache)])
+        if h:
+            h.remove()
+            assert seen
+    for a, b in zip(*res):
+        assert a.shape == b.shape and _rel(a, b) < 0.02
+    layer.self_attn.k_cache, layer.self_attn.v_cache = kv
+    assert not layer._norms_in_projections(x, r)  # weights tracked by autograd

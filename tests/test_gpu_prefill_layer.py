@@ -1,9 +1,9 @@
 """Prefill projections (qmi_linear_tiles) and the prefill layer as one library
 call (qmi_prefill_layer) against fp32 torch products and the layer's modules.
 
-Tolerances: a projection rounds an fp32 sum once to bf16 (half an ulp, 2^-9
-relative; 2-norm of the error over 2-norm of the result ~ 2^-9 / sqrt(3)); the
-SwiGLU form rounds three times.  Two layers that differ in the order of their
+Tolerances: a projection rounds an fp32 sum once to bf16 (8 significant bits:
+half an ulp is at most 2^-8 of the value); the SwiGLU form rounds g, u and the
+result.  Two layers that differ in the order of their
 fp32 sums differ by flipped roundings along six bf16 steps."""
 import pytest
 import torch
@@ -32,7 +32,7 @@ def test_linear_tiles(pkg, gpu, m, n, k, swiglu):
     if swiglu:
         gate, up = want.bfloat16().float().chunk(2, -1)
         want = torch.nn.functional.silu(gate) * up
-    assert _rel(y[:m], want) < (2 ** -8 if swiglu else 2 ** -9)
+    assert _rel(y[:m], want) < (2 ** -7 if swiglu else 2 ** -8)
     assert bool((y[m] == 7).all())  # nothing past the last row
     assert torch.equal(y[:m], pkg.kernels.linear_tiles(x, w, swiglu))
 
@@ -40,7 +40,7 @@ def test_linear_tiles(pkg, gpu, m, n, k, swiglu):
 def test_linear_tiles_strides(pkg, gpu):
     x = torch.randn(70, 200, device=gpu).bfloat16()[:, 8:136]
     w = torch.randn(48, 160, device=gpu).bfloat16()[:, :128]
-    assert _rel(pkg.kernels.linear_tiles(x, w), x.float() @ w.float().T) < 2 ** -9
+    assert _rel(pkg.kernels.linear_tiles(x, w), x.float() @ w.float().T) < 2 ** -8
     with pytest.raises(Exception):
         pkg.kernels.linear_tiles(x[:, :96], w[:, :96])  # K % 64
 
