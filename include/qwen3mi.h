@@ -436,6 +436,52 @@ int64_t qmi_prefill_layer_workspace_bytes(int64_t n_tok, int64_t hidden, int64_t
 int qmi_prefill_layer(const qmi_prefill_layer_args* args, void* stream);
 
 /*
+ * Element-wise passes of the training batch (RMSNorm, SwiGLU, QK-norm + RoPE
+ * and the causal mask of the batch forward, qwen3_naive.py:156-169, :553-590,
+ * :695-702, and their gradients), with the fp32 operations and bf16 roundings
+ * of the torch formulas.  Rows: `heads` adjacent rows of n elements (n % 8 ==
+ * 0, <= 65536) in each bf16 row of `stride`; fp32 arrays and dy are
+ * contiguous.  Pointers 16-byte aligned.
+ *   square_rows:  sq = x^2 (its row means are `mean` below)
+ *   norm_apply:   y = bf16(x * rsqrt(mean + eps) * w), heads = 1, y contiguous
+ *   norm_prod:    prod = (dy * w) * x, whose row sums are `dr` below
+ *   norm_grad:    dx (laid out as x) and qmi_norm_grad_parts(rows, n) rows of
+ *                 partial sums of dw
+ *   silu_mul_train: dy NULL: out = bf16(bf16(silu(gate)) * up); else out =
+ *                 the gradient of the packed [rows][2 inter] gate_up
+ *   train_qkv:    packed qkv [batch * t] rows -> normed, rotated q
+ *                 [batch][hq][t][128], k transposed [batch][hq][128][t] and v
+ *                 [batch][hq][t][128] in fp32, KV heads repeated
+ *   train_qkv_grad: gradients of those -> bf16 gradients of the norms' outputs
+ *                 [batch * t][h][128], and v's into the packed d qkv
+ *   train_heads:  fp32 [batch][heads][t][128] -> bf16 [batch][t][heads][128]
+ *                 (to_bf16 1) or back (0)
+ *   scale_mask:   s[row][j] = j > row % t ? masked : s * scale, [rows][t] in place
+ */
+int qmi_square_rows(const uint16_t* x, int64_t rows, int64_t stride, int64_t heads, int64_t n,
+                    float* sq, void* stream);
+int qmi_norm_apply(const uint16_t* x, int64_t rows, int64_t stride, int64_t n, const float* mean,
+                   const uint16_t* w, float eps, uint16_t* y, void* stream);
+int qmi_norm_prod(const uint16_t* x, int64_t rows, int64_t stride, int64_t heads, int64_t n,
+                  const uint16_t* w, const uint16_t* dy, float* prod, void* stream);
+int64_t qmi_norm_grad_parts(int64_t rows, int64_t n);
+int qmi_norm_grad(const uint16_t* x, int64_t rows, int64_t stride, int64_t heads, int64_t n,
+                  const float* mean, const uint16_t* w, float eps, const uint16_t* dy,
+                  const float* dr, uint16_t* dx, float* dw, void* stream);
+int qmi_silu_mul_train(const uint16_t* gate_up, int64_t rows, int64_t inter, const uint16_t* dy,
+                       uint16_t* out, void* stream);
+int qmi_train_qkv(const uint16_t* qkv, int64_t stride, int64_t batch, int64_t t, int64_t hq,
+                  int64_t hkv, const float* q_mean, const float* k_mean, const uint16_t* q_w,
+                  const uint16_t* k_w, float eps, const float* cache, float* qf, float* kt,
+                  float* vf, void* stream);
+int qmi_train_qkv_grad(int64_t batch, int64_t t, int64_t hq, int64_t hkv, const float* dq,
+                       const float* dkt, const float* dv, const float* cache, uint16_t* dn_q,
+                       uint16_t* dn_k, uint16_t* dqkv, void* stream);
+int qmi_train_heads(float* f, uint16_t* o, int64_t batch, int64_t t, int64_t heads, int32_t to_bf16,
+                    void* stream);
+int qmi_scale_mask(float* s, int64_t rows, int64_t t, float scale, float masked, void* stream);
+
+/*
  * Row-wise log-softmax gathered at one token per row.
  * Replaces `F.log_softmax(logits.float(), -1).gather(-1, ids)` of
  * forward_logprob (qwen3_grpo_train.py:46-53) and the rollout's

@@ -48,7 +48,11 @@ HIPCC_FLAGS = [
 # thread and uses the value only after the next item's loads; the AMDGPU
 # atomic optimizer would rewrite that atomic into a wave-wide form whose
 # result is consumed (and waited for) at once.
+#
+# The training kernels repeat torch's element-wise chains bit for bit, each of
+# whose operations rounds by itself.
 EXTRA_FLAGS = {
+    "train_rows.hip": ["-ffp-contract=off"],
     "varlen_prefill.hip": ["-fno-honor-nans", "-mllvm", "-amdgpu-atomic-optimizer-strategy=None"],
 }
 

@@ -1,0 +1,269 @@
+"""The training batch's element-wise chains as autograd Functions on fused
+HIP kernels (csrc/train_rows.hip).
+
+Each gives the values of the torch formula beside it, in both directions: the
+kernels repeat its fp32 operations and bf16 roundings, sums along a row, the
+softmax and the products are the same torch calls on the same operands.  Only
+the norm weights' gradients are summed in another (fixed) order.  The formula
+serves every call the kernels do not take, and a backward that has to be
+differentiable itself (``create_graph=True``) differentiates the formula.
+"""
+from __future__ import annotations
+
+import torch
+from torch.autograd import forward_ad
+
+from . import kernels as K
+from ._lib import check, lib, stream_handle
+
+HEAD_DIM = K.HEAD_DIM
+F32, BF16 = torch.float32, torch.bfloat16
+
+
+def kernels_ok(*tensors: torch.Tensor) -> bool:
+    """Whether the training kernels take a call on these tensors: plain bf16
+    tensors of one GPU, run eagerly with a gradient wanted of the first.
+    Function transforms (vmap, functional and forward-mode derivatives),
+    tracing and autocast need torch ops."""
+    dev = tensors[0].device
+    if dev.type != "cuda" or not (torch.is_grad_enabled() and tensors[0].requires_grad):
+        return False
+    for t in tensors:
+        if (type(t) not in (torch.Tensor, torch.nn.Parameter) or t.dtype != BF16 or t.device != dev):
+            return False
+    return not (torch.compiler.is_compiling() or torch.jit.is_tracing()
+                or torch.is_autocast_enabled("cuda") or forward_ad._current_level >= 0
+                or torch._C._functorch.peek_interpreter_stack() is not None)
+
+
+def _formula_grads(formula, inputs, needs, grads):
+    """Gradients of ``formula(*inputs)`` that autograd can differentiate again."""
+    with torch.enable_grad():
+        out = formula(*inputs)
+    wanted = [t for t, n in zip(inputs, needs) if n]
+    got = iter(torch.autograd.grad(out, wanted, grads, create_graph=True, allow_unused=True))
+    return tuple(next(got) if n else None for n in needs)
+
+
+def _call(name, device, *args):
+    check(getattr(lib(), name)(*args, stream_handle(device)), name)
+
+
+# ---------------------------------------------------------------------------
+# RMSNorm (qwen3_naive.py:156-162)
+# ---------------------------------------------------------------------------
+def rms_norm_formula(x, weight, eps):
+    xf = x.float()
+    return (xf * torch.rsqrt(xf.pow(2).mean(dim=-1, keepdim=True) + eps)
+            * weight.float()).to(x.dtype)
+
+
+def _mean_square(x, rows, stride, heads, n, shape):
+    """``x.float().pow(2).mean(-1, keepdim=True)`` of ``heads`` adjacent rows of ``n`` per row of ``x``."""
+    sq = torch.empty(shape, dtype=F32, device=x.device)
+    _call("qmi_square_rows", x.device, x.data_ptr(), rows, stride, heads, n, sq.data_ptr())
+    return sq.mean(dim=-1, keepdim=True)
+
+
+def _norm_grad(x, rows, stride, heads, n, shape, mean, w, eps, dy, dx):
+    """Gradients of the norm: ``dx`` is written (laid out as ``x``), the weight's is returned."""
+    prod = torch.empty(shape, dtype=F32, device=w.device)
+    _call("qmi_norm_prod", w.device, x.data_ptr(), rows, stride, heads, n, w.data_ptr(),
+          dy.data_ptr(), prod.data_ptr())
+    dr = prod.sum(dim=-1, keepdim=True)
+    parts = torch.empty((lib().qmi_norm_grad_parts(rows, n), n), dtype=F32, device=w.device)
+    _call("qmi_norm_grad", w.device, x.data_ptr(), rows, stride, heads, n, mean.data_ptr(),
+          w.data_ptr(), eps, dy.data_ptr(), dr.data_ptr(), dx.data_ptr(), parts.data_ptr())
+    return parts.sum(0).to(BF16)
+
+
+def norm_ok(x, weight) -> bool:
+    return (kernels_ok(x, weight) and x.numel() > 0 and x.numel() < 1 << 33
+            and weight.shape == x.shape[-1:] and x.shape[-1] % 8 == 0 and x.shape[-1] <= 65536
+            and x.is_contiguous() and x.data_ptr() % 16 == 0)
+
+
+class RmsNorm(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, weight, eps):
+        n = x.shape[-1]
+        rows = x.numel() // n
+        w = K._dense16(weight)
+        mean = _mean_square(x, rows, n, 1, n, x.shape)
+        y = torch.empty_like(x)
+        _call("qmi_norm_apply", x.device, x.data_ptr(), rows, n, n, mean.data_ptr(), w.data_ptr(),
+              eps, y.data_ptr())
+        ctx.save_for_backward(x, weight, mean)
+        ctx.eps = eps
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, weight, mean = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        if torch.is_grad_enabled():
+            return (*_formula_grads(lambda x, w: rms_norm_formula(x, w, ctx.eps), (x, weight),
+                                    need[:2], dy), None)
+        n = x.shape[-1]
+        x = K._dense16(x)  # saved-tensor hooks may have moved it
+        dx = torch.empty_like(x)
+        dw = _norm_grad(x, x.numel() // n, n, 1, n, x.shape, mean, K._dense16(weight), ctx.eps,
+                        K._dense16(dy), dx)
+        return dx if need[0] else None, dw if need[1] else None, None
+
+
+# ---------------------------------------------------------------------------
+# SwiGLU (qwen3_naive.py:695-702)
+# ---------------------------------------------------------------------------
+def silu_mul_formula(gate_up):
+    gate, up = gate_up.chunk(2, dim=-1)
+    return torch.nn.functional.silu(gate) * up
+
+
+def silu_mul_ok(gate_up) -> bool:
+    return (kernels_ok(gate_up) and gate_up.numel() > 0 and gate_up.numel() < 1 << 33
+            and gate_up.shape[-1] % 16 == 0 and gate_up.shape[-1] <= 65536
+            and gate_up.is_contiguous() and gate_up.data_ptr() % 16 == 0)
+
+
+class SiluMul(torch.autograd.Function):
+    """``silu(gate) * up`` of a packed ``[..., 2 * inter]`` projection."""
+
+    @staticmethod
+    def forward(ctx, gate_up):
+        inter = gate_up.shape[-1] // 2
+        y = torch.empty((*gate_up.shape[:-1], inter), dtype=BF16, device=gate_up.device)
+        _call("qmi_silu_mul_train", y.device, gate_up.data_ptr(), y.numel() // inter, inter, None,
+              y.data_ptr())
+        ctx.save_for_backward(gate_up)
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        gate_up, = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return _formula_grads(silu_mul_formula, (gate_up,), ctx.needs_input_grad, dy)
+        gate_up, dy = K._dense16(gate_up), K._dense16(dy)
+        dgu = torch.empty_like(gate_up)
+        inter = gate_up.shape[-1] // 2
+        _call("qmi_silu_mul_train", dy.device, gate_up.data_ptr(), dy.numel() // inter, inter,
+              dy.data_ptr(), dgu.data_ptr())
+        return dgu
+
+
+# ---------------------------------------------------------------------------
+# Attention of a training batch (qwen3_naive.py:553-590)
+# ---------------------------------------------------------------------------
+def rotate(x: torch.Tensor, positions: torch.Tensor, cache: torch.Tensor) -> torch.Tensor:
+    """Differentiable half-split rotation (fp32 math, cast back)."""
+    half = x.shape[-1] // 2
+    cs = cache[positions]
+    while cs.dim() < x.dim():
+        cs = cs.unsqueeze(-2)
+    c, s = cs[..., :half], cs[..., half:]
+    x1, x2 = x[..., :half].float(), x[..., half:].float()
+    return torch.cat((x1 * c - x2 * s, x2 * c + x1 * s), dim=-1).to(x.dtype)
+
+
+def attention_formula(qkv, norm_q, norm_k, cache, num_heads, num_kv_heads, scale):
+    """QK-norm, RoPE and causal attention of ``qkv [B, T, (Hq + 2 Hkv) * D]`` ->
+    ``[B, T, Hq * D]``; ``norm_q`` / ``norm_k`` map ``[B, T, heads, D]``."""
+    batch, seq_len, width = qkv.shape
+    d = width // (num_heads + 2 * num_kv_heads)
+    q, k, v = qkv.split([num_heads * d, num_kv_heads * d, num_kv_heads * d], dim=-1)
+    q = norm_q(q.reshape(batch, seq_len, num_heads, d))
+    k = norm_k(k.reshape(batch, seq_len, num_kv_heads, d))
+    v = v.reshape(batch, seq_len, num_kv_heads, d)
+    positions = torch.arange(seq_len, device=qkv.device)[None, :].expand(batch, -1)
+    q = rotate(q, positions, cache)
+    k = rotate(k, positions, cache)
+    rep = num_heads // num_kv_heads
+    # Attention core in fp32: batched bf16 products with transposed operands
+    # (and their autograd) are avoided on this platform.
+    qf = q.transpose(1, 2).float()
+    kf = k.transpose(1, 2).float().repeat_interleave(rep, dim=1)
+    vf = v.transpose(1, 2).float().repeat_interleave(rep, dim=1)
+    scores = torch.matmul(qf, kf.transpose(-2, -1).contiguous()) * scale
+    mask = torch.triu(torch.ones(seq_len, seq_len, device=qkv.device, dtype=torch.bool), 1)
+    scores = scores.masked_fill(mask, float("-inf"))
+    w = torch.softmax(scores, dim=-1)
+    o = torch.matmul(w, vf).to(qkv.dtype)
+    return o.transpose(1, 2).reshape(batch, seq_len, -1)
+
+
+def attention_ok(qkv, q_weight, k_weight, cache, num_heads, num_kv_heads) -> bool:
+    """Whether ``QkvAttention`` takes this batch."""
+    return (kernels_ok(qkv, q_weight, k_weight) and qkv.dim() == 3 and qkv.numel() > 0
+            and qkv.is_contiguous() and qkv.data_ptr() % 16 == 0 and num_heads % num_kv_heads == 0
+            and qkv.shape[2] == (num_heads + 2 * num_kv_heads) * HEAD_DIM
+            and qkv.shape[0] * num_heads * qkv.shape[1] < 1 << 27 and qkv.shape[0] <= 65535
+            and q_weight.shape == k_weight.shape == (HEAD_DIM,)
+            and cache.dtype == F32 and cache.device == qkv.device and cache.is_contiguous()
+            and cache.data_ptr() % 16 == 0 and cache.shape[1] == HEAD_DIM
+            and qkv.shape[1] <= cache.shape[0])
+
+
+class QkvAttention(torch.autograd.Function):
+    """``attention_formula`` with RMS norms of a packed bf16 qkv; the backward
+    writes one packed ``d qkv``."""
+
+    @staticmethod
+    def forward(ctx, qkv, q_weight, k_weight, cache, hq, hkv, eps, scale):
+        b, t, width = qkv.shape
+        dev, d = qkv.device, HEAD_DIM
+        qw, kw = K._dense16(q_weight), K._dense16(k_weight)
+        q_mean = _mean_square(qkv, b * t * hq, width, hq, d, (b, t, hq, d))
+        k_mean = _mean_square(qkv[..., hq * d:], b * t * hkv, width, hkv, d, (b, t, hkv, d))
+        qf = torch.empty((b * hq, t, d), dtype=F32, device=dev)
+        kt = torch.empty((b * hq, d, t), dtype=F32, device=dev)
+        vf = torch.empty_like(qf)
+        _call("qmi_train_qkv", dev, qkv.data_ptr(), width, b, t, hq, hkv, q_mean.data_ptr(),
+              k_mean.data_ptr(), qw.data_ptr(), kw.data_ptr(), eps, cache.data_ptr(), qf.data_ptr(),
+              kt.data_ptr(), vf.data_ptr())
+        scores = torch.bmm(qf, kt)
+        _call("qmi_scale_mask", dev, scores.data_ptr(), b * hq * t, t, scale, float("-inf"))
+        w = torch.softmax(scores, dim=-1)
+        del scores
+        o = torch.bmm(w, vf)
+        out = torch.empty((b, t, hq * d), dtype=BF16, device=dev)
+        _call("qmi_train_heads", dev, o.data_ptr(), out.data_ptr(), b, t, hq, 1)
+        ctx.save_for_backward(qkv, q_weight, k_weight, cache, q_mean, k_mean, qf, kt, vf, w)
+        ctx.args = (hq, hkv, eps, scale)
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        qkv, q_weight, k_weight, cache, q_mean, k_mean, qf, kt, vf, w = ctx.saved_tensors
+        hq, hkv, eps, scale = ctx.args
+        need = ctx.needs_input_grad
+        if torch.is_grad_enabled():  # create_graph: the gradients are differentiated again
+            def formula(qkv, q_weight, k_weight):
+                return attention_formula(qkv, lambda a: rms_norm_formula(a, q_weight, eps),
+                                         lambda a: rms_norm_formula(a, k_weight, eps), cache, hq,
+                                         hkv, scale)
+            return (*_formula_grads(formula, (qkv, q_weight, k_weight), need[:3], dout), None, None,
+                    None, None, None)
+        qkv, cache = K._dense16(qkv), K._dense16(cache)
+        b, t, width = qkv.shape
+        dev, d = qkv.device, HEAD_DIM
+        qw, kw = K._dense16(q_weight), K._dense16(k_weight)
+        do = torch.empty((b * hq, t, d), dtype=F32, device=dev)
+        _call("qmi_train_heads", dev, do.data_ptr(), K._dense16(dout).data_ptr(), b, t, hq, 0)
+        dw = torch.bmm(do, vf.transpose(1, 2))
+        dv = torch.bmm(w.transpose(1, 2), do)
+        ds = torch.ops.aten._softmax_backward_data(dw, w, -1, F32)
+        del dw
+        _call("qmi_scale_mask", dev, ds.data_ptr(), b * hq * t, t, scale, 0.0)
+        dq = torch.bmm(ds, kt.transpose(1, 2))
+        dkt = torch.bmm(qf.transpose(1, 2), ds)
+        del ds
+        dqkv = torch.empty_like(qkv)
+        dn_q = torch.empty((b, t, hq, d), dtype=BF16, device=dev)
+        dn_k = torch.empty((b, t, hkv, d), dtype=BF16, device=dev)
+        _call("qmi_train_qkv_grad", dev, b, t, hq, hkv, dq.data_ptr(), dkt.data_ptr(), dv.data_ptr(),
+              cache.data_ptr(), dn_q.data_ptr(), dn_k.data_ptr(), dqkv.data_ptr())
+        dqw = _norm_grad(qkv, b * t * hq, width, hq, d, dn_q.shape, q_mean, qw, eps, dn_q, dqkv)
+        dkw = _norm_grad(qkv[..., hq * d:], b * t * hkv, width, hkv, d, dn_k.shape, k_mean, kw, eps,
+                         dn_k, dqkv[..., hq * d:])
+        return (dqkv if need[0] else None, dqw if need[1] else None, dkw if need[2] else None, None,
+                None, None, None, None)

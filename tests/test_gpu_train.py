@@ -1,0 +1,113 @@
+"""The training batch's fused autograd Functions against the torch formulas
+they stand for.  Forward values and the gradients that flow on are the same
+bit for bit; the norm weights' gradients, summed in another order, agree to
+one bf16 rounding (half an ulp of 8 significant bits, 2^-8)."""
+import importlib
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def T(pkg):
+    return importlib.import_module(pkg.__name__ + ".train_ops")
+
+
+def _rel(a, b):
+    return ((a.double() - b.double()).norm() / b.double().norm()).item()
+
+
+def _both(fused, formula, inputs, seed=3):
+    res = []
+    for f in (fused, formula):
+        leaves = [t.detach().clone().requires_grad_() for t in inputs]
+        y = f(*leaves)
+        g = torch.Generator(device=y.device).manual_seed(seed)
+        y.backward(torch.randn(y.shape, generator=g, device=y.device).bfloat16())
+        res.append([y] + [t.grad for t in leaves])
+    return res
+
+
+# One row; rows that leave lane groups idle; the narrowest row, one whose
+# chunks do not divide a workgroup, one of several passes per workgroup.
+@pytest.mark.parametrize("shape", [(1, 1024), (2, 389, 1024), (3, 24), (1500, 8), (7, 2056), (5, 4096)])
+def test_rms_norm(T, gpu, shape):
+    g = torch.Generator(device=gpu).manual_seed(shape[0])
+    x = torch.randn(shape, generator=g, device=gpu).bfloat16()
+    w = torch.rand(shape[-1], generator=g, device=gpu).bfloat16() + 0.5
+    a, b = _both(lambda x, w: T.RmsNorm.apply(x, w, 1e-6), lambda x, w: T.rms_norm_formula(x, w, 1e-6),
+                 (x, w))
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1]) and _rel(a[2], b[2]) < 2 ** -8
+
+
+@pytest.mark.parametrize("shape", [(1, 16), (3, 5, 48), (2, 389, 6144)])
+def test_silu_mul(T, gpu, shape):
+    gu = (torch.randn(shape, device=gpu) * 4).bfloat16()
+    gu[..., 0], gu[..., 1] = 200.0, -200.0  # saturated gates
+    a, b = _both(T.SiluMul.apply, T.silu_mul_formula, (gu,))
+    assert all(torch.equal(p, q) for p, q in zip(a, b))
+
+
+# Token counts around the transposing tile (64) and not a multiple of 4; one
+# token; query heads per KV head 1, 2 and 4.
+@pytest.mark.parametrize("b,t", [(1, 1), (2, 33), (1, 64), (3, 65), (1, 130), (1, 1152)])
+@pytest.mark.parametrize("hq,hkv", [(2, 2), (4, 2), (8, 2)])
+def test_attention(pkg, T, gpu, b, t, hq, hkv):
+    g = torch.Generator(device=gpu).manual_seed(b * t)
+    qkv = torch.randn(b, t, (hq + 2 * hkv) * 128, generator=g, device=gpu).bfloat16()
+    qw, kw = (torch.rand(128, generator=g, device=gpu).bfloat16() + 0.5 for _ in range(2))
+    cache = pkg.qwen3_naive.get_rope(128, 2048, 1e6).cos_sin_cache.to(gpu)
+
+    def formula(qkv, qw, kw):
+        return T.attention_formula(qkv, lambda x: T.rms_norm_formula(x, qw, 1e-6),
+                                   lambda x: T.rms_norm_formula(x, kw, 1e-6), cache, hq, hkv, 0.09)
+
+    a, ref = _both(lambda *z: T.QkvAttention.apply(*z, cache, hq, hkv, 1e-6, 0.09), formula, (qkv, qw, kw))
+    assert torch.equal(a[0], ref[0])
+    if hq // hkv <= 2:
+        assert torch.equal(a[1], ref[1])
+    else:  # four heads' k gradients are added in another order, then rounded
+        assert _rel(a[1], ref[1]) < 2 ** -8
+    if t > 1:  # one token: the scores have no gradient
+        assert _rel(a[2], ref[2]) < 2 ** -8 and _rel(a[3], ref[3]) < 2 ** -8
+    else:
+        assert not a[2].any() and not ref[2].any()
+
+
+def test_layer_routes(pkg, T, gpu):
+    """The layer takes the fused Functions, unless a norm is hooked or a
+    function transform or a second derivative needs torch ops; same values."""
+    torch.manual_seed(0)
+    layer = pkg.Qwen3DecoderLayer(pkg.Qwen3Config(
+        hidden_size=128, num_attention_heads=2, num_key_value_heads=1, intermediate_size=256,
+        num_hidden_layers=1, max_position_embeddings=64)).to(gpu).bfloat16()
+    x = torch.randn(2, 33, 128, device=gpu).bfloat16().requires_grad_()
+    res, seen = [], []
+    for hook in (False, True):
+        h = layer.self_attn.q_norm.register_forward_hook(lambda *_: seen.append(1)) if hook else None
+        layer.zero_grad()
+        x.grad = None
+        y = layer(x)
+        y.float().square().mean().backward()
+        res.append([y.detach(), x.grad])
+        if h:
+            h.remove()
+    assert seen and all(torch.equal(a, b) for a, b in zip(*res))
+    # A gradient that is differentiated again: through the formulas.  x's second
+    # gradient is the sum of two, here each rounded to bf16 (2^-8) before it.
+    out = []
+    for f in (lambda: T.RmsNorm.apply(x, layer.input_layernorm.weight, 1e-6),
+              lambda: T.rms_norm_formula(x, layer.input_layernorm.weight, 1e-6)):
+        g, = torch.autograd.grad(f().float().pow(3).sum(), x, create_graph=True)
+        out.append(torch.autograd.grad(g.float().square().sum(), x)[0])
+    assert out[0].abs().max() > 0 and _rel(*out) < 2 ** -7
+    # Saved tensors that a hook packs and unpacks elsewhere.
+    with torch.autograd.graph.save_on_cpu():
+        y = layer(x)
+    x.grad = None
+    y.float().square().mean().backward()
+    assert torch.equal(x.grad, res[0][1])
+    with torch.no_grad():
+        assert not T.norm_ok(x, layer.input_layernorm.weight)
