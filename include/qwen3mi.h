@@ -456,6 +456,10 @@ int qmi_prefill_layer(const qmi_prefill_layer_args* args, void* stream);
  *                 [batch * t][h][128], and v's into the packed d qkv
  *   train_heads:  fp32 [batch][heads][t][128] -> bf16 [batch][t][heads][128]
  *                 (to_bf16 1) or back (0)
+ *   sum_rows:     y[n] = bf16(the sum of `parts` contiguous fp32 rows)
+ *   causal_softmax: w NULL: s[row] = softmax(s[row][j] * scale, j <= row % t),
+ *                 0 past it; else the gradient: s holds dw and becomes
+ *                 (s w - w sum(s w)) * scale; [rows][t] in place, t <= 1024
  *   scale_mask:   s[row][j] = j > row % t ? masked : s * scale, [rows][t] in place
  */
 int qmi_square_rows(const uint16_t* x, int64_t rows, int64_t stride, int64_t heads, int64_t n,
@@ -479,6 +483,8 @@ int qmi_train_qkv_grad(int64_t batch, int64_t t, int64_t hq, int64_t hkv, const 
                        uint16_t* dn_k, uint16_t* dqkv, void* stream);
 int qmi_train_heads(float* f, uint16_t* o, int64_t batch, int64_t t, int64_t heads, int32_t to_bf16,
                     void* stream);
+int qmi_sum_rows(const float* x, int64_t parts, int64_t n, uint16_t* y, void* stream);
+int qmi_causal_softmax(float* s, const float* w, int64_t rows, int64_t t, float scale, void* stream);
 int qmi_scale_mask(float* s, int64_t rows, int64_t t, float scale, float masked, void* stream);
 
 /*

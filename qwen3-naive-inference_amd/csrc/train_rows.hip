@@ -397,6 +397,118 @@ __global__ __launch_bounds__(kThreads) void scale_mask_kernel(float* __restrict_
   }
 }
 
+// Rows of causal attention, one wave each, NI x 64 columns: lane l holds
+// columns l, l + 64, ..., adds its own in that order and the lanes by a
+// butterfly of offsets 32 .. 1, the order of torch's softmax kernels for rows
+// of at most 1,024, whose bits these are.  Columns past the diagonal hold
+// exact zeros and are not read.  At 8 x 16 x 640 x 640 (210 MB) the forward
+// reads half of it and writes it once, where mask and softmax moved four times
+// as much; the backward likewise.
+__device__ __forceinline__ float butterfly_sum(float x) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+  return x;
+}
+
+template <int NI>
+__global__ __launch_bounds__(kThreads) void causal_softmax_kernel(float* __restrict__ s, uint32_t rows,
+                                                                  int t, float scale) {
+  const uint32_t row = blockIdx.x * (kThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  if (row >= rows) return;
+  const int lane = threadIdx.x & 63, q = row % (uint32_t)t;  // q, and so which chunks are skipped: uniform
+  float* p = s + (int64_t)row * t;
+  float v[NI];
+  float m = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int j = lane + 64 * i;
+    v[i] = -INFINITY;
+    if (64 * i > q) continue;
+    if (j <= q) v[i] = p[j] * scale;
+    m = v[i] > m || v[i] != v[i] ? v[i] : m;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const float b = __shfl_xor(m, o, 64);
+    m = m < b ? b : m;
+  }
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    if (64 * i > q) continue;
+    v[i] = expf(v[i] - m);
+    sum += v[i];
+  }
+  sum = butterfly_sum(sum);
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int j = lane + 64 * i;
+    if (j < t) p[j] = j <= q ? v[i] / sum : 0.f;
+  }
+}
+
+// ds = (dp * w - w * sum(dp * w)) * scale, in place of dp, the difference an FMA as
+// in torch's kernel.
+template <int NI>
+__global__ __launch_bounds__(kThreads) void causal_softmax_grad_kernel(float* __restrict__ dp,
+                                                                       const float* __restrict__ w,
+                                                                       uint32_t rows, int t, float scale) {
+  const uint32_t row = blockIdx.x * (kThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  if (row >= rows) return;
+  const int lane = threadIdx.x & 63, q = row % (uint32_t)t;  // q, and so which chunks are skipped: uniform
+  float* p = dp + (int64_t)row * t;
+  const float* pw = w + (int64_t)row * t;
+  float g[NI], o[NI];
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int j = lane + 64 * i;
+    o[i] = g[i] = 0.f;
+    if (64 * i > q) continue;
+    if (j <= q) {
+      o[i] = pw[j];
+      g[i] = p[j] * o[i];
+    }
+    sum += g[i];
+  }
+  sum = butterfly_sum(sum);
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int j = lane + 64 * i;
+    if (j < t) p[j] = j <= q ? fmaf(-o[i], sum, g[i]) * scale : 0.f;
+  }
+}
+
+// y = bf16(sum of `parts` fp32 rows), summed in two levels of a fixed order:
+// workgroup = 16 columns x 64 row groups, each with 8 loads in flight (16
+// groups of one load each took 20 us for 1,024 rows).
+constexpr int kSumGroups = 64;
+__global__ __launch_bounds__(16 * kSumGroups) void sum_rows_kernel(const float* __restrict__ x, int parts,
+                                                                   int n, uint16_t* __restrict__ y) {
+  __shared__ float sm[kSumGroups][17];
+  const int c = threadIdx.x % 16, grp = threadIdx.x / 16, col = blockIdx.x * 16 + c;
+  float s = 0.f;
+  if (col < n)
+    for (int r = grp; r < parts; r += 8 * kSumGroups) {
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const int rr = r + k * kSumGroups;
+        v[k] = rr < parts ? x[(int64_t)rr * n + col] : 0.f;
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k) s += v[k];
+    }
+  sm[grp][c] = s;
+  __syncthreads();
+  if (threadIdx.x < 16 && col < n) {
+    s = sm[0][c];
+#pragma unroll
+    for (int g = 1; g < kSumGroups; ++g) s += sm[g][c];
+    y[col] = f32_to_bf16(s);
+  }
+}
+
 inline bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Items of 8 elements; 32-bit item arithmetic.
@@ -542,4 +654,39 @@ extern "C" int qmi_scale_mask(float* s, int64_t rows, int64_t t, float scale, fl
   if (!al16(s)) return QMI_E_BAD_STRIDE;
   hipLaunchKernelGGL(scale_mask_kernel, dim3((unsigned)rows), dim3(kThreads), 0, QMI_ST, s, (int)t, scale, masked);
   QMI_RETURN_LAUNCH_STATUS();
+}
+
+extern "C" int qmi_sum_rows(const float* x, int64_t parts, int64_t n, uint16_t* y, void* stream) {
+  if (parts <= 0 || n <= 0) return QMI_E_BAD_SHAPE;
+  if (parts > (1 << 20) || n > (1 << 20)) return QMI_E_UNSUPPORTED;
+  if (!x || !y) return QMI_E_NULL_POINTER;
+  hipLaunchKernelGGL(sum_rows_kernel, dim3((unsigned)((n + 15) / 16)), dim3(16 * kSumGroups), 0, QMI_ST, x, (int)parts,
+                     (int)n, y);
+  QMI_RETURN_LAUNCH_STATUS();
+}
+
+extern "C" int qmi_causal_softmax(float* s, const float* w, int64_t rows, int64_t t, float scale,
+                                  void* stream) {
+  if (rows <= 0 || t <= 0 || rows % t) return QMI_E_BAD_SHAPE;
+  if (rows > 0x7fffffffLL || t > 1024) return QMI_E_UNSUPPORTED;
+  if (!s) return QMI_E_NULL_POINTER;
+  const dim3 grid((unsigned)((rows + kThreads / 64 - 1) / (kThreads / 64)));
+#define QMI_CS(NI)                                                                                       \
+  if (t <= 64 * NI) {                                                                                    \
+    if (w)                                                                                               \
+      hipLaunchKernelGGL(causal_softmax_grad_kernel<NI>, grid, dim3(kThreads), 0, QMI_ST, s, w,          \
+                         (uint32_t)rows, (int)t, scale);                                                 \
+    else                                                                                                 \
+      hipLaunchKernelGGL(causal_softmax_kernel<NI>, grid, dim3(kThreads), 0, QMI_ST, s, (uint32_t)rows,  \
+                         (int)t, scale);                                                                 \
+    QMI_RETURN_LAUNCH_STATUS();                                                                          \
+  }
+  QMI_CS(1)
+  QMI_CS(2)
+  QMI_CS(4)
+  QMI_CS(8)
+  QMI_CS(12)
+  QMI_CS(16)
+#undef QMI_CS
+  return QMI_E_UNSUPPORTED;
 }

@@ -74,7 +74,9 @@ def _norm_grad(x, rows, stride, heads, n, shape, mean, w, eps, dy, dx):
     parts = torch.empty((lib().qmi_norm_grad_parts(rows, n), n), dtype=F32, device=w.device)
     _call("qmi_norm_grad", w.device, x.data_ptr(), rows, stride, heads, n, mean.data_ptr(),
           w.data_ptr(), eps, dy.data_ptr(), dr.data_ptr(), dx.data_ptr(), parts.data_ptr())
-    return parts.sum(0).to(BF16)
+    dw = torch.empty(n, dtype=BF16, device=w.device)
+    _call("qmi_sum_rows", w.device, parts.data_ptr(), parts.shape[0], n, dw.data_ptr())
+    return dw
 
 
 def norm_ok(x, weight) -> bool:
@@ -203,6 +205,11 @@ def attention_ok(qkv, q_weight, k_weight, cache, num_heads, num_kv_heads) -> boo
             and qkv.shape[1] <= cache.shape[0])
 
 
+# Longest row of the fused causal softmax; torch's own kernel adds longer rows in
+# another order.
+SOFTMAX_MAX = 1024
+
+
 class QkvAttention(torch.autograd.Function):
     """``attention_formula`` with RMS norms of a packed bf16 qkv; the backward
     writes one packed ``d qkv``."""
@@ -221,8 +228,12 @@ class QkvAttention(torch.autograd.Function):
               k_mean.data_ptr(), qw.data_ptr(), kw.data_ptr(), eps, cache.data_ptr(), qf.data_ptr(),
               kt.data_ptr(), vf.data_ptr())
         scores = torch.bmm(qf, kt)
-        _call("qmi_scale_mask", dev, scores.data_ptr(), b * hq * t, t, scale, float("-inf"))
-        w = torch.softmax(scores, dim=-1)
+        if t <= SOFTMAX_MAX:
+            _call("qmi_causal_softmax", dev, scores.data_ptr(), None, b * hq * t, t, scale)
+            w = scores
+        else:
+            _call("qmi_scale_mask", dev, scores.data_ptr(), b * hq * t, t, scale, float("-inf"))
+            w = torch.softmax(scores, dim=-1)
         del scores
         o = torch.bmm(w, vf)
         out = torch.empty((b, t, hq * d), dtype=BF16, device=dev)
@@ -251,9 +262,13 @@ class QkvAttention(torch.autograd.Function):
         _call("qmi_train_heads", dev, do.data_ptr(), K._dense16(dout).data_ptr(), b, t, hq, 0)
         dw = torch.bmm(do, vf.transpose(1, 2))
         dv = torch.bmm(w.transpose(1, 2), do)
-        ds = torch.ops.aten._softmax_backward_data(dw, w, -1, F32)
+        if t <= SOFTMAX_MAX:
+            ds = dw
+            _call("qmi_causal_softmax", dev, ds.data_ptr(), w.data_ptr(), b * hq * t, t, scale)
+        else:
+            ds = torch.ops.aten._softmax_backward_data(dw, w, -1, F32)
+            _call("qmi_scale_mask", dev, ds.data_ptr(), b * hq * t, t, scale, 0.0)
         del dw
-        _call("qmi_scale_mask", dev, ds.data_ptr(), b * hq * t, t, scale, 0.0)
         dq = torch.bmm(ds, kt.transpose(1, 2))
         dkt = torch.bmm(qf.transpose(1, 2), ds)
         del ds

@@ -50,9 +50,10 @@ def test_silu_mul(T, gpu, shape):
     assert all(torch.equal(p, q) for p, q in zip(a, b))
 
 
-# Token counts around the transposing tile (64) and not a multiple of 4; one
-# token; query heads per KV head 1, 2 and 4.
-@pytest.mark.parametrize("b,t", [(1, 1), (2, 33), (1, 64), (3, 65), (1, 130), (1, 1152)])
+# Token counts around the transposing tile and the softmax's chunk (64), not a
+# multiple of 4, around the fused softmax's longest row (1,024); one token; query heads per KV head 1, 2 and 4.
+@pytest.mark.parametrize("b,t", [(1, 1), (2, 33), (1, 64), (3, 65), (1, 130), (2, 700), (1, 1024),
+                                 (1, 1025), (1, 1152)])
 @pytest.mark.parametrize("hq,hkv", [(2, 2), (4, 2), (8, 2)])
 def test_attention(pkg, T, gpu, b, t, hq, hkv):
     g = torch.Generator(device=gpu).manual_seed(b * t)
