@@ -21,6 +21,9 @@
 //   * The 8 partial tiles are added in wave order through LDS: no split-K
 //     partials in memory, so the next norm reads bf16 rows.
 //   * SwiGLU (packed [gate; up] weight): 8 gate rows and their 8 up rows.
+//
+// Eight layers, 4 sequences of 37-700 tokens, as a graph: 324 -> 274 us (the
+// rows' loads behind the weights', which return in order: 307).
 #include "qmi_common.h"
 
 namespace {

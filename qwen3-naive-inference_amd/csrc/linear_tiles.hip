@@ -18,9 +18,16 @@
 //     between gate and up, so a wave holds both for the same columns and
 //     writes silu(bf16(g)) * bf16(u) (the rounding points of a bf16 GEMM
 //     followed by silu_mul) without the 2 I wide intermediate.
+//   * Operands of the next k-step are read while one's products run, across
+//     the chunk boundary too (one barrier per chunk).
 //   * Workgroup -> tile: consecutive workgroups go to different XCDs, so each
 //     XCD takes a contiguous run of a tile order that walks the rows of a few
 //     column tiles first; its L2 then serves the re-reads.
+//
+// Hidden 1024, MLP 3072, weights from HBM, us for qkv / o / gate_up with SwiGLU /
+// down (the library's product, with silu_mul for gate_up): 512 rows 9 / 9 / 12 /
+// 12 (11 / 10 / 19 / 13), 2,048 rows 22 / 14 / 27 / 20 (21 / 16 / 36 / 21), 4,096
+// rows 39 / 25 / 56 / 35 (30 / 22 / 70 / 31).
 #include "qmi_common.h"
 
 namespace {

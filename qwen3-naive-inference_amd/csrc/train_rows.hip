@@ -14,7 +14,9 @@
 // What bounds them is memory: a norm forward moved its fp32 rows through
 // memory 9 times in 9 launches and backward ~20 times, the scores took 3
 // passes per direction outside the softmax.  All are one 8-element item per
-// lane with 16- or 32-byte accesses.
+// lane with 16- or 32-byte accesses.  One decoder layer forward + backward, 8 x
+// 640 tokens of hidden 1024: 4,020 -> 2,000 us (900 of them fp32 products); a
+// two-layer training step, 2 x 389 tokens: 5,300-5,900 -> 2,870 us.
 #include <algorithm>
 
 #include "qmi_common.h"

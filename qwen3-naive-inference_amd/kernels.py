@@ -726,6 +726,7 @@ def prefill_layer(x, residual, norms, mats, eps, positions, cos_sin_cache, num_q
     inter = down_w.shape[1]
     if not (0 < t <= PREFILL_LAYER_ROWS and t * max(q_n + 2 * kv_n, 2 * inter) <= PREFILL_LAYER_OUTPUT
             and hidden <= NORM_MAX_WIDTH and hidden % 64 == 0 and inter % 64 == 0
+            and max(q_n + 2 * kv_n, inter) <= 65536  # 32-bit load offsets
             and num_q_heads in (num_kv_heads, 2 * num_kv_heads, 4 * num_kv_heads)
             and qkv_w.shape == (q_n + 2 * kv_n, hidden) and o_w.shape == (hidden, q_n)
             and gu_w.shape == (2 * inter, hidden) and down_w.shape == (hidden, inter)):

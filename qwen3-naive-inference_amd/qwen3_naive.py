@@ -11,10 +11,11 @@ in under its generator and GRPO loop:
 
 Inference paths (no autograd) run the HIP kernels: fused QK-RMSNorm + RoPE,
 slot-mapped KV store, paged decode / varlen prefill attention, RMSNorm /
-add+RMSNorm, SwiGLU; projections use torch GEMMs (hipBLASLt).  The batch
-``forward`` used for training keeps torch ops so autograd works, with a
-differentiable RoPE (the reference's RoPE kernel has no backward) and the
-attention core in fp32.
+add+RMSNorm, SwiGLU, and the projections of decode batches and of prefill
+steps of up to 2,048 tokens (larger ones use torch GEMMs).  The batch
+``forward`` used for training runs its element-wise chains as autograd
+Functions (train_ops.py; the reference's RoPE kernel has no backward), with
+the attention core in fp32.
 """
 from __future__ import annotations
 
