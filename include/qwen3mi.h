@@ -457,10 +457,11 @@ int qmi_prefill_layer(const qmi_prefill_layer_args* args, void* stream);
  *   train_heads:  fp32 [batch][heads][t][128] -> bf16 [batch][t][heads][128]
  *                 (to_bf16 1) or back (0)
  *   sum_rows:     y[n] = bf16(the sum of `parts` contiguous fp32 rows)
- *   causal_softmax: w NULL: s[row] = softmax(s[row][j] * scale, j <= row % t),
- *                 0 past it; else the gradient: s holds dw and becomes
- *                 (s w - w sum(s w)) * scale; [rows][t] in place, t <= 1024
- *   scale_mask:   s[row][j] = j > row % t ? masked : s * scale, [rows][t] in place
+ *   causal_softmax: w NULL: out[row] = softmax(s[row][j] * scale, j <= row % t),
+ *                 0 past it; else the gradient, s being dw: out =
+ *                 (s w - w sum(s w)) * scale; [rows][t], t <= 1024
+ *   scale_mask:   out[row][j] = j > row % t ? masked : s * scale, [rows][t]
+ * No output overlaps an input.
  */
 int qmi_square_rows(const uint16_t* x, int64_t rows, int64_t stride, int64_t heads, int64_t n,
                     float* sq, void* stream);
@@ -484,8 +485,10 @@ int qmi_train_qkv_grad(int64_t batch, int64_t t, int64_t hq, int64_t hkv, const 
 int qmi_train_heads(float* f, uint16_t* o, int64_t batch, int64_t t, int64_t heads, int32_t to_bf16,
                     void* stream);
 int qmi_sum_rows(const float* x, int64_t parts, int64_t n, uint16_t* y, void* stream);
-int qmi_causal_softmax(float* s, const float* w, int64_t rows, int64_t t, float scale, void* stream);
-int qmi_scale_mask(float* s, int64_t rows, int64_t t, float scale, float masked, void* stream);
+int qmi_causal_softmax(const float* s, const float* w, int64_t rows, int64_t t, float scale, float* out,
+                       void* stream);
+int qmi_scale_mask(const float* s, int64_t rows, int64_t t, float scale, float masked, float* out,
+                   void* stream);
 
 /*
  * Row-wise log-softmax gathered at one token per row.

@@ -105,8 +105,8 @@ SIGNATURES: dict[str, tuple] = {
                                           _c_p, _c_p, _c_p, _c_p]),
     "qmi_train_heads": (ctypes.c_int, [_c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i32, _c_p]),
     "qmi_sum_rows": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_p, _c_p]),
-    "qmi_causal_softmax": (ctypes.c_int, [_c_p, _c_p, _c_i64, _c_i64, _c_f32, _c_p]),
-    "qmi_scale_mask": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_f32, _c_f32, _c_p]),
+    "qmi_causal_softmax": (ctypes.c_int, [_c_p, _c_p, _c_i64, _c_i64, _c_f32, _c_p, _c_p]),
+    "qmi_scale_mask": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_f32, _c_f32, _c_p, _c_p]),
     "qmi_logprob_gather": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_p, _c_i64, _c_i64, _c_i64,
                                           _c_i64, _c_i64, _c_p, _c_p, _c_p]),
     "qmi_grpo_advantage": (ctypes.c_int, [_c_p, _c_p, _c_i64, _c_f32, _c_p, _c_p]),

@@ -378,24 +378,25 @@ __global__ __launch_bounds__(kThreads) void heads_kernel(float* __restrict__ f, 
     store8f(src, load8(dst));
 }
 
-// s[row][j] = j > row % t ? masked : s * scale, in place; row-major [rows][t].
-__global__ __launch_bounds__(kThreads) void scale_mask_kernel(float* __restrict__ s, int t, float scale,
-                                                              float masked) {
+// out[row][j] = j > row % t ? masked : s * scale; row-major [rows][t].
+__global__ __launch_bounds__(kThreads) void scale_mask_kernel(const float* __restrict__ s, int t, float scale,
+                                                              float masked, float* __restrict__ out) {
   const uint32_t row = blockIdx.x;
   const int q = row % (uint32_t)t;
-  float* p = s + (int64_t)row * t;
+  const float* p = s + (int64_t)row * t;
+  float* y = out + (int64_t)row * t;
   if (t % 4 == 0) {
     for (int j = 4 * threadIdx.x; j < t; j += 4 * kThreads) {
       f32x4_t v = {masked, masked, masked, masked};
       if (j <= q) {
-        v = *reinterpret_cast<f32x4_t*>(p + j);
+        v = *reinterpret_cast<const f32x4_t*>(p + j);
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = j + e > q ? masked : v[e] * scale;
       }
-      *reinterpret_cast<f32x4_t*>(p + j) = v;
+      *reinterpret_cast<f32x4_t*>(y + j) = v;
     }
   } else {
-    for (int j = threadIdx.x; j < t; j += kThreads) p[j] = j > q ? masked : p[j] * scale;
+    for (int j = threadIdx.x; j < t; j += kThreads) y[j] = j > q ? masked : p[j] * scale;
   }
 }
 
@@ -413,12 +414,14 @@ __device__ __forceinline__ float butterfly_sum(float x) {
 }
 
 template <int NI>
-__global__ __launch_bounds__(kThreads) void causal_softmax_kernel(float* __restrict__ s, uint32_t rows,
-                                                                  int t, float scale) {
+__global__ __launch_bounds__(kThreads) void causal_softmax_kernel(const float* __restrict__ s,
+                                                                  uint32_t rows, int t, float scale,
+                                                                  float* __restrict__ out) {
   const uint32_t row = blockIdx.x * (kThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   if (row >= rows) return;
   const int lane = threadIdx.x & 63, q = row % (uint32_t)t;  // q, and so which chunks are skipped: uniform
-  float* p = s + (int64_t)row * t;
+  const float* p = s + (int64_t)row * t;
+  float* y = out + (int64_t)row * t;
   float v[NI];
   float m = -INFINITY;
 #pragma unroll
@@ -445,21 +448,23 @@ __global__ __launch_bounds__(kThreads) void causal_softmax_kernel(float* __restr
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int j = lane + 64 * i;
-    if (j < t) p[j] = j <= q ? v[i] / sum : 0.f;
+    if (j < t) y[j] = j <= q ? v[i] / sum : 0.f;
   }
 }
 
-// ds = (dp * w - w * sum(dp * w)) * scale, in place of dp, the difference an FMA as
-// in torch's kernel.
+// ds = (dp * w - w * sum(dp * w)) * scale, the difference an FMA as in torch's
+// kernel.
 template <int NI>
-__global__ __launch_bounds__(kThreads) void causal_softmax_grad_kernel(float* __restrict__ dp,
+__global__ __launch_bounds__(kThreads) void causal_softmax_grad_kernel(const float* __restrict__ dp,
                                                                        const float* __restrict__ w,
-                                                                       uint32_t rows, int t, float scale) {
+                                                                       uint32_t rows, int t, float scale,
+                                                                       float* __restrict__ ds) {
   const uint32_t row = blockIdx.x * (kThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   if (row >= rows) return;
   const int lane = threadIdx.x & 63, q = row % (uint32_t)t;  // q, and so which chunks are skipped: uniform
-  float* p = dp + (int64_t)row * t;
+  const float* p = dp + (int64_t)row * t;
   const float* pw = w + (int64_t)row * t;
+  float* y = ds + (int64_t)row * t;
   float g[NI], o[NI];
   float sum = 0.f;
 #pragma unroll
@@ -477,7 +482,7 @@ __global__ __launch_bounds__(kThreads) void causal_softmax_grad_kernel(float* __
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int j = lane + 64 * i;
-    if (j < t) p[j] = j <= q ? fmaf(-o[i], sum, g[i]) * scale : 0.f;
+    if (j < t) y[j] = j <= q ? fmaf(-o[i], sum, g[i]) * scale : 0.f;
   }
 }
 
@@ -649,12 +654,14 @@ extern "C" int qmi_train_heads(float* f, uint16_t* o, int64_t batch, int64_t t, 
   QMI_RETURN_LAUNCH_STATUS();
 }
 
-extern "C" int qmi_scale_mask(float* s, int64_t rows, int64_t t, float scale, float masked, void* stream) {
+extern "C" int qmi_scale_mask(const float* s, int64_t rows, int64_t t, float scale, float masked, float* out,
+                              void* stream) {
   if (rows <= 0 || t <= 0 || rows % t) return QMI_E_BAD_SHAPE;
   if (rows > 0x7fffffffLL || t > 0x7fffffffLL / 4) return QMI_E_UNSUPPORTED;
-  if (!s) return QMI_E_NULL_POINTER;
-  if (!al16(s)) return QMI_E_BAD_STRIDE;
-  hipLaunchKernelGGL(scale_mask_kernel, dim3((unsigned)rows), dim3(kThreads), 0, QMI_ST, s, (int)t, scale, masked);
+  if (!s || !out) return QMI_E_NULL_POINTER;
+  if (!al16(s) || !al16(out)) return QMI_E_BAD_STRIDE;
+  hipLaunchKernelGGL(scale_mask_kernel, dim3((unsigned)rows), dim3(kThreads), 0, QMI_ST, s, (int)t, scale, masked,
+                     out);
   QMI_RETURN_LAUNCH_STATUS();
 }
 
@@ -667,20 +674,20 @@ extern "C" int qmi_sum_rows(const float* x, int64_t parts, int64_t n, uint16_t* 
   QMI_RETURN_LAUNCH_STATUS();
 }
 
-extern "C" int qmi_causal_softmax(float* s, const float* w, int64_t rows, int64_t t, float scale,
-                                  void* stream) {
+extern "C" int qmi_causal_softmax(const float* s, const float* w, int64_t rows, int64_t t, float scale,
+                                  float* out, void* stream) {
   if (rows <= 0 || t <= 0 || rows % t) return QMI_E_BAD_SHAPE;
   if (rows > 0x7fffffffLL || t > 1024) return QMI_E_UNSUPPORTED;
-  if (!s) return QMI_E_NULL_POINTER;
+  if (!s || !out) return QMI_E_NULL_POINTER;
   const dim3 grid((unsigned)((rows + kThreads / 64 - 1) / (kThreads / 64)));
 #define QMI_CS(NI)                                                                                       \
   if (t <= 64 * NI) {                                                                                    \
     if (w)                                                                                               \
       hipLaunchKernelGGL(causal_softmax_grad_kernel<NI>, grid, dim3(kThreads), 0, QMI_ST, s, w,          \
-                         (uint32_t)rows, (int)t, scale);                                                 \
+                         (uint32_t)rows, (int)t, scale, out);                                            \
     else                                                                                                 \
       hipLaunchKernelGGL(causal_softmax_kernel<NI>, grid, dim3(kThreads), 0, QMI_ST, s, (uint32_t)rows,  \
-                         (int)t, scale);                                                                 \
+                         (int)t, scale, out);                                                            \
     QMI_RETURN_LAUNCH_STATUS();                                                                          \
   }
   QMI_CS(1)

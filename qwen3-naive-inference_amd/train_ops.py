@@ -228,12 +228,15 @@ class QkvAttention(torch.autograd.Function):
               k_mean.data_ptr(), qw.data_ptr(), kw.data_ptr(), eps, cache.data_ptr(), qf.data_ptr(),
               kt.data_ptr(), vf.data_ptr())
         scores = torch.bmm(qf, kt)
+        # Kernels write to tensors of their own: a dispatch mode (selective
+        # checkpointing) may keep what a torch op returned, and sees no write.
+        w = torch.empty_like(scores)
         if t <= SOFTMAX_MAX:
-            _call("qmi_causal_softmax", dev, scores.data_ptr(), None, b * hq * t, t, scale)
-            w = scores
+            _call("qmi_causal_softmax", dev, scores.data_ptr(), None, b * hq * t, t, scale, w.data_ptr())
         else:
-            _call("qmi_scale_mask", dev, scores.data_ptr(), b * hq * t, t, scale, float("-inf"))
-            w = torch.softmax(scores, dim=-1)
+            _call("qmi_scale_mask", dev, scores.data_ptr(), b * hq * t, t, scale, float("-inf"),
+                  w.data_ptr())
+            w = torch.softmax(w, dim=-1)
         del scores
         o = torch.bmm(w, vf)
         out = torch.empty((b, t, hq * d), dtype=BF16, device=dev)
@@ -262,12 +265,13 @@ class QkvAttention(torch.autograd.Function):
         _call("qmi_train_heads", dev, do.data_ptr(), K._dense16(dout).data_ptr(), b, t, hq, 0)
         dw = torch.bmm(do, vf.transpose(1, 2))
         dv = torch.bmm(w.transpose(1, 2), do)
+        ds = torch.empty_like(dw)
         if t <= SOFTMAX_MAX:
-            ds = dw
-            _call("qmi_causal_softmax", dev, ds.data_ptr(), w.data_ptr(), b * hq * t, t, scale)
+            _call("qmi_causal_softmax", dev, dw.data_ptr(), w.data_ptr(), b * hq * t, t, scale,
+                  ds.data_ptr())
         else:
-            ds = torch.ops.aten._softmax_backward_data(dw, w, -1, F32)
-            _call("qmi_scale_mask", dev, ds.data_ptr(), b * hq * t, t, scale, 0.0)
+            dw = torch.ops.aten._softmax_backward_data(dw, w, -1, F32)
+            _call("qmi_scale_mask", dev, dw.data_ptr(), b * hq * t, t, scale, 0.0, ds.data_ptr())
         del dw
         dq = torch.bmm(ds, kt.transpose(1, 2))
         dkt = torch.bmm(qf.transpose(1, 2), ds)

@@ -112,3 +112,34 @@ def test_layer_routes(pkg, T, gpu):
     assert torch.equal(x.grad, res[0][1])
     with torch.no_grad():
         assert not T.norm_ok(x, layer.input_layernorm.weight)
+
+
+def _layer(pkg, gpu, max_position=64):
+    torch.manual_seed(0)
+    return pkg.Qwen3DecoderLayer(pkg.Qwen3Config(
+        hidden_size=128, num_attention_heads=2, num_key_value_heads=1, intermediate_size=256,
+        num_hidden_layers=1, max_position_embeddings=max_position)).to(gpu).bfloat16()
+
+
+def _grads(layer, y, x):
+    y.float().square().mean().backward()
+    res = [x.grad] + [p.grad for p in layer.parameters()]
+    x.grad = None
+    layer.zero_grad()
+    return res
+
+
+# Both softmax forms; the products kept by a selective checkpoint, or every op's result.
+@pytest.mark.parametrize("t", [33, 1030])
+@pytest.mark.parametrize("keep", ["products", "all"])
+def test_selective_checkpoint(pkg, gpu, t, keep):
+    from torch.utils import checkpoint as C
+    layer = _layer(pkg, gpu, 2048)
+    x = torch.randn(1, t, 128, device=gpu).bfloat16().requires_grad_()
+    want = _grads(layer, layer(x), x)
+    aten = torch.ops.aten
+    policy = ([aten.mm.default, aten.bmm.default, aten.addmm.default] if keep == "products" else
+              lambda ctx, op, *a, **k: C.CheckpointPolicy.MUST_SAVE)
+    y = C.checkpoint(layer, x, use_reentrant=False,
+                     context_fn=lambda: C.create_selective_checkpoint_contexts(policy))
+    assert all(torch.equal(a, b) for a, b in zip(_grads(layer, y, x), want))
