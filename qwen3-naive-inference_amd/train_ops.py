@@ -37,8 +37,10 @@ def kernels_ok(*tensors: torch.Tensor) -> bool:
 
 
 def _formula_grads(formula, inputs, needs, grads):
-    """Gradients of ``formula(*inputs)`` that autograd can differentiate again."""
+    """Gradients of ``formula(*inputs)`` that autograd can differentiate again:
+    those of each argument, also where one tensor is passed as several."""
     with torch.enable_grad():
+        inputs = [t.view_as(t) for t in inputs]
         out = formula(*inputs)
     wanted = [t for t, n in zip(inputs, needs) if n]
     got = iter(torch.autograd.grad(out, wanted, grads, create_graph=True, allow_unused=True))

@@ -143,3 +143,26 @@ def test_selective_checkpoint(pkg, gpu, t, keep):
     y = C.checkpoint(layer, x, use_reentrant=False,
                      context_fn=lambda: C.create_selective_checkpoint_contexts(policy))
     assert all(torch.equal(a, b) for a, b in zip(_grads(layer, y, x), want))
+
+
+def test_shared_norm_weight_second_derivative(pkg, T, gpu):
+    """One weight as both q and k norm: a differentiable gradient counts each use once."""
+    g = torch.Generator(device=gpu).manual_seed(7)
+    qkv = torch.randn(1, 20, 4 * 128, generator=g, device=gpu).bfloat16()
+    w = torch.rand(128, generator=g, device=gpu).bfloat16() + 0.5
+    cache = pkg.qwen3_naive.get_rope(128, 64, 1e6).cos_sin_cache.to(gpu)
+
+    def norm(x):
+        return T.rms_norm_formula(x, w, 1e-6)
+
+    out = []
+    for f in (lambda: T.QkvAttention.apply(qkv, w, w, cache, 2, 1, 1e-6, 0.09),
+              lambda: T.attention_formula(qkv, norm, norm, cache, 2, 1, 0.09)):
+        qkv, w = qkv.detach().requires_grad_(), w.detach().requires_grad_()
+        first = torch.autograd.grad(f().float().pow(3).sum(), (qkv, w), create_graph=True)
+        second = torch.autograd.grad(first[0].float().square().sum(), (qkv, w))
+        out.append([*first, *second])
+    # Two uses' gradients are each rounded to bf16 before they are added (2^-8), and
+    # with them the terms of the second derivative.
+    assert all(_rel(a, b) < 2 ** -6 for a, b in zip(*out))
+
