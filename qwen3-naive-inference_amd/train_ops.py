@@ -5,8 +5,9 @@ Each gives the values of the torch formula beside it, in both directions: the
 kernels repeat its fp32 operations and bf16 roundings, sums along a row, the
 softmax and the products are the same torch calls on the same operands.  Only
 the norm weights' gradients are summed in another (fixed) order.  The formula
-serves every call the kernels do not take, and a backward that has to be
-differentiable itself (``create_graph=True``) differentiates the formula.
+serves every call the kernels do not take, and a backward that is
+differentiated itself (``create_graph=True``, forward mode) differentiates
+the formula.
 """
 from __future__ import annotations
 
@@ -32,8 +33,19 @@ def kernels_ok(*tensors: torch.Tensor) -> bool:
         if (type(t) not in (torch.Tensor, torch.nn.Parameter) or t.dtype != BF16 or t.device != dev):
             return False
     return not (torch.compiler.is_compiling() or torch.jit.is_tracing()
-                or torch.is_autocast_enabled("cuda") or forward_ad._current_level >= 0
+                or torch.is_autocast_enabled("cuda") or any(map(_has_tangent, tensors))
                 or torch._C._functorch.peek_interpreter_stack() is not None)
+
+
+def _has_tangent(t: torch.Tensor) -> bool:
+    return forward_ad._current_level >= 0 and forward_ad.unpack_dual(t).tangent is not None
+
+
+def _differentiated(*tensors: torch.Tensor) -> bool:
+    """Whether a backward on these tensors (the gradient that comes in and the
+    saved ones) is differentiated itself (``create_graph=True``, forward mode
+    over it) and so goes through the formula."""
+    return torch.is_grad_enabled() or any(map(_has_tangent, tensors))
 
 
 def _formula_grads(formula, inputs, needs, grads):
@@ -43,7 +55,8 @@ def _formula_grads(formula, inputs, needs, grads):
         inputs = [t.view_as(t) for t in inputs]
         out = formula(*inputs)
     wanted = [t for t, n in zip(inputs, needs) if n]
-    got = iter(torch.autograd.grad(out, wanted, grads, create_graph=True, allow_unused=True))
+    got = iter(torch.autograd.grad(out, wanted, grads, create_graph=torch.is_grad_enabled(),
+                                   allow_unused=True))
     return tuple(next(got) if n else None for n in needs)
 
 
@@ -105,7 +118,7 @@ class RmsNorm(torch.autograd.Function):
     def backward(ctx, dy):
         x, weight, mean = ctx.saved_tensors
         need = ctx.needs_input_grad
-        if torch.is_grad_enabled():
+        if _differentiated(dy, x, weight):
             return (*_formula_grads(lambda x, w: rms_norm_formula(x, w, ctx.eps), (x, weight),
                                     need[:2], dy), None)
         n = x.shape[-1]
@@ -145,7 +158,7 @@ class SiluMul(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         gate_up, = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if _differentiated(dy, gate_up):
             return _formula_grads(silu_mul_formula, (gate_up,), ctx.needs_input_grad, dy)
         gate_up, dy = K._dense16(gate_up), K._dense16(dy)
         dgu = torch.empty_like(gate_up)
@@ -252,7 +265,7 @@ class QkvAttention(torch.autograd.Function):
         qkv, q_weight, k_weight, cache, q_mean, k_mean, qf, kt, vf, w = ctx.saved_tensors
         hq, hkv, eps, scale = ctx.args
         need = ctx.needs_input_grad
-        if torch.is_grad_enabled():  # create_graph: the gradients are differentiated again
+        if _differentiated(dout, qkv, q_weight, k_weight):
             def formula(qkv, q_weight, k_weight):
                 return attention_formula(qkv, lambda a: rms_norm_formula(a, q_weight, eps),
                                          lambda a: rms_norm_formula(a, k_weight, eps), cache, hq,

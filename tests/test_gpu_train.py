@@ -166,3 +166,48 @@ def test_shared_norm_weight_second_derivative(pkg, T, gpu):
     # with them the terms of the second derivative.
     assert all(_rel(a, b) < 2 ** -6 for a, b in zip(*out))
 
+
+def _functions(pkg, T, gpu):
+    """(fused, formula, inputs) of the three Functions, small."""
+    g = torch.Generator(device=gpu).manual_seed(11)
+    x, gu, qkv = (torch.randn(1, 5, n, generator=g, device=gpu).bfloat16() for n in (64, 32, 512))
+    w, qw, kw = (torch.rand(n, generator=g, device=gpu).bfloat16() + 0.5 for n in (64, 128, 128))
+    cache = pkg.qwen3_naive.get_rope(128, 64, 1e6).cos_sin_cache.to(gpu)
+    return [(lambda x, w: T.RmsNorm.apply(x, w, 1e-6), lambda x, w: T.rms_norm_formula(x, w, 1e-6), (x, w)),
+            (T.SiluMul.apply, T.silu_mul_formula, (gu,)),
+            (lambda *z: T.QkvAttention.apply(*z, cache, 2, 1, 1e-6, 0.09),
+             lambda z, a, b: T.attention_formula(z, lambda t: T.rms_norm_formula(t, a, 1e-6),
+                                                 lambda t: T.rms_norm_formula(t, b, 1e-6), cache, 2, 1, 0.09),
+             (qkv, qw, kw))]
+
+
+def test_forward_mode_over_a_backward(pkg, T, gpu):
+    from torch.autograd import forward_ad as fwAD
+    for fused, formula, inputs in _functions(pkg, T, gpu):
+        out = []
+        for f in (fused, formula):
+            leaves = [t.detach().clone().requires_grad_() for t in inputs]
+            y = f(*leaves)
+            with fwAD.dual_level():
+                tangent = torch.linspace(-1, 1, y.numel(), device=gpu).view_as(y).bfloat16()
+                dy = fwAD.make_dual(torch.ones_like(y), tangent)
+                if len(inputs) == 1:  # torch has no forward mode over silu's gradient
+                    with pytest.raises(NotImplementedError):
+                        torch.autograd.grad(y, leaves, dy)
+                    continue
+                got = [fwAD.unpack_dual(g) for g in torch.autograd.grad(y, leaves, dy)]
+                assert all(g.tangent is not None for g in got)
+                out.append([t.clone() for g in got for t in (g.primal, g.tangent)])
+        assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
+def test_checkpoint_recomputed_under_forward_mode(pkg, gpu):
+    """The recomputation of a checkpointed layer saves what its forward did."""
+    from torch.autograd import forward_ad as fwAD
+    from torch.utils.checkpoint import checkpoint
+    layer = _layer(pkg, gpu)
+    x = torch.randn(1, 9, 128, device=gpu).bfloat16().requires_grad_()
+    want = _grads(layer, layer(x), x)
+    y = checkpoint(layer, x, use_reentrant=False)
+    with fwAD.dual_level():
+        assert all(torch.equal(a, b) for a, b in zip(_grads(layer, y, x), want))
