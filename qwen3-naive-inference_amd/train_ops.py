@@ -6,8 +6,8 @@ kernels repeat its fp32 operations and bf16 roundings, sums along a row, the
 softmax and the products are the same torch calls on the same operands.  Only
 the norm weights' gradients are summed in another (fixed) order.  The formula
 serves every call the kernels do not take, and a backward that is
-differentiated itself (``create_graph=True``, forward mode) differentiates
-the formula.
+differentiated itself (``create_graph=True``, forward mode) or runs on a batch
+of gradients (vmap) goes through the formula.
 """
 from __future__ import annotations
 
@@ -41,11 +41,16 @@ def _has_tangent(t: torch.Tensor) -> bool:
     return forward_ad._current_level >= 0 and forward_ad.unpack_dual(t).tangent is not None
 
 
-def _differentiated(*tensors: torch.Tensor) -> bool:
+def _formula_backward(*tensors: torch.Tensor) -> bool:
     """Whether a backward on these tensors (the gradient that comes in and the
-    saved ones) is differentiated itself (``create_graph=True``, forward mode
-    over it) and so goes through the formula."""
-    return torch.is_grad_enabled() or any(map(_has_tangent, tensors))
+    saved ones) goes through the formula: it is differentiated itself
+    (``create_graph=True``, forward mode over it), or its gradient is a batch
+    (``is_grads_batched``, vmap) or another type, which kernels cannot read."""
+    batched = torch._C._functorch
+    return torch.is_grad_enabled() or any(
+        type(t) not in (torch.Tensor, torch.nn.Parameter) or _has_tangent(t)
+        or batched.is_legacy_batchedtensor(t) or batched.is_functorch_wrapped_tensor(t)
+        for t in tensors)
 
 
 def _formula_grads(formula, inputs, needs, grads):
@@ -118,7 +123,7 @@ class RmsNorm(torch.autograd.Function):
     def backward(ctx, dy):
         x, weight, mean = ctx.saved_tensors
         need = ctx.needs_input_grad
-        if _differentiated(dy, x, weight):
+        if _formula_backward(dy, x, weight):
             return (*_formula_grads(lambda x, w: rms_norm_formula(x, w, ctx.eps), (x, weight),
                                     need[:2], dy), None)
         n = x.shape[-1]
@@ -158,7 +163,7 @@ class SiluMul(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         gate_up, = ctx.saved_tensors
-        if _differentiated(dy, gate_up):
+        if _formula_backward(dy, gate_up):
             return _formula_grads(silu_mul_formula, (gate_up,), ctx.needs_input_grad, dy)
         gate_up, dy = K._dense16(gate_up), K._dense16(dy)
         dgu = torch.empty_like(gate_up)
@@ -265,7 +270,7 @@ class QkvAttention(torch.autograd.Function):
         qkv, q_weight, k_weight, cache, q_mean, k_mean, qf, kt, vf, w = ctx.saved_tensors
         hq, hkv, eps, scale = ctx.args
         need = ctx.needs_input_grad
-        if _differentiated(dout, qkv, q_weight, k_weight):
+        if _formula_backward(dout, qkv, q_weight, k_weight):
             def formula(qkv, q_weight, k_weight):
                 return attention_formula(qkv, lambda a: rms_norm_formula(a, q_weight, eps),
                                          lambda a: rms_norm_formula(a, k_weight, eps), cache, hq,

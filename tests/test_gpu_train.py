@@ -211,3 +211,29 @@ def test_checkpoint_recomputed_under_forward_mode(pkg, gpu):
     y = checkpoint(layer, x, use_reentrant=False)
     with fwAD.dual_level():
         assert all(torch.equal(a, b) for a, b in zip(_grads(layer, y, x), want))
+
+
+@pytest.mark.parametrize("vmap", ["is_grads_batched", "func"])
+def test_batched_gradients(pkg, T, gpu, vmap):
+    """A batch of output gradients in one backward gives what one at a time gives."""
+    for fused, _, inputs in _functions(pkg, T, gpu):
+        leaves = [t.detach().clone().requires_grad_() for t in inputs]
+        y = fused(*leaves)
+        dys = torch.linspace(-2, 2, 3 * y.numel(), device=gpu).view(3, *y.shape).bfloat16()
+        want = [torch.autograd.grad(y, leaves, d, retain_graph=True) for d in dys]
+        if vmap == "func":
+            got = torch.vmap(lambda d: torch.autograd.grad(y, leaves, d, retain_graph=True))(dys)
+        else:
+            got = torch.autograd.grad(y, leaves, dys, is_grads_batched=True)
+        # Sums over rows in another order, and batched products: one bf16 rounding.
+        for i, g in enumerate(got):
+            assert _rel(g, torch.stack([w[i] for w in want])) < 2 ** -8
+
+
+def test_vectorized_jacobian(pkg, gpu):
+    layer = _layer(pkg, gpu)
+    x = torch.randn(1, 2, 128, device=gpu).bfloat16()
+    for p in layer.parameters():
+        p.requires_grad_(False)
+    a, b = (torch.autograd.functional.jacobian(layer, x, vectorize=v) for v in (True, False))
+    assert _rel(a, b) < 2 ** -7
