@@ -701,8 +701,10 @@ PREFILL_LAYER_OUTPUT = 2048 * 6144
 
 
 def _plain(t: torch.Tensor, dtype: torch.dtype, device: int) -> bool:
-    return (t.dtype == dtype and t.get_device() == device and t.is_contiguous()
-            and t.data_ptr() % 16 == 0)
+    """A dense, aligned tensor of one GPU.  A subclass is none: its ops, not its
+    storage (a wrapper has none), say what it holds."""
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == dtype
+            and t.get_device() == device and t.is_contiguous() and t.data_ptr() % 16 == 0)
 
 
 def prefill_layer(x, residual, norms, mats, eps, positions, cos_sin_cache, num_q_heads, num_kv_heads,
@@ -738,6 +740,7 @@ def prefill_layer(x, residual, norms, mats, eps, positions, cos_sin_cache, num_q
             and positions.shape == (t,) and slot_mapping.shape == (t,)
             and cu_seqlens_k.shape == cu_seqlens_q.shape
             and block_table.shape[0] == bsz and block_table.shape[1] > 0
+            and type(block_table) is torch.Tensor
             and block_table.stride(1) == 1 and block_table.dtype == i32
             and block_table.get_device() == dev
             and cos_sin_cache.dim() == 2 and cos_sin_cache.shape[1] == HEAD_DIM):
@@ -754,7 +757,8 @@ def prefill_layer(x, residual, norms, mats, eps, positions, cos_sin_cache, num_q
         return None
     for a, dtype in ((positions, torch.int64), (slot_mapping, i32), (cu_seqlens_q, i32),
                      (cu_seqlens_k, i32)):
-        if a.dtype != dtype or a.get_device() != dev or not a.is_contiguous():
+        if (type(a) is not torch.Tensor or a.dtype != dtype or a.get_device() != dev
+                or not a.is_contiguous()):
             return None
     L = lib()
     device = x.device

@@ -159,3 +159,26 @@ def test_layer_in_a_graph(pkg, gpu):
             torch.cuda.synchronize()
             assert all(torch.equal(a, b) for a, b in zip(got, want))
             layer.forward_prefill(*args, residual=r)
+
+
+def test_layer_with_a_subclass_weight(pkg, gpu):
+    """A weight whose class has its own product (as a quantised one has) is used through it."""
+    seen = []
+
+    class Doubled(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            if func is torch.nn.functional.linear:
+                seen.append(1)
+                return func(args[0], args[1].as_subclass(torch.Tensor) * 2)
+            return super().__torch_function__(func, types, args, kwargs)
+
+    layer, cfg = _layer(pkg, gpu)
+    args, r = _batch(layer, cfg, gpu, [40], 0)
+    down = layer.mlp.down_proj
+    with torch.no_grad():
+        want, _ = layer.forward_prefill(*args, residual=r)
+        down.weight = torch.nn.Parameter(down.weight.detach().as_subclass(Doubled))
+        assert layer._prefill_native(*args, r) is None
+        got, _ = layer.forward_prefill(*args, residual=r)
+    assert seen and _rel(got, 2 * want) < 0.02
