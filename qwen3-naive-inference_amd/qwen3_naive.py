@@ -28,6 +28,7 @@ from functools import lru_cache
 import numpy as np
 import torch
 import torch.nn as nn
+from torch.utils._device import DeviceContext
 
 from . import kernels as K
 from . import train_ops as T
@@ -321,13 +322,13 @@ class Qwen3DecoderLayer(nn.Module):
 
     def _prefill_native(self, x, positions, cu_q, cu_k, max_q, max_k, slots, tables, residual):
         """The layer as one library call, or None: a call whose modules are
-        hooked, replaced or tracked by autograd, or that ``K.prefill_layer``
-        does not take, goes through the modules."""
+        hooked, replaced, watched by a mode or tracked by autograd, or that
+        ``K.prefill_layer`` does not take, goes through the modules."""
         sub = self._modules
         attn, mlp = sub.get("self_attn"), sub.get("mlp")
         if (tables is None or type(attn) is not Qwen3Attention or type(mlp) is not Qwen3MLP
                 or attn.k_cache is None or nn.modules.module._has_any_global_hook()
-                or torch.is_autocast_enabled("cuda") or _prefill_methods() != _PREFILL_METHODS):
+                or torch.is_autocast_enabled("cuda") or _observed() or _prefill_methods() != _PREFILL_METHODS):
             return None
         a, m = attn._modules, mlp._modules
         norms = (sub.get("input_layernorm"), a.get("q_norm"), a.get("k_norm"),
@@ -411,6 +412,14 @@ class Qwen3DecoderLayer(nn.Module):
         h = self.self_attn.forward_decode(h, positions, context_lens, block_tables, slot_mapping)
         h, residual = self.post_attention_layernorm(h, residual)
         return self.mlp.forward_decode(h), residual
+
+
+def _observed() -> bool:
+    """Whether a dispatch or function mode (a FLOP counter, a tracer; a default
+    device aside) is there to see the torch ops of a call."""
+    return torch._C._len_torch_dispatch_stack() > 0 or any(
+        type(torch._C._get_function_stack_at(i)) is not DeviceContext
+        for i in range(torch._C._len_torch_function_stack()))
 
 
 def _prefill_methods():

@@ -182,3 +182,25 @@ def test_layer_with_a_subclass_weight(pkg, gpu):
         assert layer._prefill_native(*args, r) is None
         got, _ = layer.forward_prefill(*args, residual=r)
     assert seen and _rel(got, 2 * want) < 0.02
+
+
+def test_layer_under_a_mode(pkg, gpu):
+    """A mode sees the products; a default device is no such mode."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils.flop_counter import FlopCounterMode
+
+    class Watch(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    layer, cfg = _layer(pkg, gpu)
+    args, r = _batch(layer, cfg, gpu, [40], 0)
+    with torch.no_grad():
+        with torch.device(gpu):
+            assert layer._prefill_native(*args, r) is not None
+        with Watch():
+            assert layer._prefill_native(*args, r) is None
+        with FlopCounterMode(display=False) as counter:
+            layer.forward_prefill(*args, residual=r)
+    h, i, qkv = cfg.hidden_size, cfg.intermediate_size, 8 * 128
+    assert counter.get_total_flops() == 2 * 40 * (h * qkv + 4 * 128 * h + 3 * h * i)
