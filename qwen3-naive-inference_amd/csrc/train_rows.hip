@@ -518,6 +518,9 @@ __global__ __launch_bounds__(16 * kSumGroups) void sum_rows_kernel(const float* 
 
 inline bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// A launch has fewer than 2^32 lanes in x, whole workgroups.
+constexpr int64_t kMaxLanes = (1LL << 32) - kThreads;
+
 // Items of 8 elements; 32-bit item arithmetic.
 int check_rows(int64_t rows, int64_t stride, int64_t heads, int64_t n) {
   if (rows <= 0 || heads <= 0 || n <= 0 || rows % heads) return QMI_E_BAD_SHAPE;
@@ -530,7 +533,9 @@ unsigned grid_of(int64_t items) { return (unsigned)((items + kThreads - 1) / kTh
 
 int check_heads(int64_t batch, int64_t t, int64_t hq, int64_t hkv) {
   if (batch <= 0 || t <= 0 || hq <= 0 || hkv <= 0 || hq % hkv) return QMI_E_BAD_SHAPE;
-  if (batch > 65535 || hkv > 65535 || batch * t * (hq + hkv) > 0x7fffff00LL) return QMI_E_UNSUPPORTED;
+  if (batch > 65535 || t > 0x7fffffffLL || hq > 65535 || hkv > 65535 ||
+      batch * t * (hq + hkv) > kMaxLanes / 16)
+    return QMI_E_UNSUPPORTED;
   return QMI_OK;
 }
 
@@ -657,7 +662,7 @@ extern "C" int qmi_train_heads(float* f, uint16_t* o, int64_t batch, int64_t t, 
 extern "C" int qmi_scale_mask(const float* s, int64_t rows, int64_t t, float scale, float masked, float* out,
                               void* stream) {
   if (rows <= 0 || t <= 0 || rows % t) return QMI_E_BAD_SHAPE;
-  if (rows > 0x7fffffffLL || t > 0x7fffffffLL / 4) return QMI_E_UNSUPPORTED;
+  if (rows > kMaxLanes / kThreads || t > 0x7fffffffLL / 4) return QMI_E_UNSUPPORTED;
   if (!s || !out) return QMI_E_NULL_POINTER;
   if (!al16(s) || !al16(out)) return QMI_E_BAD_STRIDE;
   hipLaunchKernelGGL(scale_mask_kernel, dim3((unsigned)rows), dim3(kThreads), 0, QMI_ST, s, (int)t, scale, masked,
@@ -677,7 +682,7 @@ extern "C" int qmi_sum_rows(const float* x, int64_t parts, int64_t n, uint16_t* 
 extern "C" int qmi_causal_softmax(const float* s, const float* w, int64_t rows, int64_t t, float scale,
                                   float* out, void* stream) {
   if (rows <= 0 || t <= 0 || rows % t) return QMI_E_BAD_SHAPE;
-  if (rows > 0x7fffffffLL || t > 1024) return QMI_E_UNSUPPORTED;
+  if (rows > kMaxLanes / 64 || t > 1024) return QMI_E_UNSUPPORTED;
   if (!s || !out) return QMI_E_NULL_POINTER;
   const dim3 grid((unsigned)((rows + kThreads / 64 - 1) / (kThreads / 64)));
 #define QMI_CS(NI)                                                                                       \

@@ -213,12 +213,19 @@ def attention_formula(qkv, norm_q, norm_k, cache, num_heads, num_kv_heads, scale
     return o.transpose(1, 2).reshape(batch, seq_len, -1)
 
 
+def _score_rows_ok(rows: int, t: int) -> bool:
+    """Whether one launch (fewer than 2^32 lanes) covers the score rows: a wave
+    of 64 lanes per row, 256 lanes above ``SOFTMAX_MAX`` columns."""
+    return rows < 1 << (26 if t <= SOFTMAX_MAX else 24)
+
+
 def attention_ok(qkv, q_weight, k_weight, cache, num_heads, num_kv_heads) -> bool:
     """Whether ``QkvAttention`` takes this batch."""
     return (kernels_ok(qkv, q_weight, k_weight) and qkv.dim() == 3 and qkv.numel() > 0
             and qkv.is_contiguous() and qkv.data_ptr() % 16 == 0 and num_heads % num_kv_heads == 0
             and qkv.shape[2] == (num_heads + 2 * num_kv_heads) * HEAD_DIM
-            and qkv.shape[0] * num_heads * qkv.shape[1] < 1 << 27 and qkv.shape[0] <= 65535
+            and _score_rows_ok(qkv.shape[0] * num_heads * qkv.shape[1], qkv.shape[1])
+            and qkv.shape[0] <= 65535
             and q_weight.shape == k_weight.shape == (HEAD_DIM,)
             and cache.dtype == F32 and cache.device == qkv.device and cache.is_contiguous()
             and cache.data_ptr() % 16 == 0 and cache.shape[1] == HEAD_DIM

@@ -104,3 +104,18 @@ def test_product_fails_loudly_without_library(pkg, monkeypatch, tmp_path):
     monkeypatch.setattr(pkg._lib, "LIB_PATH", tmp_path / "missing.so")
     with pytest.raises(pkg._lib.QmiError):
         pkg._lib.lib()
+
+
+def test_training_rows_beyond_one_launch(pkg):
+    """A launch has fewer than 2^32 lanes: larger calls are refused, and the
+    attention of such a batch is not taken."""
+    import importlib
+    L, fake = pkg._lib.lib(), 256
+    assert L.qmi_scale_mask(fake, 1 << 24, 2048, 1.0, 0.0, fake, None) == -4
+    assert L.qmi_causal_softmax(fake, None, 1 << 26, 1024, 1.0, fake, None) == -4
+    assert L.qmi_causal_softmax(fake, fake, 1 << 26, 1024, 1.0, fake, None) == -4
+    assert L.qmi_train_heads(fake, fake, 1, 1 << 23, 16, 1, None) == -4
+    assert L.qmi_train_qkv(fake, 32 * 128, 1, 1 << 24, 8, 8, *[fake] * 4, 1e-6, *[fake] * 4, None) == -4
+    T = importlib.import_module(pkg.__name__ + ".train_ops")
+    assert T._score_rows_ok((1 << 26) - 64, 1024) and not T._score_rows_ok(1 << 26, 64)
+    assert T._score_rows_ok((1 << 24) - 2048, 2048) and not T._score_rows_ok(1 << 24, 2048)
