@@ -284,12 +284,12 @@ class QkvAttention(torch.autograd.Function):
                                          hkv, scale)
             return (*_formula_grads(formula, (qkv, q_weight, k_weight), need[:3], dout), None, None,
                     None, None, None)
-        qkv, cache = K._dense16(qkv), K._dense16(cache)
+        qkv, cache, dout = K._dense16(qkv), K._dense16(cache), K._dense16(dout)
         b, t, width = qkv.shape
         dev, d = qkv.device, HEAD_DIM
         qw, kw = K._dense16(q_weight), K._dense16(k_weight)
         do = torch.empty((b * hq, t, d), dtype=F32, device=dev)
-        _call("qmi_train_heads", dev, do.data_ptr(), K._dense16(dout).data_ptr(), b, t, hq, 0)
+        _call("qmi_train_heads", dev, do.data_ptr(), dout.data_ptr(), b, t, hq, 0)
         dw = torch.bmm(do, vf.transpose(1, 2))
         dv = torch.bmm(w.transpose(1, 2), do)
         ds = torch.empty_like(dw)

@@ -1,5 +1,10 @@
-"""Which tensors the one-call prefill layer and the training Functions may read
+"""Which tensors the one-call prefill layer and the training Functions read
 through their addresses (CPU: no kernel is launched)."""
+import importlib
+import types
+import weakref
+
+import pytest
 import torch
 
 
@@ -29,3 +34,39 @@ def test_prefill_layer_takes_plain_tensors_only(pkg):
     assert not ok(t.as_subclass(Plain), torch.bfloat16, -1)
     assert not ok(torch.nn.Parameter(t.as_subclass(Plain)), torch.bfloat16, -1)
     assert not ok(Wrapper(t), torch.bfloat16, -1)
+
+
+@pytest.mark.parametrize("name", ["norm", "silu", "attention"])
+def test_backward_keeps_its_copies_until_the_launch(pkg, monkeypatch, name):
+    """A copy made to be dense is alive when a kernel that gets its address is
+    launched (freed earlier, another thread's allocation may write to it)."""
+    T = importlib.import_module(pkg.__name__ + ".train_ops")
+    copies, passed = {}, []
+
+    def copy(t):
+        c = t.contiguous().clone()
+        copies[c.data_ptr()] = weakref.ref(c)
+        return c
+
+    def call(entry, device, *args):
+        for a in args:
+            if a in copies:
+                assert copies[a]() is not None, f"{entry}: the copy at {a:#x} is gone"
+                passed.append(a)
+
+    monkeypatch.setattr(pkg.kernels, "_dense16", copy)
+    monkeypatch.setattr(T, "_call", call)
+    b16 = torch.bfloat16
+    x, w = torch.zeros(1, 5, 512, dtype=b16), torch.zeros(512, dtype=b16)
+    f = torch.zeros(2, 5, 128)
+    cls, saved, out, args = {
+        "norm": (T.RmsNorm, (x, w, torch.zeros(1, 5, 1)), x.shape, {"eps": 1e-6}),
+        "silu": (T.SiluMul, (x,), (1, 5, 256), {}),
+        "attention": (T.QkvAttention, (x, w[:128], w[128:256], torch.zeros(64, 128), torch.zeros(1, 5, 2, 1),
+                                       torch.zeros(1, 5, 1, 1), f, f.transpose(1, 2).contiguous(), f,
+                                       torch.zeros(2, 5, 5)), (1, 5, 256), {"args": (2, 1, 1e-6, 0.1)}),
+    }[name]
+    ctx = types.SimpleNamespace(saved_tensors=saved, needs_input_grad=(True,) * 3, **args)
+    with torch.no_grad():
+        cls.backward(ctx, torch.zeros((), dtype=b16).expand(out))
+    assert passed
