@@ -127,7 +127,7 @@ class RmsNorm(torch.autograd.Function):
             return (*_formula_grads(lambda x, w: rms_norm_formula(x, w, ctx.eps), (x, weight),
                                     need[:2], dy), None)
         n = x.shape[-1]
-        x = K._dense16(x)  # saved-tensor hooks may have moved it
+        x, mean = K._dense16(x), K._dense16(mean)  # saved-tensor hooks may have laid them out anew
         dx = torch.empty_like(x)
         dw = _norm_grad(x, x.numel() // n, n, 1, n, x.shape, mean, K._dense16(weight), ctx.eps,
                         K._dense16(dy), dx)
@@ -284,7 +284,7 @@ class QkvAttention(torch.autograd.Function):
                                          hkv, scale)
             return (*_formula_grads(formula, (qkv, q_weight, k_weight), need[:3], dout), None, None,
                     None, None, None)
-        qkv, cache, dout = K._dense16(qkv), K._dense16(cache), K._dense16(dout)
+        qkv, cache, q_mean, k_mean, w, dout = map(K._dense16, (qkv, cache, q_mean, k_mean, w, dout))
         b, t, width = qkv.shape
         dev, d = qkv.device, HEAD_DIM
         qw, kw = K._dense16(q_weight), K._dense16(k_weight)

@@ -237,3 +237,23 @@ def test_vectorized_jacobian(pkg, gpu):
         p.requires_grad_(False)
     a, b = (torch.autograd.functional.jacobian(layer, x, vectorize=v) for v in (True, False))
     assert _rel(a, b) < 2 ** -7
+
+
+def test_saved_tensors_in_another_layout(pkg, T, gpu):
+    """Hooks may give saved tensors back with other strides."""
+    def spread(t):
+        buf = torch.zeros((*t.shape, 2), dtype=t.dtype, device=t.device)
+        buf[..., 0] = t.detach()
+        return buf[..., 0]
+
+    for fused, _, inputs in _functions(pkg, T, gpu):
+        res = []
+        for hooked in (False, True):
+            leaves = [t.detach().clone().requires_grad_() for t in inputs]
+            if hooked:
+                with torch.autograd.graph.saved_tensors_hooks(spread, lambda t: t):
+                    y = fused(*leaves)
+            else:
+                y = fused(*leaves)
+            res.append(torch.autograd.grad(y, leaves, torch.linspace(-1, 1, y.numel(), device=gpu).view_as(y).bfloat16()))
+        assert all(torch.equal(a, b) for a, b in zip(*res))
