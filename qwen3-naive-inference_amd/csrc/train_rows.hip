@@ -404,9 +404,9 @@ __global__ __launch_bounds__(kThreads) void scale_mask_kernel(const float* __res
 // columns l, l + 64, ..., adds its own in that order and the lanes by a
 // butterfly of offsets 32 .. 1, the order of torch's softmax kernels for rows
 // of at most 1,024, whose bits these are.  Columns past the diagonal hold
-// exact zeros and are not read.  At 8 x 16 x 640 x 640 (210 MB) the forward
-// reads half of it and writes it once, where mask and softmax moved four times
-// as much; the backward likewise.
+// exact zeros; the forward does not read them.  At 8 x 16 x 640 x 640 (210 MB)
+// the forward reads half of it and writes it once, where mask and softmax moved
+// four times as much; the backward reads half of w and all of dp.
 __device__ __forceinline__ float butterfly_sum(float x) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
@@ -445,15 +445,17 @@ __global__ __launch_bounds__(kThreads) void causal_softmax_kernel(const float* _
     sum += v[i];
   }
   sum = butterfly_sum(sum);
+  const float past = 0.f / sum;  // a row of infinities or NaN is NaN past the diagonal too
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int j = lane + 64 * i;
-    if (j < t) y[j] = j <= q ? v[i] / sum : 0.f;
+    if (j < t) y[j] = j <= q ? v[i] / sum : past;
   }
 }
 
 // ds = (dp * w - w * sum(dp * w)) * scale, the difference an FMA as in torch's
-// kernel.
+// kernel.  dp past the diagonal is read for its infinities and NaN, which make
+// the row's sum NaN although w is zero there.
 template <int NI>
 __global__ __launch_bounds__(kThreads) void causal_softmax_grad_kernel(const float* __restrict__ dp,
                                                                        const float* __restrict__ w,
@@ -471,11 +473,8 @@ __global__ __launch_bounds__(kThreads) void causal_softmax_grad_kernel(const flo
   for (int i = 0; i < NI; ++i) {
     const int j = lane + 64 * i;
     o[i] = g[i] = 0.f;
-    if (64 * i > q) continue;
-    if (j <= q) {
-      o[i] = pw[j];
-      g[i] = p[j] * o[i];
-    }
+    if (j <= q) o[i] = pw[j];
+    if (j < t) g[i] = p[j] * o[i];
     sum += g[i];
   }
   sum = butterfly_sum(sum);

@@ -257,3 +257,41 @@ def test_saved_tensors_in_another_layout(pkg, T, gpu):
                 y = fused(*leaves)
             res.append(torch.autograd.grad(y, leaves, torch.linspace(-1, 1, y.numel(), device=gpu).view_as(y).bfloat16()))
         assert all(torch.equal(a, b) for a, b in zip(*res))
+
+
+# One chunk, several, and the unfused softmax; a value of q, k or v in the
+# middle of the rows, upstream gradients of zero before it.
+@pytest.mark.parametrize("t", [5, 150, 1030])
+@pytest.mark.parametrize("where", [3, 259, 391])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_attention_nonfinite(pkg, T, gpu, t, where, value):
+    g = torch.Generator(device=gpu).manual_seed(t)
+    qkv = torch.randn(1, t, 512, generator=g, device=gpu).bfloat16()
+    qkv[0, t // 2, where] = value
+    qw, kw = (torch.rand(128, generator=g, device=gpu).bfloat16() + 0.5 for _ in range(2))
+    cache = pkg.qwen3_naive.get_rope(128, 2048, 1e6).cos_sin_cache.to(gpu)
+    dy = torch.randn(1, t, 256, generator=g, device=gpu).bfloat16()
+    dy[:, :t // 2] = 0
+    out = []
+    for f in (lambda *z: T.QkvAttention.apply(*z, cache, 2, 1, 1e-6, 0.09),
+              lambda z, a, b: T.attention_formula(z, lambda x: T.rms_norm_formula(x, a, 1e-6),
+                                                  lambda x: T.rms_norm_formula(x, b, 1e-6), cache, 2, 1, 0.09)):
+        leaves = [a.clone().requires_grad_() for a in (qkv, qw, kw)]
+        y = f(*leaves)
+        y.backward(dy)
+        out.append([y] + [a.grad for a in leaves])
+    assert not out[1][0].isfinite().all()
+    for a, b in zip(out[0][:2], out[1][:2]):
+        torch.testing.assert_close(a, b, rtol=0, atol=0, equal_nan=True)
+    for a, b in zip(out[0][2:], out[1][2:]):
+        assert torch.equal(a.isnan(), b.isnan())
+
+
+def test_rows_nonfinite(pkg, T, gpu):
+    for fused, formula, inputs in _functions(pkg, T, gpu)[:2]:
+        x = inputs[0].clone()
+        for i, value in enumerate((float("inf"), float("-inf"), float("nan"))):
+            x[0, i, 3] = x[0, i, 20] = value
+        a, b = _both(fused, formula, (x, *inputs[1:]))
+        for p, q in zip(a[:2], b[:2]):
+            torch.testing.assert_close(p, q, rtol=0, atol=0, equal_nan=True)
