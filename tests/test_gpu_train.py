@@ -295,3 +295,34 @@ def test_rows_nonfinite(pkg, T, gpu):
         a, b = _both(fused, formula, (x, *inputs[1:]))
         for p, q in zip(a[:2], b[:2]):
             torch.testing.assert_close(p, q, rtol=0, atol=0, equal_nan=True)
+
+
+@pytest.mark.parametrize("part", ["norm", "attention"])
+def test_inputs_written_between_forward_and_backward(pkg, gpu, part):
+    """A residual stream updated in place, weights stepped and a projection's
+    output kept by a hook and written to: the gradients are the forward's."""
+    layer = _layer(pkg, gpu)
+    attn, norm = layer.self_attn, layer.input_layernorm
+    x = torch.randn(1, 9, 128, device=gpu).bfloat16().requires_grad_()
+    kept, res = [], []
+    cache = attn._cos_sin(gpu)
+    for write in (False, True):
+        h = x * 1
+        hook = attn.qkv_proj.register_forward_hook(lambda m, i, o: kept.append(o)) if write else None
+        y = norm(h) if part == "norm" else attn(h)
+        if write:
+            with torch.no_grad():
+                written = [h, norm.weight] if part == "norm" else [attn.q_norm.weight, attn.k_norm.weight,
+                                                                    cache, *kept]
+                before = [t.clone() for t in written]
+                for t in written:
+                    t.add_(1)
+            hook.remove()
+        res.append(_grads(layer, y, x))
+        if write:
+            with torch.no_grad():
+                for t, b in zip(written, before):
+                    t.copy_(b)
+    assert part == "norm" or kept
+    for a, b in zip(*res):
+        assert a is b is None or torch.equal(a, b)
