@@ -164,6 +164,9 @@ class RotaryEmbedding(nn.Module):
                 self.rotate(k, positions, self.cos_sin_cache))
 
 
+_ROTATE = RotaryEmbedding.rotate  # a program may replace it (another RoPE scaling)
+
+
 @lru_cache(8)
 def _rope_cpu(head_dim: int, max_position: int, rope_theta: float) -> RotaryEmbedding:
     return RotaryEmbedding(head_dim, max_position, rope_theta)
@@ -234,7 +237,9 @@ class Qwen3Attention(nn.Module):
         qkv = self.qkv_proj(x)
         cache = self._cos_sin(x.device)
         qw, kw = self.q_norm.weight, self.k_norm.weight
-        if (_unhooked_norms(self.q_norm, self.k_norm) and self.q_norm.eps == self.k_norm.eps
+        rotate = RotaryEmbedding.rotate
+        if (rotate is _ROTATE and _unhooked_norms(self.q_norm, self.k_norm)
+                and self.q_norm.eps == self.k_norm.eps
                 and T.attention_ok(qkv, qw, kw, cache, self.num_heads, self.num_kv_heads)):
             # What it saves is out of the program's reach, as what the formula saves
             # is: copies, and a qkv that only this call has seen.
@@ -246,7 +251,7 @@ class Qwen3Attention(nn.Module):
                                      self.num_heads, self.num_kv_heads, self.q_norm.eps, self.scale)
         else:
             o = T.attention_formula(qkv, self.q_norm, self.k_norm, cache, self.num_heads,
-                                    self.num_kv_heads, self.scale)
+                                    self.num_kv_heads, self.scale, rotate)
         return self.o_proj(o)
 
     # ----- continuous batching (qwen3_naive.py:597-683) -----
@@ -336,7 +341,8 @@ class Qwen3DecoderLayer(nn.Module):
         attn, mlp = sub.get("self_attn"), sub.get("mlp")
         if (tables is None or type(attn) is not Qwen3Attention or type(mlp) is not Qwen3MLP
                 or attn.k_cache is None or nn.modules.module._has_any_global_hook()
-                or torch.is_autocast_enabled("cuda") or _observed() or _prefill_methods() != _PREFILL_METHODS):
+                or torch.is_autocast_enabled("cuda") or _observed()
+                or _prefill_methods() != _PREFILL_METHODS or "_project_store" in attn.__dict__):
             return None
         a, m = attn._modules, mlp._modules
         norms = (sub.get("input_layernorm"), a.get("q_norm"), a.get("k_norm"),
@@ -382,15 +388,15 @@ class Qwen3DecoderLayer(nn.Module):
                                                   "post_attention_layernorm"))
         if (type(x) is not torch.Tensor or x.dim() != 2 or type(attn) is not Qwen3Attention
                 or type(mlp) is not Qwen3MLP or nn.modules.module._has_any_global_hook()
-                or (Qwen3Attention.forward_decode, Qwen3MLP.forward_decode, RMSNorm.forward,
-                    K.rms_norm, K.add_rms_norm) != _DECODE_METHODS):
+                or _decode_methods() != _DECODE_METHODS):
             return False
         for mod in (n1, n2):
             if (type(mod) is not RMSNorm or mod._forward_hooks or mod._forward_pre_hooks
                     or mod._backward_hooks or mod._backward_pre_hooks or "forward" in mod.__dict__
                     or mod.weight.shape != x.shape[1:]):
                 return False
-        if "forward_decode" in attn.__dict__ or "forward_decode" in mlp.__dict__:
+        if not ({"forward_decode", "_project_store"}.isdisjoint(attn.__dict__)
+                and "forward_decode" not in mlp.__dict__):
             return False
         qkv, o, gu = attn.qkv_proj, attn.o_proj, mlp.gate_up_proj
         if not (qkv.bias is None and o.bias is None and gu.bias is None
@@ -438,9 +444,14 @@ def _prefill_methods():
             K.qk_norm_rope_store, K.varlen_prefill_attention, K.silu_mul)
 
 
+def _decode_methods():
+    """The same of a decode layer whose norms run inside its projections."""
+    return (Qwen3Attention.forward_decode, Qwen3Attention._project_store, Qwen3MLP.forward_decode,
+            RMSNorm.forward, K.rms_norm, K.add_rms_norm)
+
+
 _PREFILL_METHODS = _prefill_methods()
-_DECODE_METHODS = (Qwen3Attention.forward_decode, Qwen3MLP.forward_decode, RMSNorm.forward,
-                   K.rms_norm, K.add_rms_norm)
+_DECODE_METHODS = _decode_methods()
 
 
 class Qwen3Model(nn.Module):

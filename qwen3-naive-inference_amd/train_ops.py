@@ -187,7 +187,7 @@ def rotate(x: torch.Tensor, positions: torch.Tensor, cache: torch.Tensor) -> tor
     return torch.cat((x1 * c - x2 * s, x2 * c + x1 * s), dim=-1).to(x.dtype)
 
 
-def attention_formula(qkv, norm_q, norm_k, cache, num_heads, num_kv_heads, scale):
+def attention_formula(qkv, norm_q, norm_k, cache, num_heads, num_kv_heads, scale, rotate=rotate):
     """QK-norm, RoPE and causal attention of ``qkv [B, T, (Hq + 2 Hkv) * D]`` ->
     ``[B, T, Hq * D]``; ``norm_q`` / ``norm_k`` map ``[B, T, heads, D]``."""
     batch, seq_len, width = qkv.shape

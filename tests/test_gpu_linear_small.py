@@ -90,3 +90,31 @@ def test_decode_layer_matches_modules(pkg, gpu, batch, first, fused_qkv):
         assert a.shape == b.shape and _rel(a, b) < 0.02
     layer.self_attn.k_cache, layer.self_attn.v_cache = kv
     assert not layer._norms_in_projections(x, r)  # weights tracked by autograd
+
+
+def test_replaced_projection_gets_rows(pkg, gpu, monkeypatch):
+    """A program's own _project_store, on the class or one module, is called with
+    the normed rows, as a tensor."""
+    torch.manual_seed(0)
+    cfg = pkg.Qwen3Config(hidden_size=1024, num_attention_heads=8, num_key_value_heads=4,
+                          intermediate_size=2048, num_hidden_layers=1, max_position_embeddings=1024)
+    layer = pkg.Qwen3DecoderLayer(cfg).to(gpu).bfloat16()
+    attn = layer.self_attn
+    attn.decode_fused_qkv = False
+    attn.k_cache, attn.v_cache = (torch.zeros(2, 256, 4, 128, device=gpu).bfloat16() for _ in range(2))
+    ctx = torch.zeros(2, dtype=torch.int32, device=gpu)
+    bt = torch.arange(2, dtype=torch.int32, device=gpu).view(2, 1)
+    x = torch.randn(2, 1024, device=gpu).bfloat16()
+    own, seen = pkg.qwen3_naive.Qwen3Attention._project_store, []
+
+    def wrapped(self, rows, *args, **kwargs):
+        seen.append(type(rows))
+        return own(self, rows, *args, **kwargs)
+
+    with torch.no_grad():
+        for target, name in ((pkg.qwen3_naive.Qwen3Attention, wrapped),
+                             (attn, lambda *a, **k: wrapped(attn, *a, **k))):
+            with monkeypatch.context() as mp:
+                mp.setattr(target, "_project_store", name)
+                layer.forward_decode(x, ctx.long(), ctx, bt)
+    assert seen == [torch.Tensor] * 2

@@ -70,3 +70,20 @@ def test_backward_keeps_its_copies_until_the_launch(pkg, monkeypatch, name):
     with torch.no_grad():
         cls.backward(ctx, torch.zeros((), dtype=b16).expand(out))
     assert passed
+
+
+def test_replaced_rotation_is_used(pkg, monkeypatch):
+    """A program's own RoPE, set on RotaryEmbedding, is the batch forward's."""
+    torch.manual_seed(0)
+    attn = pkg.Qwen3DecoderLayer(pkg.Qwen3Config(
+        hidden_size=64, num_attention_heads=2, num_key_value_heads=1, intermediate_size=64,
+        num_hidden_layers=1, max_position_embeddings=64)).self_attn
+    x, calls = torch.randn(1, 5, 64), []
+    want = attn(x)
+
+    def rotate(t, positions, cache):
+        calls.append(1)
+        return -t
+
+    monkeypatch.setattr(pkg.qwen3_naive.RotaryEmbedding, "rotate", staticmethod(rotate))
+    assert not torch.allclose(attn(x), want) and len(calls) == 2
