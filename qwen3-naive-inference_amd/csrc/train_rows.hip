@@ -467,14 +467,19 @@ __global__ __launch_bounds__(kThreads) void causal_softmax_grad_kernel(const flo
   const float* p = dp + (int64_t)row * t;
   const float* pw = w + (int64_t)row * t;
   float* y = ds + (int64_t)row * t;
+  // Loads without branches around them (indexes held inside the row), so that
+  // all are in flight at once.
   float g[NI], o[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) g[i] = p[min(lane + 64 * i, t - 1)];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) o[i] = 64 * i > q ? 0.f : pw[min(lane + 64 * i, q)];
   float sum = 0.f;
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int j = lane + 64 * i;
-    o[i] = g[i] = 0.f;
-    if (j <= q) o[i] = pw[j];
-    if (j < t) g[i] = p[j] * o[i];
+    if (j > q) o[i] = 0.f;
+    g[i] = j < t ? g[i] * o[i] : 0.f;
     sum += g[i];
   }
   sum = butterfly_sum(sum);
