@@ -443,7 +443,8 @@ int qmi_prefill_layer(const qmi_prefill_layer_args* args, void* stream);
  * 0, <= 65536) in each bf16 row of `stride`; fp32 arrays and dy are
  * contiguous.  Pointers 16-byte aligned.
  *   square_rows:  sq = x^2 (its row means are `mean` below)
- *   norm_apply:   y = bf16(x * rsqrt(mean + eps) * w), heads = 1, y contiguous
+ *   norm_apply:   y = bf16(x * rsqrt(mean + eps) * w), heads = 1, y contiguous;
+ *                 w_copy (or NULL): w as it was read
  *   norm_prod:    prod = (dy * w) * x, whose row sums are `dr` below
  *   norm_grad:    dx (laid out as x) and qmi_norm_grad_parts(rows, n) rows of
  *                 partial sums of dw
@@ -451,7 +452,9 @@ int qmi_prefill_layer(const qmi_prefill_layer_args* args, void* stream);
  *                 the gradient of the packed [rows][2 inter] gate_up
  *   train_qkv:    packed qkv [batch * t] rows -> normed, rotated q
  *                 [batch][hq][t][128], k transposed [batch][hq][128][t] and v
- *                 [batch][hq][t][128] in fp32, KV heads repeated
+ *                 [batch][hq][t][128] in fp32, KV heads repeated; w_copy
+ *                 [2][128] and cache_copy [t][128] (or NULL): the norm weights
+ *                 and cos/sin rows as they were read
  *   train_qkv_grad: gradients of those -> bf16 gradients of the norms' outputs
  *                 [batch * t][h][128], and v's into the packed d qkv
  *   train_heads:  fp32 [batch][heads][t][128] -> bf16 [batch][t][heads][128]
@@ -466,7 +469,7 @@ int qmi_prefill_layer(const qmi_prefill_layer_args* args, void* stream);
 int qmi_square_rows(const uint16_t* x, int64_t rows, int64_t stride, int64_t heads, int64_t n,
                     float* sq, void* stream);
 int qmi_norm_apply(const uint16_t* x, int64_t rows, int64_t stride, int64_t n, const float* mean,
-                   const uint16_t* w, float eps, uint16_t* y, void* stream);
+                   const uint16_t* w, float eps, uint16_t* y, uint16_t* w_copy, void* stream);
 int qmi_norm_prod(const uint16_t* x, int64_t rows, int64_t stride, int64_t heads, int64_t n,
                   const uint16_t* w, const uint16_t* dy, float* prod, void* stream);
 int64_t qmi_norm_grad_parts(int64_t rows, int64_t n);
@@ -478,7 +481,7 @@ int qmi_silu_mul_train(const uint16_t* gate_up, int64_t rows, int64_t inter, con
 int qmi_train_qkv(const uint16_t* qkv, int64_t stride, int64_t batch, int64_t t, int64_t hq,
                   int64_t hkv, const float* q_mean, const float* k_mean, const uint16_t* q_w,
                   const uint16_t* k_w, float eps, const float* cache, float* qf, float* kt,
-                  float* vf, void* stream);
+                  float* vf, uint16_t* w_copy, float* cache_copy, void* stream);
 int qmi_train_qkv_grad(int64_t batch, int64_t t, int64_t hq, int64_t hkv, const float* dq,
                        const float* dkt, const float* dv, const float* cache, uint16_t* dn_q,
                        uint16_t* dn_k, uint16_t* dqkv, void* stream);

@@ -93,14 +93,15 @@ SIGNATURES: dict[str, tuple] = {
     # The argument struct as bytes (kernels.PREFILL_LAYER_ARGS).
     "qmi_prefill_layer": (ctypes.c_int, [ctypes.c_char_p, _c_p]),
     "qmi_square_rows": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p]),
-    "qmi_norm_apply": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_f32, _c_p, _c_p]),
+    "qmi_norm_apply": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_f32, _c_p, _c_p,
+                                      _c_p]),
     "qmi_norm_prod": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_p]),
     "qmi_norm_grad_parts": (_c_i64, [_c_i64, _c_i64]),
     "qmi_norm_grad": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_f32, _c_p,
                                      _c_p, _c_p, _c_p, _c_p]),
     "qmi_silu_mul_train": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_p, _c_p, _c_p]),
     "qmi_train_qkv": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p,
-                                     _c_p, _c_f32, _c_p, _c_p, _c_p, _c_p, _c_p]),
+                                     _c_p, _c_f32, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p]),
     "qmi_train_qkv_grad": (ctypes.c_int, [_c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_p,
                                           _c_p, _c_p, _c_p, _c_p]),
     "qmi_train_heads": (ctypes.c_int, [_c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i32, _c_p]),

@@ -97,7 +97,8 @@ __global__ __launch_bounds__(kThreads) void square_kernel(const uint16_t* __rest
 
 __global__ __launch_bounds__(kThreads) void norm_apply_kernel(
     const uint16_t* __restrict__ x, Rows d, const float* __restrict__ mean,
-    const uint16_t* __restrict__ w, float eps, uint16_t* __restrict__ y) {
+    const uint16_t* __restrict__ w, float eps, uint16_t* __restrict__ y,
+    uint16_t* __restrict__ w_copy) {
   const int n8 = d.n / 8;
   const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   if (i >= d.rows * n8) return;
@@ -105,7 +106,9 @@ __global__ __launch_bounds__(kThreads) void norm_apply_kernel(
   const int col = (int)((uint32_t)i % (uint32_t)n8) * 8;
   const float r = inv_rms(mean[row], eps);
   V8 a = load8(x + d.at(row, col));
-  const V8 ww = load8(w + col);
+  const uint4 wr = load_u4(w + col);
+  if (w_copy && row == 0) *reinterpret_cast<uint4*>(w_copy + col) = wr;
+  const V8 ww = unpack8(wr);
 #pragma unroll
   for (int e = 0; e < 8; ++e) a.v[e] = a.v[e] * r * ww.v[e];
   *reinterpret_cast<uint4*>(y + 8 * i) = pack8(a);
@@ -262,7 +265,8 @@ struct Heads {
 // with each KV head repeated for its query heads.
 __global__ __launch_bounds__(kThreads) void qv_forward_kernel(
     Heads p, const float* __restrict__ q_mean, const uint16_t* __restrict__ q_w, float eps,
-    const float* __restrict__ cache, float* __restrict__ qf, float* __restrict__ vf) {
+    const float* __restrict__ cache, float* __restrict__ qf, float* __restrict__ vf,
+    uint16_t* __restrict__ w_copy) {
   const int lane16 = threadIdx.x & 15;
   const int per = p.hq + p.hkv;
   const uint32_t items = (uint32_t)p.batch * p.t * per;
@@ -272,7 +276,9 @@ __global__ __launch_bounds__(kThreads) void qv_forward_kernel(
   const uint16_t* row = p.qkv + (int64_t)tok * p.stride + 8 * lane16;
   if (h < p.hq) {
     const float r = inv_rms(q_mean[(int64_t)tok * p.hq + h], eps);
-    const V8 o = norm_rope(load8(row + h * kD), load8(q_w + 8 * lane16), r, cache + t * kD, lane16);
+    const uint4 wr = load_u4(q_w + 8 * lane16);
+    if (w_copy && item == 0) *reinterpret_cast<uint4*>(w_copy + 8 * lane16) = wr;
+    const V8 o = norm_rope(load8(row + h * kD), unpack8(wr), r, cache + t * kD, lane16);
     store8f(qf + (((int64_t)b * p.hq + h) * p.t + t) * kD + 8 * lane16, o);
   } else {
     const int hk = h - p.hq, rep = p.hq / p.hkv;
@@ -282,16 +288,22 @@ __global__ __launch_bounds__(kThreads) void qv_forward_kernel(
   }
 }
 
-// k: kt[b][h][128][t], repeated for the query heads.  Block: (64 tokens, KV head, sequence).
+// k: kt[b][h][128][t], repeated for the query heads.  Block: (64 tokens, KV head, sequence);
+// those of the first sequence and head copy the tokens' cos/sin rows, the first one the weights.
 __global__ __launch_bounds__(kThreads) void k_forward_kernel(
     Heads p, const float* __restrict__ k_mean, const uint16_t* __restrict__ k_w, float eps,
-    const float* __restrict__ cache, float* __restrict__ kt) {
+    const float* __restrict__ cache, float* __restrict__ kt, uint16_t* __restrict__ w_copy,
+    float* __restrict__ cache_copy) {
   __shared__ float tile[kD][kTile + 1];
   const int lane16 = threadIdx.x & 15, t0 = blockIdx.x * kTile, hk = blockIdx.y, b = blockIdx.z;
+  if (w_copy && blockIdx.x == 0 && hk == 0 && b == 0 && threadIdx.x < 16)
+    *reinterpret_cast<uint4*>(w_copy + 8 * lane16) = load_u4(k_w + 8 * lane16);
   for (int i = threadIdx.x / 16; i < kTile; i += 16) {
     const int t = min(t0 + i, p.t - 1);
     const int64_t tok = (int64_t)b * p.t + t;
     const float r = inv_rms(k_mean[tok * p.hkv + hk], eps);
+    if (cache_copy && hk == 0 && b == 0)
+      store8f(cache_copy + t * kD + 8 * lane16, load8f(cache + t * kD + 8 * lane16));
     const V8 o = norm_rope(load8(p.qkv + tok * p.stride + (p.hq + hk) * kD + 8 * lane16),
                            load8(k_w + 8 * lane16), r, cache + t * kD, lane16);
 #pragma unroll
@@ -559,13 +571,13 @@ extern "C" int qmi_square_rows(const uint16_t* x, int64_t rows, int64_t stride, 
 }
 
 extern "C" int qmi_norm_apply(const uint16_t* x, int64_t rows, int64_t stride, int64_t n, const float* mean,
-                              const uint16_t* w, float eps, uint16_t* y, void* stream) {
+                              const uint16_t* w, float eps, uint16_t* y, uint16_t* w_copy, void* stream) {
   const int e = check_rows(rows, stride, 1, n);
   if (e != QMI_OK) return e;
   if (!x || !mean || !w || !y) return QMI_E_NULL_POINTER;
-  if (!al16(x) || !al16(w) || !al16(y)) return QMI_E_BAD_STRIDE;
+  if (!al16(x) || !al16(w) || !al16(y) || !al16(w_copy)) return QMI_E_BAD_STRIDE;
   hipLaunchKernelGGL(norm_apply_kernel, dim3(grid_of(rows * (n / 8))), dim3(kThreads), 0, QMI_ST, x,
-                     Rows{rows, stride, 1, (int)n}, mean, w, eps, y);
+                     Rows{rows, stride, 1, (int)n}, mean, w, eps, y, w_copy);
   QMI_RETURN_LAUNCH_STATUS();
 }
 
@@ -617,18 +629,18 @@ extern "C" int qmi_silu_mul_train(const uint16_t* gate_up, int64_t rows, int64_t
 extern "C" int qmi_train_qkv(const uint16_t* qkv, int64_t stride, int64_t batch, int64_t t, int64_t hq,
                              int64_t hkv, const float* q_mean, const float* k_mean, const uint16_t* q_w,
                              const uint16_t* k_w, float eps, const float* cache, float* qf, float* kt,
-                             float* vf, void* stream) {
+                             float* vf, uint16_t* w_copy, float* cache_copy, void* stream) {
   const int e = check_heads(batch, t, hq, hkv);
   if (e != QMI_OK) return e;
   if (!qkv || !q_mean || !k_mean || !q_w || !k_w || !cache || !qf || !kt || !vf) return QMI_E_NULL_POINTER;
   if (stride < (hq + 2 * hkv) * kD || stride % 8 || !al16(qkv) || !al16(q_w) || !al16(k_w) || !al16(cache) ||
-      !al16(qf) || !al16(vf))
+      !al16(qf) || !al16(vf) || !al16(w_copy) || !al16(cache_copy))
     return QMI_E_BAD_STRIDE;
   const Heads p{qkv, stride, (int)batch, (int)t, (int)hq, (int)hkv};
   hipLaunchKernelGGL(qv_forward_kernel, dim3((unsigned)((batch * t * (hq + hkv) + 15) / 16)), dim3(kThreads), 0,
-                     QMI_ST, p, q_mean, q_w, eps, cache, qf, vf);
+                     QMI_ST, p, q_mean, q_w, eps, cache, qf, vf, w_copy);
   hipLaunchKernelGGL(k_forward_kernel, dim3((unsigned)((t + kTile - 1) / kTile), (unsigned)hkv, (unsigned)batch),
-                     dim3(kThreads), 0, QMI_ST, p, k_mean, k_w, eps, cache, kt);
+                     dim3(kThreads), 0, QMI_ST, p, k_mean, k_w, eps, cache, kt, w_copy ? w_copy + kD : nullptr, cache_copy);
   QMI_RETURN_LAUNCH_STATUS();
 }
 

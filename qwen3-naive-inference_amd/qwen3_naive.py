@@ -106,9 +106,9 @@ class RMSNorm(nn.Module):
     def _torch(self, x, residual):
         if residual is None:
             if T.norm_ok(x, self.weight):
-                # On copies, as the formula's x.float() and weight.float() are: a
-                # program may write to either before the backward.
-                return T.RmsNorm.apply(x.clone(), self.weight.clone(), self.eps)
+                # On a copy, as the formula's x.float() is: a program may write to
+                # x before the backward.
+                return T.RmsNorm.apply(x.clone(), self.weight, self.eps)
             return T.rms_norm_formula(x, self.weight, self.eps)
         dt = x.dtype
         xf = x.float() + residual.float()
@@ -241,14 +241,13 @@ class Qwen3Attention(nn.Module):
         if (rotate is _ROTATE and _unhooked_norms(self.q_norm, self.k_norm)
                 and self.q_norm.eps == self.k_norm.eps
                 and T.attention_ok(qkv, qw, kw, cache, self.num_heads, self.num_kv_heads)):
-            # What it saves is out of the program's reach, as what the formula saves
-            # is: copies, and a qkv that only this call has seen.
+            # The formula saves copies of qkv, which a hook may have kept and write to.
             proj = self.qkv_proj
             if (type(proj) is not nn.Linear or proj._forward_hooks
                     or nn.modules.module._has_any_global_hook()):
                 qkv = qkv.clone()
-            o = T.QkvAttention.apply(qkv, qw.clone(), kw.clone(), cache[:qkv.shape[1]].clone(),
-                                     self.num_heads, self.num_kv_heads, self.q_norm.eps, self.scale)
+            o = T.QkvAttention.apply(qkv, qw, kw, cache, self.num_heads, self.num_kv_heads,
+                                     self.q_norm.eps, self.scale)
         else:
             o = T.attention_formula(qkv, self.q_norm, self.k_norm, cache, self.num_heads,
                                     self.num_kv_heads, self.scale, rotate)

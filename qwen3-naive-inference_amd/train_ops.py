@@ -65,6 +65,11 @@ def _formula_grads(formula, inputs, needs, grads):
     return tuple(next(got) if n else None for n in needs)
 
 
+def _linked(t: torch.Tensor, copy: torch.Tensor, version: int) -> torch.Tensor:
+    """The values of ``copy`` (``t``'s when it had that version) in ``t``'s graph."""
+    return t if t._version == version else copy + (t - t.detach())
+
+
 def _call(name, device, *args):
     check(getattr(lib(), name)(*args, stream_handle(device)), name)
 
@@ -106,17 +111,20 @@ def norm_ok(x, weight) -> bool:
 
 
 class RmsNorm(torch.autograd.Function):
+    """``rms_norm_formula``.  The weight may be written to before the backward,
+    which reads a copy that the kernel leaves; ``x`` may not."""
+
     @staticmethod
     def forward(ctx, x, weight, eps):
         n = x.shape[-1]
         rows = x.numel() // n
         w = K._dense16(weight)
         mean = _mean_square(x, rows, n, 1, n, x.shape)
-        y = torch.empty_like(x)
+        y, w_copy = torch.empty_like(x), torch.empty_like(w)
         _call("qmi_norm_apply", x.device, x.data_ptr(), rows, n, n, mean.data_ptr(), w.data_ptr(),
-              eps, y.data_ptr())
-        ctx.save_for_backward(x, weight, mean)
-        ctx.eps = eps
+              eps, y.data_ptr(), w_copy.data_ptr())
+        ctx.save_for_backward(x, w_copy, mean)
+        ctx.weight, ctx.version, ctx.eps = weight, weight._version, eps
         return y
 
     @staticmethod
@@ -124,6 +132,8 @@ class RmsNorm(torch.autograd.Function):
         x, weight, mean = ctx.saved_tensors
         need = ctx.needs_input_grad
         if _formula_backward(dy, x, weight):
+            with torch.enable_grad():
+                weight = _linked(ctx.weight, weight, ctx.version)
             return (*_formula_grads(lambda x, w: rms_norm_formula(x, w, ctx.eps), (x, weight),
                                     need[:2], dy), None)
         n = x.shape[-1]
@@ -239,7 +249,9 @@ SOFTMAX_MAX = 1024
 
 class QkvAttention(torch.autograd.Function):
     """``attention_formula`` with RMS norms of a packed bf16 qkv; the backward
-    writes one packed ``d qkv``."""
+    writes one packed ``d qkv``.  The norm weights and the cos/sin cache may be
+    written to before the backward, which reads copies that the kernels leave;
+    ``qkv`` may not."""
 
     @staticmethod
     def forward(ctx, qkv, q_weight, k_weight, cache, hq, hkv, eps, scale):
@@ -251,9 +263,11 @@ class QkvAttention(torch.autograd.Function):
         qf = torch.empty((b * hq, t, d), dtype=F32, device=dev)
         kt = torch.empty((b * hq, d, t), dtype=F32, device=dev)
         vf = torch.empty_like(qf)
+        w_copy = torch.empty((2, d), dtype=BF16, device=dev)
+        cache_copy = torch.empty((t, d), dtype=F32, device=dev)
         _call("qmi_train_qkv", dev, qkv.data_ptr(), width, b, t, hq, hkv, q_mean.data_ptr(),
               k_mean.data_ptr(), qw.data_ptr(), kw.data_ptr(), eps, cache.data_ptr(), qf.data_ptr(),
-              kt.data_ptr(), vf.data_ptr())
+              kt.data_ptr(), vf.data_ptr(), w_copy.data_ptr(), cache_copy.data_ptr())
         scores = torch.bmm(qf, kt)
         # Kernels write to tensors of their own: a dispatch mode (selective
         # checkpointing) may keep what a torch op returned, and sees no write.
@@ -268,16 +282,20 @@ class QkvAttention(torch.autograd.Function):
         o = torch.bmm(w, vf)
         out = torch.empty((b, t, hq * d), dtype=BF16, device=dev)
         _call("qmi_train_heads", dev, o.data_ptr(), out.data_ptr(), b, t, hq, 1)
-        ctx.save_for_backward(qkv, q_weight, k_weight, cache, q_mean, k_mean, qf, kt, vf, w)
+        ctx.save_for_backward(qkv, w_copy, cache_copy, q_mean, k_mean, qf, kt, vf, w)
+        ctx.weights = [(p, p._version) for p in (q_weight, k_weight)]
         ctx.args = (hq, hkv, eps, scale)
         return out
 
     @staticmethod
     def backward(ctx, dout):
-        qkv, q_weight, k_weight, cache, q_mean, k_mean, qf, kt, vf, w = ctx.saved_tensors
+        qkv, weights, cache, q_mean, k_mean, qf, kt, vf, w = ctx.saved_tensors
         hq, hkv, eps, scale = ctx.args
         need = ctx.needs_input_grad
-        if _formula_backward(dout, qkv, q_weight, k_weight):
+        if _formula_backward(dout, qkv, weights):
+            with torch.enable_grad():
+                q_weight, k_weight = (_linked(p, c, v) for (p, v), c in zip(ctx.weights, weights))
+
             def formula(qkv, q_weight, k_weight):
                 return attention_formula(qkv, lambda a: rms_norm_formula(a, q_weight, eps),
                                          lambda a: rms_norm_formula(a, k_weight, eps), cache, hq,
@@ -287,7 +305,7 @@ class QkvAttention(torch.autograd.Function):
         qkv, cache, q_mean, k_mean, w, dout = map(K._dense16, (qkv, cache, q_mean, k_mean, w, dout))
         b, t, width = qkv.shape
         dev, d = qkv.device, HEAD_DIM
-        qw, kw = K._dense16(q_weight), K._dense16(k_weight)
+        qw, kw = K._dense16(weights)
         do = torch.empty((b * hq, t, d), dtype=F32, device=dev)
         _call("qmi_train_heads", dev, do.data_ptr(), dout.data_ptr(), b, t, hq, 0)
         dw = torch.bmm(do, vf.transpose(1, 2))

@@ -115,7 +115,8 @@ def test_training_rows_beyond_one_launch(pkg):
     assert L.qmi_causal_softmax(fake, None, 1 << 26, 1024, 1.0, fake, None) == -4
     assert L.qmi_causal_softmax(fake, fake, 1 << 26, 1024, 1.0, fake, None) == -4
     assert L.qmi_train_heads(fake, fake, 1, 1 << 23, 16, 1, None) == -4
-    assert L.qmi_train_qkv(fake, 32 * 128, 1, 1 << 24, 8, 8, *[fake] * 4, 1e-6, *[fake] * 4, None) == -4
+    assert L.qmi_train_qkv(fake, 32 * 128, 1, 1 << 24, 8, 8, *[fake] * 4, 1e-6, *[fake] * 4, None, None,
+                           None) == -4
     T = importlib.import_module(pkg.__name__ + ".train_ops")
     assert T._score_rows_ok((1 << 26) - 64, 1024) and not T._score_rows_ok(1 << 26, 64)
     assert T._score_rows_ok((1 << 24) - 2048, 2048) and not T._score_rows_ok(1 << 24, 2048)

@@ -326,3 +326,22 @@ def test_inputs_written_between_forward_and_backward(pkg, gpu, part):
     assert part == "norm" or kept
     for a, b in zip(*res):
         assert a is b is None or torch.equal(a, b)
+
+
+@pytest.mark.parametrize("written", [False, True])
+def test_second_derivative_after_a_weight_was_written(pkg, T, gpu, written):
+    for fused, formula, inputs in _functions(pkg, T, gpu)[::2]:
+        out = []
+        for f in (fused, formula):
+            leaves = [t.detach().clone().requires_grad_() for t in inputs]
+            y = f(*leaves)
+            if written:
+                with torch.no_grad():
+                    for w in leaves[1:]:
+                        w.add_(1)
+            first = torch.autograd.grad(y.float().square().sum(), leaves, create_graph=True)
+            second = torch.autograd.grad(sum(g.float().square().sum() for g in first), leaves)
+            out.append([*first, *second])
+        # Partial gradients are each rounded to bf16 before they are added (2^-8),
+        # at both levels.
+        assert all(_rel(a, b) < 2 ** -6 for a, b in zip(*out))
