@@ -628,11 +628,39 @@ class PendingNorm:
 
 LINEAR_SMALL_ROWS = 16
 LINEAR_SMALL_K = (1024, 2048, 3072, 4096)
+# A whole layer on linear_small: every workgroup normalises the rows anew, so
+# what it saves (two launches) shrinks with rows x depth, and o_proj / down_proj
+# cost more than as partial products (3072 -> 1024 at 12 rows 6.0 us against
+# 4.1).  Layer with its depths (hidden, heads, MLP) and 1 / largest / next
+# row count, us, against norms and linear_rows: (1024, 2048, 3072) 43.1 : 48.5 /
+# 12 rows 49.5 : 51.3 / 16 rows 52.3 : 50.9; (2048, 2048, 3072) 54.6 : 61.4 / 10
+# rows 63.1 : 63.3 / 14 rows 67.7 : 64.1; (4096, 2048, 4096) 73.6 : 83.7 / 6 rows
+# 81.3 : 83.2 / 10 rows 92.3 : 84.0.
+LINEAR_SMALL_CHAIN = 72 * 1024
+# One projection whose rows are there already, by depth: up to this many rows it
+# is faster than linear_rows, which reads the rows once per weight tile of twice
+# the height (1024 -> 2 x 3072 at 8 rows 6.1 us against 6.7, 16 rows 7.0 : 6.7;
+# 2048 -> 2 x 6144 13.8 : 14.5 / 16.7 : 14.5; 3072 -> 2 x 8192 at 2 rows 20.6 :
+# 21.2, 4 rows 22.0 : 21.1; 4096 -> 2 x 12288 at 8 rows 45.7 : 48.3, 12 rows 51.7 :
+# 48.5).
+LINEAR_SMALL_ALONE = {1024: 8, 2048: 8, 3072: 2, 4096: 8}
 
 
 def linear_small_ok(x: torch.Tensor) -> bool:
     """Whether ``linear_small`` takes a product that ``linear_rows_ok`` holds for."""
     return x.shape[0] <= LINEAR_SMALL_ROWS and x.shape[1] in LINEAR_SMALL_K
+
+
+def linear_small_wins(x: torch.Tensor) -> bool:
+    """Whether ``linear_small`` of these rows is faster than ``linear_rows``."""
+    return x.shape[0] <= LINEAR_SMALL_ALONE.get(x.shape[1], 0)
+
+
+def norms_in_projections_win(rows: int, *depths: int) -> bool:
+    """Whether a decode layer of these projection depths (hidden, heads x head
+    dim, MLP) is faster with its norms inside ``linear_small``."""
+    return (0 < rows <= LINEAR_SMALL_ROWS and rows * sum(depths) <= LINEAR_SMALL_CHAIN
+            and all(k in LINEAR_SMALL_K for k in depths))
 
 
 def linear_small(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = False,

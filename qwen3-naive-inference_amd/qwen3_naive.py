@@ -79,19 +79,20 @@ def _use_kernels(*tensors: torch.Tensor) -> bool:
     return all(t.is_cuda for t in tensors)
 
 
-def _decode_linear(proj: nn.Linear, x: torch.Tensor, parts: bool = False):
+def _decode_linear(proj: nn.Linear, x: torch.Tensor, parts: bool = False, small: bool = False):
     """A decode-step projection: the HIP decode-batch GEMM for bf16 inference
-    at <= 256 rows (as fp32 partial products when ``parts`` and above 16 rows:
-    the residual add + RMSNorm that follows sums them), else ``proj(x)``."""
+    at <= 256 rows (as fp32 partial products when ``parts``: the residual add +
+    RMSNorm that follows sums them; whole rows when ``small``: the norm that
+    follows is computed by ``linear_small``), else ``proj(x)``."""
     w = proj.weight
     if isinstance(x, K.PendingNorm):  # made for this projection by the layer
         return x.project(w)
     if proj.bias is None and _use_kernels(x, w) and K.linear_rows_ok(x, w):
-        if K.linear_small_ok(x):
+        if small and K.linear_small_ok(x):
             return K.linear_small(x, w)[0]
         if parts and w.shape[0] <= K.NORM_MAX_WIDTH:  # the norm that sums them takes the width
             return K.linear_rows_parts(x, w)
-        return K.linear_rows(x, w)
+        return K.linear_small(x, w)[0] if K.linear_small_wins(x) else K.linear_rows(x, w)
     return proj(x)
 
 
@@ -286,7 +287,7 @@ class Qwen3Attention(nn.Module):
             o = K.paged_decode_attention(q, self.k_cache, self.v_cache, context_lens,
                                          block_tables, self.scale, seqlen_bias=1,
                                          pages_per_split=self.decode_pages_per_split)
-        return _decode_linear(self.o_proj, o.view(batch, -1), parts=True)
+        return _decode_linear(self.o_proj, o.view(batch, -1), parts=True, small=rows is not x)
 
 
 class Qwen3MLP(nn.Module):
@@ -311,12 +312,12 @@ class Qwen3MLP(nn.Module):
         GEMMs at <= 256 rows; otherwise as ``forward``)."""
         w = self.gate_up_proj.weight
         if isinstance(x, K.PendingNorm):
-            return _decode_linear(self.down_proj, x.project(w, swiglu=True), parts=True)
+            return _decode_linear(self.down_proj, x.project(w, swiglu=True), parts=True, small=True)
         if (self.gate_up_proj.bias is None and _use_kernels(x, w)
                 and K.linear_rows_ok(x, w, swiglu=True)):
-            if K.linear_small_ok(x):
-                return _decode_linear(self.down_proj, K.linear_small(x, w, swiglu=True)[0], parts=True)
-            return _decode_linear(self.down_proj, K.linear_rows(x, w, swiglu=True), parts=True)
+            act = (K.linear_small(x, w, swiglu=True)[0] if K.linear_small_wins(x)
+                   else K.linear_rows(x, w, swiglu=True))
+            return _decode_linear(self.down_proj, act, parts=True)
         return self.forward(x)
 
 
@@ -385,8 +386,8 @@ class Qwen3DecoderLayer(nn.Module):
         sub = self._modules
         attn, mlp, n1, n2 = (sub.get(k) for k in ("self_attn", "mlp", "input_layernorm",
                                                   "post_attention_layernorm"))
-        if (type(x) is not torch.Tensor or x.dim() != 2 or type(attn) is not Qwen3Attention
-                or type(mlp) is not Qwen3MLP or nn.modules.module._has_any_global_hook()
+        if (type(x) is not torch.Tensor or x.dim() != 2 or x.shape[0] > K.LINEAR_SMALL_ROWS
+                or type(attn) is not Qwen3Attention or type(mlp) is not Qwen3MLP or nn.modules.module._has_any_global_hook()
                 or _decode_methods() != _DECODE_METHODS):
             return False
         for mod in (n1, n2):
@@ -405,10 +406,10 @@ class Qwen3DecoderLayer(nn.Module):
                                          and residual.shape == x.shape
                                          and residual.dtype == torch.bfloat16):
             return False
-        return (K.linear_small_ok(x) and K.linear_rows_ok(x, qkv.weight)
-                and K.linear_rows_ok(x, gu.weight, swiglu=True)
+        return (K.norms_in_projections_win(x.shape[0], x.shape[1], attn.q_size, gu.weight.shape[0] // 2)
+                and K.linear_rows_ok(x, qkv.weight) and K.linear_rows_ok(x, gu.weight, swiglu=True)
                 and o.weight.dtype == torch.bfloat16 and o.weight.shape[0] == x.shape[1]
-                and o.weight.shape[1] == attn.q_size and attn.q_size in K.LINEAR_SMALL_K)
+                and o.weight.shape[1] == attn.q_size)
 
     def forward_decode(self, x, positions, context_lens, block_tables, slot_mapping=None,
                        residual=None):

@@ -1,0 +1,19 @@
+"""Which decode projections run on the small-batch kernel (CPU: the rule alone)."""
+import torch
+
+
+def test_norms_in_projections(pkg):
+    win = pkg.kernels.norms_in_projections_win
+    # Measured on both sides of the rule: layers of depths (hidden, heads, MLP).
+    for depths, most in (((1024, 2048, 3072), 12), ((2048, 2048, 3072), 10), ((4096, 2048, 4096), 7),
+                         ((1024, 1024, 2048), 16)):
+        assert all(win(rows, *depths) == (rows <= most) for rows in range(1, 20))
+    assert not win(0, 1024, 2048, 3072)
+    # A layer with a depth that the kernel does not have keeps its norms.
+    assert not win(1, 2560, 4096, 9728) and not win(1, 2048, 2048, 6144) and not win(1, 4096, 4096, 12288)
+
+
+def test_single_projections(pkg):
+    win = pkg.kernels.linear_small_wins
+    for k, most in ((1024, 8), (2048, 8), (3072, 2), (4096, 8), (2560, 0)):
+        assert all(win(torch.empty(rows, k)) == (rows <= most) for rows in range(1, 18))
