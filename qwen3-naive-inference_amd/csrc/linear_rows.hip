@@ -312,8 +312,10 @@ Cfg pick(int64_t m, int64_t n, int64_t k, int epi) {
     // tiles 32 rows (two parts) for K <= 2048 and 64 rows (four parts) above
     // — fewer parts also mean fewer partial bytes for the norm that sums them
     // (o_proj / down at 256 rows: 6.4 -> 5.6 / 8.4 -> 7.4 us; at 64 rows
-    // 3.9 -> 3.8 / 4.7 -> 4.4 us).
-    c = n_mt == 2 ? Cfg{16, 4, 1} : (n_mt >= 3 && k > 2048) ? Cfg{64, 3, 1} : Cfg{32, 4, 1};
+    // 3.9 -> 3.8 / 4.7 -> 4.4 us).  Two row tiles of 4,096 columns or more fill the
+    // chip without a split at 32 rows per tile, which read the activations half
+    // as often (K = 12288 at 77 rows: 53 -> 45 us).
+    c = n_mt == 2 && n < 4096 ? Cfg{16, 4, 1} : (n_mt >= 3 && k > 2048) ? Cfg{64, 3, 1} : Cfg{32, 4, 1};
     if (n % c.nt) c = Cfg{16, 4, 1};
     const int64_t tiles = n_mt * (n / c.nt);
     const int64_t want = std::max<int64_t>(1, std::min<int64_t>({256 / tiles, 8, k / kKC}));

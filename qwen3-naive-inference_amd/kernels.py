@@ -726,6 +726,20 @@ PREFILL_LAYER_ARGS = struct.Struct("@44q4f")
 # library's host time.
 PREFILL_LAYER_ROWS = 2048
 PREFILL_LAYER_OUTPUT = 2048 * 6144
+# Wider layers are bound by the products from fewer rows on (us per layer, this
+# form against the modules): hidden 2560 / MLP 9728 at 300 rows 169 : 197, 450 rows
+# 199 : 199, 512 rows 221 : 199; 3072 / 8192 at 300 rows 145 : 197, 640 rows 226 :
+# 206; 4096 / 12288 at 256 rows 203 : 219, 300 rows 234 : 236, 350 rows 258 : 245.
+PREFILL_LAYER_WIDE = 2048
+PREFILL_LAYER_WIDE_ROWS = 300
+
+
+def prefill_layer_size_ok(rows: int, hidden: int, qkv_columns: int, inter: int) -> bool:
+    """Whether a prefill step of this size is one that ``prefill_layer`` is for."""
+    most = PREFILL_LAYER_ROWS if hidden <= PREFILL_LAYER_WIDE else PREFILL_LAYER_WIDE_ROWS
+    return (0 < rows <= most and rows * max(qkv_columns, 2 * inter) <= PREFILL_LAYER_OUTPUT
+            and hidden <= NORM_MAX_WIDTH and hidden % 64 == 0 and inter % 64 == 0
+            and max(qkv_columns, inter) <= 65536)  # 32-bit load offsets
 
 
 def _plain(t: torch.Tensor, dtype: torch.dtype, device: int) -> bool:
@@ -754,9 +768,7 @@ def prefill_layer(x, residual, norms, mats, eps, positions, cos_sin_cache, num_q
     if down_w.dim() != 2 or k_cache.dim() != 4 or cu_seqlens_q.dim() != 1 or block_table.dim() != 2:
         return None
     inter = down_w.shape[1]
-    if not (0 < t <= PREFILL_LAYER_ROWS and t * max(q_n + 2 * kv_n, 2 * inter) <= PREFILL_LAYER_OUTPUT
-            and hidden <= NORM_MAX_WIDTH and hidden % 64 == 0 and inter % 64 == 0
-            and max(q_n + 2 * kv_n, inter) <= 65536  # 32-bit load offsets
+    if not (prefill_layer_size_ok(t, hidden, q_n + 2 * kv_n, inter)
             and num_q_heads in (num_kv_heads, 2 * num_kv_heads, 4 * num_kv_heads)
             and qkv_w.shape == (q_n + 2 * kv_n, hidden) and o_w.shape == (hidden, q_n)
             and gu_w.shape == (2 * inter, hidden) and down_w.shape == (hidden, inter)):

@@ -1,4 +1,5 @@
-"""Which decode projections run on the small-batch kernel (CPU: the rule alone)."""
+"""Which decode projections run on the small-batch kernel, and which prefill steps
+as one call (CPU: the rules alone)."""
 import torch
 
 
@@ -17,3 +18,11 @@ def test_single_projections(pkg):
     win = pkg.kernels.linear_small_wins
     for k, most in ((1024, 8), (2048, 8), (3072, 2), (4096, 8), (2560, 0)):
         assert all(win(torch.empty(rows, k)) == (rows <= most) for rows in range(1, 18))
+
+
+def test_prefill_layer_sizes(pkg):
+    ok = pkg.kernels.prefill_layer_size_ok
+    for hidden, qkv, inter, most in ((1024, 4096, 3072, 2048), (2048, 4096, 6144, 1024),
+                                     (2560, 6144, 9728, 300), (4096, 6144, 12288, 300)):
+        assert ok(1, hidden, qkv, inter) and ok(most, hidden, qkv, inter)
+        assert not ok(most + 1, hidden, qkv, inter) and not ok(0, hidden, qkv, inter)

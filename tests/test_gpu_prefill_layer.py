@@ -204,3 +204,20 @@ def test_layer_under_a_mode(pkg, gpu):
             layer.forward_prefill(*args, residual=r)
     h, i, qkv = cfg.hidden_size, cfg.intermediate_size, 8 * 128
     assert counter.get_total_flops() == 2 * 40 * (h * qkv + 4 * 128 * h + 3 * h * i)
+
+
+# A wide layer runs natively up to 300 rows; 4,096 columns at two row tiles take
+# o_proj and down_proj without a split.
+@pytest.mark.parametrize("hidden,rows", [(2560, 300), (2560, 301), (4096, 77), (4096, 128)])
+def test_wide_layer(pkg, gpu, hidden, rows):
+    layer, cfg = _layer(pkg, gpu, hidden=hidden, heads=8, kv=2, inter=512)
+    args, r = _batch(layer, cfg, gpu, [rows], 0)
+    with torch.no_grad():
+        native = layer._prefill_native(*args, r)
+        assert (native is not None) == (rows <= 300)
+        got = layer.forward_prefill(*args, residual=r)
+        h = layer.mlp.down_proj.register_forward_hook(lambda *_: None)
+        want = layer.forward_prefill(*args, residual=r)
+        h.remove()
+    for a, b in zip(got, want):
+        assert _rel(a, b) < 0.02
