@@ -340,7 +340,10 @@ class Qwen3DecoderLayer(nn.Module):
         sub = self._modules
         attn, mlp = sub.get("self_attn"), sub.get("mlp")
         if (tables is None or type(attn) is not Qwen3Attention or type(mlp) is not Qwen3MLP
-                or attn.k_cache is None or nn.modules.module._has_any_global_hook()
+                or attn.k_cache is None or x.dim() != 2
+                or not K.prefill_layer_size_ok(*x.shape, attn.q_size + 2 * attn.kv_size,
+                                               getattr(mlp._modules.get("down_proj"), "in_features", 0))
+                or nn.modules.module._has_any_global_hook()
                 or torch.is_autocast_enabled("cuda") or _observed()
                 or _prefill_methods() != _PREFILL_METHODS or "_project_store" in attn.__dict__):
             return None

@@ -26,3 +26,20 @@ def test_prefill_layer_sizes(pkg):
                                      (2560, 6144, 9728, 300), (4096, 6144, 12288, 300)):
         assert ok(1, hidden, qkv, inter) and ok(most, hidden, qkv, inter)
         assert not ok(most + 1, hidden, qkv, inter) and not ok(0, hidden, qkv, inter)
+
+
+def test_large_steps_skip_the_module_checks(pkg, monkeypatch):
+    """A step that a fused form is not for pays for no look at its modules."""
+    layer = pkg.Qwen3DecoderLayer(pkg.Qwen3Config(
+        hidden_size=64, num_attention_heads=2, num_key_value_heads=1, intermediate_size=64,
+        num_hidden_layers=1, max_position_embeddings=64))
+    layer.self_attn.k_cache = torch.zeros(1)
+
+    def look(*_):
+        raise AssertionError("modules looked at")
+
+    monkeypatch.setattr(pkg.qwen3_naive, "_prefill_methods", look)
+    monkeypatch.setattr(pkg.qwen3_naive, "_decode_methods", look)
+    x = torch.empty(2049, 64)
+    assert layer._prefill_native(x, *[None] * 6, x, None) is None
+    assert not layer._norms_in_projections(x, None)
