@@ -32,9 +32,14 @@ def kernels_ok(*tensors: torch.Tensor) -> bool:
     for t in tensors:
         if (type(t) not in (torch.Tensor, torch.nn.Parameter) or t.dtype != BF16 or t.device != dev):
             return False
-    return not (torch.compiler.is_compiling() or torch.jit.is_tracing()
+    return not (torch.compiler.is_compiling() or torch.jit.is_tracing() or _make_fx()
                 or torch.is_autocast_enabled("cuda") or any(map(_has_tangent, tensors))
                 or torch._C._functorch.peek_interpreter_stack() is not None)
+
+
+def _make_fx() -> bool:
+    """Whether ops are being recorded into a graph that would not hold the kernels."""
+    return torch._C._get_dispatch_mode(torch._C._TorchDispatchModeKey.PROXY) is not None
 
 
 def _has_tangent(t: torch.Tensor) -> bool:

@@ -345,3 +345,19 @@ def test_second_derivative_after_a_weight_was_written(pkg, T, gpu, written):
         # Partial gradients are each rounded to bf16 before they are added (2^-8),
         # at both levels.
         assert all(_rel(a, b) < 2 ** -6 for a, b in zip(*out))
+
+
+def test_traced_layer_holds_its_ops(pkg, gpu):
+    """A graph recorded from the layer and its gradient computes them for other inputs."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    layer = _layer(pkg, gpu)
+
+    def step(x):
+        x = x.detach().requires_grad_()
+        y = layer(x)
+        return y, torch.autograd.grad(y.float().square().sum(), x)[0]
+
+    a, b = (torch.randn(1, 9, 128, device=gpu).bfloat16() for _ in range(2))
+    graph = make_fx(step)(a)
+    for got, want in zip(graph(b), step(b)):
+        assert _rel(got, want) < 2 ** -7
