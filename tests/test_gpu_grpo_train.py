@@ -123,3 +123,15 @@ def test_shifted_loss_gradient(pkg, gpu, t):
     gb, = torch.autograd.grad(b[0], logits)
     assert all(torch.equal(x, y) for x, y in zip(a, b))
     assert gb.abs().max() > 0 and torch.equal(ga, gb) and bool((ga[:, -1] == 0).all())
+
+
+def test_shifted_loss_of_one_position(pkg, gpu):
+    """No position has a next token: refused, as the empty slices are."""
+    logits = torch.randn(2, 1, 100, device=gpu).bfloat16().requires_grad_()
+    ids = torch.zeros(2, 1, dtype=torch.int64, device=gpu)
+    old, mask = torch.zeros(2, 1, device=gpu), torch.ones(2, 1, device=gpu)
+    rewards, groups = torch.rand(2, device=gpu), torch.zeros(2, dtype=torch.int64, device=gpu)
+    for args, shift in (((logits, ids, old, mask), True),
+                        ((logits[:, :-1], ids[:, 1:], old[:, 1:], mask[:, 1:]), False)):
+        with pytest.raises(pkg._lib.QmiError):
+            pkg.grpo_fused_loss(*args, rewards, groups, shift=shift)

@@ -46,6 +46,31 @@ def test_linear_small(pkg, gpu, m, n, k, swiglu):
     assert torch.equal(s, total) and _rel(y, ref(h)) < 2 * tol
 
 
+# Eight weight rows per workgroup: the fewest columns that take them, and a count
+# past whole multiples of the chip.  Each element by itself: one rounding (2^-8)
+# after k terms summed in fp32, here and in the reference (2^-23 k of the terms'
+# magnitudes); with the norm, rows whose elements may have rounded the other way
+# (2^-8 of a term each, 2^-8 of their root sum of squares on average, 8 times that
+# over all elements).
+@pytest.mark.parametrize("m", [1, 9, 16])
+@pytest.mark.parametrize("n", [2048, 3088])
+@pytest.mark.parametrize("k", [1024, 2048, 3072, 4096])
+def test_linear_small_eight_rows(pkg, gpu, m, n, k):
+    K = pkg.kernels
+    g = torch.Generator(device=gpu).manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device=gpu).bfloat16()
+    r = torch.randn(m, k, generator=g, device=gpu).bfloat16()
+    w = (torch.randn(n, k, generator=g, device=gpu) * 0.05).bfloat16()
+    nw = torch.rand(k, generator=g, device=gpu).bfloat16() + 0.5
+    for rows, args in ((x, ()), (K.rms_norm(x, nw, 1e-6), (nw, 1e-6)),
+                       (K.add_rms_norm(x, r, nw, 1e-6)[0], (nw, 1e-6, r))):
+        want = rows.float() @ w.float().T
+        bound = 2 ** -8 * want.abs() + 2 ** -23 * k * (rows.float().abs() @ w.float().abs().T)
+        if args:
+            bound = bound + 2 ** -5 * (rows.float().square() @ w.float().square().T).sqrt()
+        assert bool(((K.linear_small(x, w, False, *args)[0].float() - want).abs() <= bound).all())
+
+
 def test_linear_small_refuses(pkg, gpu):
     K = pkg.kernels
     x = torch.zeros(17, 1024, device=gpu).bfloat16()

@@ -37,6 +37,37 @@ def test_linear_tiles(pkg, gpu, m, n, k, swiglu):
     assert torch.equal(y[:m], pkg.kernels.linear_tiles(x, w, swiglu))
 
 
+# The two 192-column forms (ring of three and of two chunks) with partial last
+# tiles both ways, at K of fewer chunks than the ring, as many and more; each
+# element by itself: one rounding (2^-8 of it) after k terms summed in fp32, in
+# the product and its reference (2^-23 k of the terms' magnitudes), and for SwiGLU
+# the roundings of gate (silu changes by at most 1 + |g| times its relative
+# error), up and the result.
+@pytest.mark.parametrize("m", [1000, 1999])
+@pytest.mark.parametrize("n,swiglu", [(6128, False), (3056, True)])
+@pytest.mark.parametrize("k", [64, 128, 192, 1024])
+def test_linear_tiles_wide_forms(pkg, gpu, m, n, swiglu, k):
+    g = torch.Generator(device=gpu).manual_seed(m + k)
+    x = torch.randn(m, k, generator=g, device=gpu).bfloat16()
+    w = (torch.randn((2 * n if swiglu else n), k, generator=g, device=gpu) * 0.05).bfloat16()
+    y = torch.full((m + 1, n), 7.0, device=gpu).bfloat16()
+    st = pkg._lib.lib().qmi_linear_tiles(x.data_ptr(), k, w.data_ptr(), k, m, n, k, int(swiglu),
+                                         y.data_ptr(), n, pkg._lib.stream_handle(x.device))
+    assert st == 0
+    want = x.float() @ w.float().T
+    slack = 2 ** -23 * k * (x.float().abs() @ w.float().abs().T)
+    bound = 2 ** -8 * want.abs() + slack
+    if swiglu:
+        gate, up = want.chunk(2, -1)
+        sg, su = slack.chunk(2, -1)
+        silu = torch.nn.functional.silu(gate)
+        want = silu * up
+        bound = 2 ** -8 * want.abs() * (3 + gate.abs()) + 1.1 * sg * up.abs() + su * silu.abs()
+        bound = 1.02 * bound + 1e-6  # products of the errors; __expf
+    assert bool(((y[:m].float() - want).abs() <= bound).all())
+    assert bool((y[m] == 7).all())
+
+
 def test_linear_tiles_strides(pkg, gpu):
     x = torch.randn(70, 200, device=gpu).bfloat16()[:, 8:136]
     w = torch.randn(48, 160, device=gpu).bfloat16()[:, :128]
@@ -218,6 +249,22 @@ def test_wide_layer(pkg, gpu, hidden, rows):
         got = layer.forward_prefill(*args, residual=r)
         h = layer.mlp.down_proj.register_forward_hook(lambda *_: None)
         want = layer.forward_prefill(*args, residual=r)
+        h.remove()
+    for a, b in zip(got, want):
+        assert _rel(a, b) < 0.02
+
+
+@pytest.mark.parametrize("heads,kv", [(2, 2), (8, 2)])
+def test_layer_head_ratios(pkg, gpu, heads, kv):
+    """One and four query heads per KV head, over a cached prefix."""
+    layer, cfg = _layer(pkg, gpu, heads=heads, kv=kv)
+    args, r = _batch(layer, cfg, gpu, [3, 200], 77)
+    cache = layer.self_attn.k_cache.clone()
+    with torch.no_grad():
+        got = (*layer._prefill_native(*args, r), layer.self_attn.k_cache.clone())
+        layer.self_attn.k_cache.copy_(cache)
+        h = layer.mlp.down_proj.register_forward_hook(lambda *_: None)
+        want = (*layer.forward_prefill(*args, residual=r), layer.self_attn.k_cache)
         h.remove()
     for a, b in zip(got, want):
         assert _rel(a, b) < 0.02

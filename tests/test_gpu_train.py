@@ -361,3 +361,23 @@ def test_traced_layer_holds_its_ops(pkg, gpu):
     graph = make_fx(step)(a)
     for got, want in zip(graph(b), step(b)):
         assert _rel(got, want) < 2 ** -7
+
+
+# Five to eight chunks of the fused softmax (its form for 257 to 512 tokens).
+@pytest.mark.parametrize("t", [257, 389, 512])
+@pytest.mark.parametrize("hq,hkv", [(2, 2), (4, 2), (8, 2)])
+def test_attention_eight_chunks(pkg, T, gpu, t, hq, hkv):
+    test_attention(pkg, T, gpu, 2, t, hq, hkv)
+
+
+def test_layer_on_a_side_stream(pkg, gpu):
+    """Forward and backward on another stream than the default one."""
+    layer = _layer(pkg, gpu)
+    x = torch.randn(2, 33, 128, device=gpu).bfloat16().requires_grad_()
+    want = _grads(layer, layer(x), x)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        got = _grads(layer, layer(x), x)
+    torch.cuda.current_stream().wait_stream(side)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
