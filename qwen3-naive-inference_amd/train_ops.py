@@ -11,6 +11,8 @@ of gradients (vmap) goes through the formula.
 """
 from __future__ import annotations
 
+import functools
+
 import torch
 from torch.autograd import forward_ad
 
@@ -75,6 +77,18 @@ def _linked(t: torch.Tensor, copy: torch.Tensor, version: int) -> torch.Tensor:
     return t if t._version == version else copy + (t - t.detach())
 
 
+def _no_autocast(backward):
+    """A backward without autocast, as its forward ran: under it the products of
+    fp32 tensors, which the kernels read, would come out in 16 bits."""
+    @functools.wraps(backward)
+    def run(ctx, *grads):
+        if not torch.is_autocast_enabled("cuda"):
+            return backward(ctx, *grads)
+        with torch.autocast("cuda", enabled=False):
+            return backward(ctx, *grads)
+    return run
+
+
 def _call(name, device, *args):
     # Some 45 launches a training step: the raw handle of the current stream, 5 us
     # less each than through a Stream object.
@@ -135,6 +149,7 @@ class RmsNorm(torch.autograd.Function):
         return y
 
     @staticmethod
+    @_no_autocast
     def backward(ctx, dy):
         x, weight, mean = ctx.saved_tensors
         need = ctx.needs_input_grad
@@ -178,6 +193,7 @@ class SiluMul(torch.autograd.Function):
         return y
 
     @staticmethod
+    @_no_autocast
     def backward(ctx, dy):
         gate_up, = ctx.saved_tensors
         if _formula_backward(dy, gate_up):
@@ -295,6 +311,7 @@ class QkvAttention(torch.autograd.Function):
         return out
 
     @staticmethod
+    @_no_autocast
     def backward(ctx, dout):
         qkv, weights, cache, q_mean, k_mean, qf, kt, vf, w = ctx.saved_tensors
         hq, hkv, eps, scale = ctx.args

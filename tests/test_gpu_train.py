@@ -381,3 +381,15 @@ def test_layer_on_a_side_stream(pkg, gpu):
         got = _grads(layer, layer(x), x)
     torch.cuda.current_stream().wait_stream(side)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_backward_under_autocast(pkg, T, gpu):
+    """Autocast around the backward alone changes nothing."""
+    for fused, _, inputs in _functions(pkg, T, gpu):
+        out = []
+        for on in (False, True):
+            leaves = [t.detach().clone().requires_grad_() for t in inputs]
+            y = fused(*leaves)
+            with torch.autocast("cuda", dtype=torch.bfloat16, enabled=on):
+                out.append(torch.autograd.grad(y, leaves, torch.ones_like(y)))
+        assert all(torch.equal(a, b) for a, b in zip(*out))

@@ -36,6 +36,23 @@ def test_prefill_layer_takes_plain_tensors_only(pkg):
     assert not ok(Wrapper(t), torch.bfloat16, -1)
 
 
+def _backward(T, name):
+    """Runs a Function's backward on CPU tensors; its launches are the caller's to replace."""
+    b16 = torch.bfloat16
+    x, w = torch.zeros(1, 5, 512, dtype=b16), torch.zeros(512, dtype=b16)
+    f = torch.zeros(2, 5, 128)
+    cls, saved, out, args = {
+        "norm": (T.RmsNorm, (x, w, torch.zeros(1, 5, 1)), x.shape, {"eps": 1e-6}),
+        "silu": (T.SiluMul, (x,), (1, 5, 256), {}),
+        "attention": (T.QkvAttention, (x, w[:256].view(2, 128), torch.zeros(5, 128), torch.zeros(1, 5, 2, 1),
+                                       torch.zeros(1, 5, 1, 1), f, f.transpose(1, 2).contiguous(), f,
+                                       torch.zeros(2, 5, 5)), (1, 5, 256), {"args": (2, 1, 1e-6, 0.1)}),
+    }[name]
+    ctx = types.SimpleNamespace(saved_tensors=saved, needs_input_grad=(True,) * 3, **args)
+    with torch.no_grad():
+        cls.backward(ctx, torch.zeros((), dtype=b16).expand(out))
+
+
 @pytest.mark.parametrize("name", ["norm", "silu", "attention"])
 def test_backward_keeps_its_copies_until_the_launch(pkg, monkeypatch, name):
     """A copy made to be dense is alive when a kernel that gets its address is
@@ -56,20 +73,25 @@ def test_backward_keeps_its_copies_until_the_launch(pkg, monkeypatch, name):
 
     monkeypatch.setattr(pkg.kernels, "_dense16", copy)
     monkeypatch.setattr(T, "_call", call)
-    b16 = torch.bfloat16
-    x, w = torch.zeros(1, 5, 512, dtype=b16), torch.zeros(512, dtype=b16)
-    f = torch.zeros(2, 5, 128)
-    cls, saved, out, args = {
-        "norm": (T.RmsNorm, (x, w, torch.zeros(1, 5, 1)), x.shape, {"eps": 1e-6}),
-        "silu": (T.SiluMul, (x,), (1, 5, 256), {}),
-        "attention": (T.QkvAttention, (x, w[:256].view(2, 128), torch.zeros(5, 128), torch.zeros(1, 5, 2, 1),
-                                       torch.zeros(1, 5, 1, 1), f, f.transpose(1, 2).contiguous(), f,
-                                       torch.zeros(2, 5, 5)), (1, 5, 256), {"args": (2, 1, 1e-6, 0.1)}),
-    }[name]
-    ctx = types.SimpleNamespace(saved_tensors=saved, needs_input_grad=(True,) * 3, **args)
-    with torch.no_grad():
-        cls.backward(ctx, torch.zeros((), dtype=b16).expand(out))
+    _backward(T, name)
     assert passed
+
+
+@pytest.mark.parametrize("name", ["norm", "silu", "attention"])
+def test_backward_runs_without_autocast(pkg, monkeypatch, name):
+    """Autocast around a backward alone (its forward ran without) must not reach
+    the fp32 products whose addresses the kernels get: in 16 bits they are half
+    as long."""
+    T = importlib.import_module(pkg.__name__ + ".train_ops")
+    seen = []
+    monkeypatch.setattr(T, "_call", lambda *_: seen.append(torch.is_autocast_enabled("cuda")))
+    torch.set_autocast_enabled("cuda", True)
+    try:
+        _backward(T, name)
+        assert torch.is_autocast_enabled("cuda")
+    finally:
+        torch.set_autocast_enabled("cuda", False)
+    assert seen and not any(seen)
 
 
 def test_replaced_rotation_is_used(pkg, monkeypatch):
