@@ -21,6 +21,8 @@ from ._lib import check, lib
 
 HEAD_DIM = K.HEAD_DIM
 F32, BF16 = torch.float32, torch.bfloat16
+_current_device = torch._C._cuda_getDevice
+_raw_stream = torch._C._cuda_getCurrentRawStream
 
 
 def kernels_ok(*tensors: torch.Tensor) -> bool:
@@ -90,9 +92,14 @@ def _no_autocast(backward):
 
 
 def _call(name, device, *args):
+    """Launches on the device's current stream, also where another device is current
+    (a torch op changes to its tensors' device by itself)."""
+    if _current_device() != device.index:
+        with torch.cuda.device(device):
+            return _call(name, device, *args)
     # Some 45 launches a training step: the raw handle of the current stream, 5 us
     # less each than through a Stream object.
-    check(getattr(lib(), name)(*args, torch._C._cuda_getCurrentRawStream(device.index)), name)
+    check(getattr(lib(), name)(*args, _raw_stream(device.index)), name)
 
 
 # ---------------------------------------------------------------------------

@@ -94,6 +94,31 @@ def test_backward_runs_without_autocast(pkg, monkeypatch, name):
     assert seen and not any(seen)
 
 
+def test_launch_on_the_tensors_device(pkg, monkeypatch):
+    """A training batch on another GPU than the current one is launched there."""
+    T = importlib.import_module(pkg.__name__ + ".train_ops")
+    current, launched = [0], []
+
+    class Device:
+        def __init__(self, device):
+            self.index = device.index
+
+        def __enter__(self):
+            current.append(self.index)
+
+        def __exit__(self, *_):
+            current.pop()
+
+    entry = types.SimpleNamespace(f=lambda *args: launched.append((current[-1], *args)) or 0)
+    monkeypatch.setattr(T, "lib", lambda: entry)
+    monkeypatch.setattr(T, "_current_device", lambda: current[-1])
+    monkeypatch.setattr(T, "_raw_stream", lambda index: 100 + index)
+    monkeypatch.setattr(torch.cuda, "device", Device)
+    T._call("f", torch.device("cuda", 0), 7)
+    T._call("f", torch.device("cuda", 1), 8)
+    assert launched == [(0, 7, 100), (1, 8, 101)] and current == [0]
+
+
 def test_replaced_rotation_is_used(pkg, monkeypatch):
     """A program's own RoPE, set on RotaryEmbedding, is the batch forward's."""
     torch.manual_seed(0)
