@@ -633,10 +633,10 @@ LINEAR_SMALL_K = (1024, 2048, 3072, 4096)
 # cost more than as partial products (3072 -> 1024 at 12 rows 6.0 us against
 # 4.1).  Layer with its depths (hidden, heads, MLP) and 1 / largest / next
 # row count, us, against norms and linear_rows: (1024, 2048, 3072) 43.1 : 48.5 /
-# 12 rows 49.5 : 51.3 / 16 rows 52.3 : 50.9; (2048, 2048, 3072) 54.6 : 61.4 / 10
-# rows 63.1 : 63.3 / 14 rows 67.7 : 64.1; (4096, 2048, 4096) 73.6 : 83.7 / 6 rows
-# 81.3 : 83.2 / 10 rows 92.3 : 84.0.
-LINEAR_SMALL_CHAIN = 72 * 1024
+# 14 rows 51.6 : 52.3 / 16 rows 52.3 : 50.9; (2048, 2048, 3072) 54.6 : 61.4 / 12
+# rows 63.5 : 63.9 / 14 rows 67.7 : 64.1; (4096, 2048, 4096) 73.6 : 83.7 / 8 rows
+# 82.7 : 83.2 / 10 rows 92.3 : 84.0.
+LINEAR_SMALL_CHAIN = 84 * 1024
 # One projection whose rows are there already, by depth: up to this many rows it
 # is faster than linear_rows, which reads the rows once per weight tile of twice
 # the height (1024 -> 2 x 3072 at 8 rows 6.1 us against 6.7, 16 rows 7.0 : 6.7;
