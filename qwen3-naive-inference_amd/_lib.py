@@ -166,5 +166,8 @@ def check(status: int, what: str) -> None:
 
 
 def stream_handle(device: torch.device | None = None) -> int:
-    """Raw hipStream_t of torch's current stream on ``device``."""
-    return torch.cuda.current_stream(device).cuda_stream
+    """Raw hipStream_t of torch's current stream on ``device`` (of a tensor, so that
+    the GPU is initialised; without a Stream object, which takes 5 us to make)."""
+    if device is None or device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)

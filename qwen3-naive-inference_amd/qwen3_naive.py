@@ -434,9 +434,9 @@ class Qwen3DecoderLayer(nn.Module):
 def _observed() -> bool:
     """Whether a dispatch or function mode (a FLOP counter, a tracer; a default
     device aside) is there to see the torch ops of a call."""
-    return torch._C._len_torch_dispatch_stack() > 0 or any(
-        type(torch._C._get_function_stack_at(i)) is not DeviceContext
-        for i in range(torch._C._len_torch_function_stack()))
+    n = torch._C._len_torch_function_stack()
+    return torch._C._len_torch_dispatch_stack() > 0 or n > 0 and any(
+        type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(n))
 
 
 def _prefill_methods():

@@ -17,12 +17,11 @@ import torch
 from torch.autograd import forward_ad
 
 from . import kernels as K
-from ._lib import check, lib
+from ._lib import check, lib, stream_handle
 
 HEAD_DIM = K.HEAD_DIM
 F32, BF16 = torch.float32, torch.bfloat16
 _current_device = torch._C._cuda_getDevice
-_raw_stream = torch._C._cuda_getCurrentRawStream
 
 
 def kernels_ok(*tensors: torch.Tensor) -> bool:
@@ -97,9 +96,7 @@ def _call(name, device, *args):
     if _current_device() != device.index:
         with torch.cuda.device(device):
             return _call(name, device, *args)
-    # Some 45 launches a training step: the raw handle of the current stream, 5 us
-    # less each than through a Stream object.
-    check(getattr(lib(), name)(*args, _raw_stream(device.index)), name)
+    check(getattr(lib(), name)(*args, stream_handle(device)), name)
 
 
 # ---------------------------------------------------------------------------

@@ -112,7 +112,7 @@ def test_launch_on_the_tensors_device(pkg, monkeypatch):
     entry = types.SimpleNamespace(f=lambda *args: launched.append((current[-1], *args)) or 0)
     monkeypatch.setattr(T, "lib", lambda: entry)
     monkeypatch.setattr(T, "_current_device", lambda: current[-1])
-    monkeypatch.setattr(T, "_raw_stream", lambda index: 100 + index)
+    monkeypatch.setattr(T, "stream_handle", lambda device: 100 + device.index)
     monkeypatch.setattr(torch.cuda, "device", Device)
     T._call("f", torch.device("cuda", 0), 7)
     T._call("f", torch.device("cuda", 1), 8)
