@@ -1,7 +1,8 @@
 """The training batch's fused autograd Functions against the torch formulas
 they stand for.  Forward values and the gradients that flow on are the same
-bit for bit; the norm weights' gradients, summed in another order, agree to
-one bf16 rounding (half an ulp of 8 significant bits, 2^-8)."""
+bit for bit, but where a sum has another order: the norm weights' gradients, and
+k's and v's over four query heads per KV head, agree to one bf16 rounding (half
+an ulp of 8 significant bits, 2^-8)."""
 import importlib
 
 import pytest
@@ -78,8 +79,8 @@ def test_attention(pkg, T, gpu, b, t, hq, hkv):
 
 
 def test_layer_routes(pkg, T, gpu):
-    """The layer takes the fused Functions, unless a norm is hooked or a
-    function transform or a second derivative needs torch ops; same values."""
+    """The layer takes the fused Functions, unless a norm is hooked or a second
+    derivative needs torch ops; same values."""
     torch.manual_seed(0)
     layer = pkg.Qwen3DecoderLayer(pkg.Qwen3Config(
         hidden_size=128, num_attention_heads=2, num_key_value_heads=1, intermediate_size=256,
@@ -393,3 +394,15 @@ def test_backward_under_autocast(pkg, T, gpu):
             with torch.autocast("cuda", dtype=torch.bfloat16, enabled=on):
                 out.append(torch.autograd.grad(y, leaves, torch.ones_like(y)))
         assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
+def test_function_transforms(pkg, gpu):
+    """torch.func's grad and vmap run on torch ops."""
+    layer = _layer(pkg, gpu)
+    x = torch.randn(1, 9, 128, device=gpu).bfloat16()
+    leaf = x.clone().requires_grad_()
+    want = _grads(layer, layer(leaf), leaf)[0]
+    # The products run in other forms there: flipped bf16 roundings along the layer's steps.
+    assert _rel(torch.func.grad(lambda z: layer(z).float().square().mean())(x), want) < 0.02
+    norm = layer.input_layernorm
+    assert torch.equal(torch.func.vmap(norm)(x[0]), norm(leaf)[0])
