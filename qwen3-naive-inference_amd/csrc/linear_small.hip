@@ -11,19 +11,23 @@
 // latency: the launch, one trip to HBM for the weights, the epilogue.  So:
 //   * One trip.  Workgroup = 8 waves = 16 weight rows; wave w takes an eighth
 //     of K and loads its whole share of the weight rows straight into the
-//     MFMA A registers before anything else (32 KB per workgroup at K = 1024).
-//   * The norm is computed by every workgroup while those loads are in flight
+//     MFMA A registers (32 KB per workgroup at K = 1024), right after the few
+//     rows that the norm waits for: loads return in order.
+//   * The norm is computed by every workgroup while the weights are in flight
 //     (16 KB of rows from L2 at 4 sequences), so the separate norm launch and
 //     its gap go away; its output, the B operand, stays in LDS (16-byte chunks
 //     XOR-swizzled by the row).  Row r's residual sum is written by workgroup
-//     r (modulo the grid).  Above 16 rows the rows' re-reads by every
-//     workgroup cost more than the launch.
+//     r (modulo the grid).  Every workgroup reads the rows anew, which costs
+//     more than the launch from some rows x depth on; the callers' rules say
+//     where (hidden 1024: 14 rows of 16).
 //   * The 8 partial tiles are added in wave order through LDS: no split-K
 //     partials in memory, so the next norm reads bf16 rows.
 //   * SwiGLU (packed [gate; up] weight): 8 gate rows and their 8 up rows.
 //
-// Eight layers, 4 sequences of 37-700 tokens, as a graph: 324 -> 274 us (the
-// rows' loads behind the weights', which return in order: 307).
+// Eight layers, 4 sequences of 37-700 tokens, as a graph: 324 -> 307 us with
+// the weights' loads before the rows'; 279 with the rows' first, four weight rows
+// per workgroup in o_proj / down_proj and 32-bit divisions in the attention's
+// schedule; 274 with the attention merge's loads four at a time.
 #include "qmi_common.h"
 
 namespace {

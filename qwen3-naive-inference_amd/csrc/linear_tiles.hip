@@ -211,9 +211,10 @@ void launch(const uint16_t* x, int64_t x_stride, const uint16_t* w, int64_t w_st
 }
 
 // Tile forms with the time one 64-element K chunk takes on an MI355X (ns, all
-// CUs busy; weights from HBM, qkv / gate_up / o / down of hidden 1024): a CU
-// receives 35-60 GB/s whatever is in flight, so a chunk's time follows its
-// (BM + BN) rows and a form's merit is the bytes per CU that its tiles and
+// CUs busy; weights from HBM, qkv / gate_up / o / down of hidden 1024): here a CU
+// receives 35-60 GB/s however deep the ring is (loads alone reach 80-147 GB/s
+// per CU; what keeps this kernel below that is not known), so a chunk's time
+// follows its (BM + BN) rows and a form's merit is the bytes per CU that its tiles and
 // their last, partly filled round give.  F(BM, BN, WM, WN, NSTAGE, ns).
 #define QMI_LT_FORMS(F)        \
   F(64, 64, 2, 2, 4, 360)   \

@@ -3,20 +3,22 @@
 //
 // Reference semantics: the batch forward of RMSNorm, Qwen3MLP and
 // Qwen3Attention (qwen3_naive.py:156-169, :553-590, :695-702) and its
-// gradients, as torch's formulas compute them.  These kernels give the
-// formulas' values bit for bit: the same fp32 operations in the same
-// grouping, the same roundings to bf16 in between, no contraction to FMA (the
-// file is built with -ffp-contract=off).  Sums along a row (mean of squares,
-// softmax, the norm's row gradient) and products stay with torch, whose
-// summation order they share; the weights' gradients, which nothing reads
-// again, are summed here in a fixed order.
+// gradients, as torch's formulas compute them.  These kernels repeat the
+// formulas: the same fp32 operations in the same grouping, the same roundings
+// to bf16 in between, no contraction to FMA but the ones named (the file is
+// built with -ffp-contract=off).  The norms' sums along a row (mean of squares,
+// the row's gradient) and the products stay with torch; the softmax of rows of
+// up to 1,024 adds in torch's order.  So values are torch's bits, except where
+// a sum has another, fixed order: the norm weights' gradients, and k's and v's
+// gradients summed over four or more query heads per KV head.
 //
 // What bounds them is memory: a norm forward moved its fp32 rows through
 // memory 9 times in 9 launches and backward ~20 times, the scores took 3
 // passes per direction outside the softmax.  All are one 8-element item per
 // lane with 16- or 32-byte accesses.  One decoder layer forward + backward, 8 x
-// 640 tokens of hidden 1024: 4,020 -> 2,000 us (900 of them fp32 products); a
-// two-layer training step, 2 x 389 tokens: 5,300-5,900 -> 2,870 us.
+// 640 tokens of hidden 1024: 4,000 -> 1,985-2,100 us (850 of them fp32
+// products); a two-layer training step, 2 x 389 tokens: 5,400-5,600 -> 2,890-
+// 2,940 us.
 #include <algorithm>
 
 #include "qmi_common.h"

@@ -1,10 +1,13 @@
 """The training batch's element-wise chains as autograd Functions on fused
 HIP kernels (csrc/train_rows.hip).
 
-Each gives the values of the torch formula beside it, in both directions: the
-kernels repeat its fp32 operations and bf16 roundings, sums along a row, the
-softmax and the products are the same torch calls on the same operands.  Only
-the norm weights' gradients are summed in another (fixed) order.  The formula
+Each follows the torch formula beside it in both directions: the kernels
+repeat its fp32 operations and bf16 roundings, and sums along a norm's row and
+the products are the same torch calls on the same operands.  The softmax and
+its gradient are own kernels that add in torch's order up to 1,024 columns and
+torch calls above.  The values are the formula's, bit for bit, but for sums in
+another fixed order: the norm weights' gradients, and from four query heads per
+KV head on the sums of k's and v's gradients over those heads.  The formula
 serves every call the kernels do not take, and a backward that is
 differentiated itself (``create_graph=True``, forward mode) or runs on a batch
 of gradients (vmap) goes through the formula.
