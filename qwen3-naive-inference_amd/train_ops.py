@@ -36,7 +36,8 @@ def kernels_ok(*tensors: torch.Tensor) -> bool:
     if dev.type != "cuda" or not (torch.is_grad_enabled() and tensors[0].requires_grad):
         return False
     for t in tensors:
-        if (type(t) not in (torch.Tensor, torch.nn.Parameter) or t.dtype != BF16 or t.device != dev):
+        if (type(t) not in (torch.Tensor, torch.nn.Parameter) or t.dtype != BF16 or t.device != dev
+                or t.is_inference()):  # no version, not saved for a backward
             return False
     return not (torch.compiler.is_compiling() or torch.jit.is_tracing() or _make_fx()
                 or torch.is_autocast_enabled("cuda") or any(map(_has_tangent, tensors))

@@ -406,3 +406,14 @@ def test_function_transforms(pkg, gpu):
     assert _rel(torch.func.grad(lambda z: layer(z).float().square().mean())(x), want) < 0.02
     norm = layer.input_layernorm
     assert torch.equal(torch.func.vmap(norm)(x[0]), norm(leaf)[0])
+
+
+def test_norm_weight_made_in_inference_mode(pkg, gpu):
+    """Such a weight cannot be saved for a backward; the formula saves a copy."""
+    norm = pkg.qwen3_naive.RMSNorm(128).to(gpu).bfloat16()
+    x = torch.randn(3, 128, device=gpu).bfloat16().requires_grad_()
+    norm.requires_grad_(False)
+    want = torch.autograd.grad(norm(x).float().square().sum(), x)[0]
+    with torch.inference_mode():
+        norm.weight = torch.nn.Parameter(norm.weight.clone(), requires_grad=False)
+    assert torch.equal(torch.autograd.grad(norm(x).float().square().sum(), x)[0], want)
