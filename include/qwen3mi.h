@@ -442,7 +442,8 @@ int qmi_prefill_layer(const qmi_prefill_layer_args* args, void* stream);
  * of the torch formulas.  Rows: `heads` adjacent rows of n elements (n % 8 ==
  * 0, <= 65536) in each bf16 row of `stride`; fp32 arrays and dy are
  * contiguous.  Pointers 16-byte aligned.
- *   square_rows:  sq = x^2 (its row means are `mean` below)
+ *   square_rows:  sq = x^2 (its row means are `mean` below); x_copy (or NULL): the
+ *                 rows as they were read, contiguous; zero (or NULL): 0.0f
  *   norm_apply:   y = bf16(x * rsqrt(mean + eps) * w), heads = 1, y contiguous;
  *                 w_copy (or NULL): w as it was read
  *   norm_prod:    prod = (dy * w) * x, whose row sums are `dr` below
@@ -467,7 +468,7 @@ int qmi_prefill_layer(const qmi_prefill_layer_args* args, void* stream);
  * No output overlaps an input.
  */
 int qmi_square_rows(const uint16_t* x, int64_t rows, int64_t stride, int64_t heads, int64_t n,
-                    float* sq, void* stream);
+                    float* sq, uint16_t* x_copy, float* zero, void* stream);
 int qmi_norm_apply(const uint16_t* x, int64_t rows, int64_t stride, int64_t n, const float* mean,
                    const uint16_t* w, float eps, uint16_t* y, uint16_t* w_copy, void* stream);
 int qmi_norm_prod(const uint16_t* x, int64_t rows, int64_t stride, int64_t heads, int64_t n,

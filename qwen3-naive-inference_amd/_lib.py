@@ -92,7 +92,7 @@ SIGNATURES: dict[str, tuple] = {
     "qmi_prefill_layer_workspace_bytes": (_c_i64, [_c_i64] * 6),
     # The argument struct as bytes (kernels.PREFILL_LAYER_ARGS).
     "qmi_prefill_layer": (ctypes.c_int, [ctypes.c_char_p, _c_p]),
-    "qmi_square_rows": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p]),
+    "qmi_square_rows": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_p]),
     "qmi_norm_apply": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_f32, _c_p, _c_p,
                                       _c_p]),
     "qmi_norm_prod": (ctypes.c_int, [_c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_p]),

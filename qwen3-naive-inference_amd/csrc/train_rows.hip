@@ -85,13 +85,18 @@ struct Rows {
 };
 
 __global__ __launch_bounds__(kThreads) void square_kernel(const uint16_t* __restrict__ x, Rows d,
-                                                          float* __restrict__ sq) {
+                                                          float* __restrict__ sq,
+                                                          uint16_t* __restrict__ x_copy,
+                                                          float* __restrict__ zero) {
   const int n8 = d.n / 8;
   const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (zero && i == 0) *zero = 0.f;
   if (i >= d.rows * n8) return;
   const uint32_t row = (uint32_t)i / (uint32_t)n8;
   const int col = (int)((uint32_t)i % (uint32_t)n8) * 8;
-  V8 a = load8(x + d.at(row, col));
+  const uint4 raw = load_u4(x + d.at(row, col));
+  if (x_copy) *reinterpret_cast<uint4*>(x_copy + 8 * i) = raw;
+  V8 a = unpack8(raw);
 #pragma unroll
   for (int e = 0; e < 8; ++e) a.v[e] = a.v[e] * a.v[e];
   store8f(sq + 8 * i, a);
@@ -562,13 +567,13 @@ int check_heads(int64_t batch, int64_t t, int64_t hq, int64_t hkv) {
 #define QMI_ST reinterpret_cast<hipStream_t>(stream)
 
 extern "C" int qmi_square_rows(const uint16_t* x, int64_t rows, int64_t stride, int64_t heads, int64_t n,
-                               float* sq, void* stream) {
+                               float* sq, uint16_t* x_copy, float* zero, void* stream) {
   const int e = check_rows(rows, stride, heads, n);
   if (e != QMI_OK) return e;
   if (!x || !sq) return QMI_E_NULL_POINTER;
-  if (!al16(x) || !al16(sq)) return QMI_E_BAD_STRIDE;
+  if (!al16(x) || !al16(sq) || !al16(x_copy)) return QMI_E_BAD_STRIDE;
   hipLaunchKernelGGL(square_kernel, dim3(grid_of(rows * (n / 8))), dim3(kThreads), 0, QMI_ST, x,
-                     Rows{rows, stride, (int)heads, (int)n}, sq);
+                     Rows{rows, stride, (int)heads, (int)n}, sq, x_copy, zero);
   QMI_RETURN_LAUNCH_STATUS();
 }
 

@@ -107,9 +107,7 @@ class RMSNorm(nn.Module):
     def _torch(self, x, residual):
         if residual is None:
             if T.norm_ok(x, self.weight):
-                # On a copy, as the formula's x.float() is: a program may write to
-                # x before the backward.
-                return T.RmsNorm.apply(x.clone(), self.weight, self.eps)
+                return T.RmsNorm.apply(x, self.weight, self.eps)
             return T.rms_norm_formula(x, self.weight, self.eps)
         dt = x.dtype
         xf = x.float() + residual.float()

@@ -11,6 +11,14 @@ KV head on the sums of k's and v's gradients over those heads.  The formula
 serves every call the kernels do not take, and a backward that is
 differentiated itself (``create_graph=True``, forward mode) or runs on a batch
 of gradients (vmap) goes through the formula.
+
+The formulas work on fp32 copies of their inputs, so a program may write to an
+input before the backward, and both parts of a second derivative meet in fp32.
+So do the Functions: they save copies that the kernels leave, and each returns,
+beside its result, a *link* per input: zeros of the input's shape in fp32, all
+one element, which the formula of a differentiated backward adds to the saved
+copy.  What flows back to the copy then reaches the same backward, with what
+flows to the result, and is rounded once.
 """
 from __future__ import annotations
 
@@ -25,6 +33,8 @@ from ._lib import check, lib, stream_handle
 HEAD_DIM = K.HEAD_DIM
 F32, BF16 = torch.float32, torch.bfloat16
 _current_device = torch._C._cuda_getDevice
+_is_legacy_batch = torch._C._functorch.is_legacy_batchedtensor
+_is_wrapped = torch._C._functorch.is_functorch_wrapped_tensor
 
 
 def kernels_ok(*tensors: torch.Tensor) -> bool:
@@ -53,33 +63,31 @@ def _has_tangent(t: torch.Tensor) -> bool:
     return forward_ad._current_level >= 0 and forward_ad.unpack_dual(t).tangent is not None
 
 
-def _formula_backward(*tensors: torch.Tensor) -> bool:
-    """Whether a backward on these tensors (the gradient that comes in and the
-    saved ones) goes through the formula: it is differentiated itself
-    (``create_graph=True``, forward mode over it), or its gradient is a batch
-    (``is_grads_batched``, vmap) or another type, which kernels cannot read."""
-    batched = torch._C._functorch
-    return torch.is_grad_enabled() or any(
-        type(t) not in (torch.Tensor, torch.nn.Parameter) or _has_tangent(t)
-        or batched.is_legacy_batchedtensor(t) or batched.is_functorch_wrapped_tensor(t)
-        for t in tensors)
+def _formula_backward(grad, links, *saved) -> bool:
+    """Whether a backward goes through the formula: it is differentiated itself
+    (``create_graph=True``, forward mode over it), has what flowed back to its
+    links, or its gradient is a batch (``is_grads_batched``, vmap) or another
+    type, which kernels cannot read."""
+    if grad is None or torch.is_grad_enabled() or any(d is not None for d in links):
+        return True
+    for t in (grad, *saved):
+        if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter or _has_tangent(t):
+            return True
+    return _is_legacy_batch(grad) or _is_wrapped(grad)
 
 
-def _formula_grads(formula, inputs, needs, grads):
-    """Gradients of ``formula(*inputs)`` that autograd can differentiate again:
-    those of each argument, also where one tensor is passed as several."""
+def _formula_grads(formula, copies, links, needs, grad, link_grads):
+    """bf16 gradients of ``formula`` with respect to the inputs that ``copies``
+    and ``links`` stand for, which autograd can differentiate again."""
     with torch.enable_grad():
-        inputs = [t.view_as(t) for t in inputs]
+        inputs = [link + copy.float() for link, copy in zip(links, copies)]
         out = formula(*inputs)
-    wanted = [t for t, n in zip(inputs, needs) if n]
-    got = iter(torch.autograd.grad(out, wanted, grads, create_graph=torch.is_grad_enabled(),
-                                   allow_unused=True))
-    return tuple(next(got) if n else None for n in needs)
-
-
-def _linked(t: torch.Tensor, copy: torch.Tensor, version: int) -> torch.Tensor:
-    """The values of ``copy`` (``t``'s when it had that version) in ``t``'s graph."""
-    return t if t._version == version else copy + (t - t.detach())
+    got = [None] * len(inputs)
+    if grad is not None:
+        got = torch.autograd.grad(out, inputs, grad, create_graph=torch.is_grad_enabled(),
+                                  allow_unused=True)
+    sums = [d if g is None else g if d is None else g + d for g, d in zip(got, link_grads)]
+    return tuple(g.to(BF16) if n and g is not None else None for g, n in zip(sums, needs))
 
 
 def _no_autocast(backward):
@@ -106,16 +114,18 @@ def _call(name, device, *args):
 # ---------------------------------------------------------------------------
 # RMSNorm (qwen3_naive.py:156-162)
 # ---------------------------------------------------------------------------
-def rms_norm_formula(x, weight, eps):
+def rms_norm_formula(x, weight, eps, dtype=None):
     xf = x.float()
     return (xf * torch.rsqrt(xf.pow(2).mean(dim=-1, keepdim=True) + eps)
-            * weight.float()).to(x.dtype)
+            * weight.float()).to(dtype or x.dtype)
 
 
-def _mean_square(x, rows, stride, heads, n, shape):
-    """``x.float().pow(2).mean(-1, keepdim=True)`` of ``heads`` adjacent rows of ``n`` per row of ``x``."""
+def _mean_square(x, rows, stride, heads, n, shape, x_copy=None, zero=None):
+    """``x.float().pow(2).mean(-1, keepdim=True)`` of ``heads`` adjacent rows of ``n`` per row of
+    ``x``; ``x_copy`` and ``zero`` get a copy of the rows and a zero."""
     sq = torch.empty(shape, dtype=F32, device=x.device)
-    _call("qmi_square_rows", x.device, x.data_ptr(), rows, stride, heads, n, sq.data_ptr())
+    _call("qmi_square_rows", x.device, x.data_ptr(), rows, stride, heads, n, sq.data_ptr(),
+          None if x_copy is None else x_copy.data_ptr(), None if zero is None else zero.data_ptr())
     return sq.mean(dim=-1, keepdim=True)
 
 
@@ -139,39 +149,45 @@ def norm_ok(x, weight) -> bool:
             and x.is_contiguous() and x.data_ptr() % 16 == 0)
 
 
-class RmsNorm(torch.autograd.Function):
-    """``rms_norm_formula``.  The weight may be written to before the backward,
-    which reads a copy that the kernel leaves; ``x`` may not."""
-
+class _RmsNorm(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, eps):
         n = x.shape[-1]
         rows = x.numel() // n
         w = K._dense16(weight)
-        mean = _mean_square(x, rows, n, 1, n, x.shape)
-        y, w_copy = torch.empty_like(x), torch.empty_like(w)
+        x_copy, y, w_copy = torch.empty_like(x), torch.empty_like(x), torch.empty_like(w)
+        zero = torch.empty(1, dtype=F32, device=x.device)
+        mean = _mean_square(x, rows, n, 1, n, x.shape, x_copy, zero)
         _call("qmi_norm_apply", x.device, x.data_ptr(), rows, n, n, mean.data_ptr(), w.data_ptr(),
               eps, y.data_ptr(), w_copy.data_ptr())
-        ctx.save_for_backward(x, w_copy, mean)
-        ctx.weight, ctx.version, ctx.eps = weight, weight._version, eps
-        return y
+        links = zero.expand(x.shape), zero.expand(n)
+        ctx.save_for_backward(x_copy, w_copy, mean, *links)
+        ctx.set_materialize_grads(False)
+        ctx.eps = eps
+        return (y, *links)
 
     @staticmethod
     @_no_autocast
-    def backward(ctx, dy):
-        x, weight, mean = ctx.saved_tensors
+    def backward(ctx, dy, *dlinks):
+        x, weight, mean, *links = ctx.saved_tensors
         need = ctx.needs_input_grad
-        if _formula_backward(dy, x, weight):
-            with torch.enable_grad():
-                weight = _linked(ctx.weight, weight, ctx.version)
-            return (*_formula_grads(lambda x, w: rms_norm_formula(x, w, ctx.eps), (x, weight),
-                                    need[:2], dy), None)
+        if _formula_backward(dy, dlinks, x, weight):
+            return (*_formula_grads(lambda x, w: rms_norm_formula(x, w, ctx.eps, BF16), (x, weight),
+                                    links, need, dy, dlinks), None)
         n = x.shape[-1]
         x, mean = K._dense16(x), K._dense16(mean)  # saved-tensor hooks may have laid them out anew
         dx = torch.empty_like(x)
         dw = _norm_grad(x, x.numel() // n, n, 1, n, x.shape, mean, K._dense16(weight), ctx.eps,
                         K._dense16(dy), dx)
         return dx if need[0] else None, dw if need[1] else None, None
+
+
+class RmsNorm:
+    """``rms_norm_formula`` as an autograd Function."""
+
+    @staticmethod
+    def apply(x, weight, eps):
+        return _RmsNorm.apply(x, weight, eps)[0]
 
 
 # ---------------------------------------------------------------------------
@@ -204,8 +220,11 @@ class SiluMul(torch.autograd.Function):
     @_no_autocast
     def backward(ctx, dy):
         gate_up, = ctx.saved_tensors
-        if _formula_backward(dy, gate_up):
-            return _formula_grads(silu_mul_formula, (gate_up,), ctx.needs_input_grad, dy)
+        if _formula_backward(dy, (), gate_up):
+            with torch.enable_grad():
+                gate_up = gate_up.view_as(gate_up)
+                y = silu_mul_formula(gate_up)
+            return torch.autograd.grad(y, gate_up, dy, create_graph=torch.is_grad_enabled())[0]
         gate_up, dy = K._dense16(gate_up), K._dense16(dy)
         dgu = torch.empty_like(gate_up)
         inter = gate_up.shape[-1] // 2
@@ -228,7 +247,8 @@ def rotate(x: torch.Tensor, positions: torch.Tensor, cache: torch.Tensor) -> tor
     return torch.cat((x1 * c - x2 * s, x2 * c + x1 * s), dim=-1).to(x.dtype)
 
 
-def attention_formula(qkv, norm_q, norm_k, cache, num_heads, num_kv_heads, scale, rotate=rotate):
+def attention_formula(qkv, norm_q, norm_k, cache, num_heads, num_kv_heads, scale, rotate=rotate,
+                      dtype=None):
     """QK-norm, RoPE and causal attention of ``qkv [B, T, (Hq + 2 Hkv) * D]`` ->
     ``[B, T, Hq * D]``; ``norm_q`` / ``norm_k`` map ``[B, T, heads, D]``."""
     batch, seq_len, width = qkv.shape
@@ -250,7 +270,7 @@ def attention_formula(qkv, norm_q, norm_k, cache, num_heads, num_kv_heads, scale
     mask = torch.triu(torch.ones(seq_len, seq_len, device=qkv.device, dtype=torch.bool), 1)
     scores = scores.masked_fill(mask, float("-inf"))
     w = torch.softmax(scores, dim=-1)
-    o = torch.matmul(w, vf).to(qkv.dtype)
+    o = torch.matmul(w, vf).to(dtype or qkv.dtype)
     return o.transpose(1, 2).reshape(batch, seq_len, -1)
 
 
@@ -278,18 +298,14 @@ def attention_ok(qkv, q_weight, k_weight, cache, num_heads, num_kv_heads) -> boo
 SOFTMAX_MAX = 1024
 
 
-class QkvAttention(torch.autograd.Function):
-    """``attention_formula`` with RMS norms of a packed bf16 qkv; the backward
-    writes one packed ``d qkv``.  The norm weights and the cos/sin cache may be
-    written to before the backward, which reads copies that the kernels leave;
-    ``qkv`` may not."""
-
+class _QkvAttention(torch.autograd.Function):
     @staticmethod
     def forward(ctx, qkv, q_weight, k_weight, cache, hq, hkv, eps, scale):
         b, t, width = qkv.shape
         dev, d = qkv.device, HEAD_DIM
         qw, kw = K._dense16(q_weight), K._dense16(k_weight)
-        q_mean = _mean_square(qkv, b * t * hq, width, hq, d, (b, t, hq, d))
+        zero = torch.empty(1, dtype=F32, device=dev)
+        q_mean = _mean_square(qkv, b * t * hq, width, hq, d, (b, t, hq, d), None, zero)
         k_mean = _mean_square(qkv[..., hq * d:], b * t * hkv, width, hkv, d, (b, t, hkv, d))
         qf = torch.empty((b * hq, t, d), dtype=F32, device=dev)
         kt = torch.empty((b * hq, d, t), dtype=F32, device=dev)
@@ -313,27 +329,25 @@ class QkvAttention(torch.autograd.Function):
         o = torch.bmm(w, vf)
         out = torch.empty((b, t, hq * d), dtype=BF16, device=dev)
         _call("qmi_train_heads", dev, o.data_ptr(), out.data_ptr(), b, t, hq, 1)
-        ctx.save_for_backward(qkv, w_copy, cache_copy, q_mean, k_mean, qf, kt, vf, w)
-        ctx.weights = [(p, p._version) for p in (q_weight, k_weight)]
+        links = zero.expand(qkv.shape), zero.expand(d), zero.expand(d)
+        ctx.save_for_backward(qkv, w_copy, cache_copy, q_mean, k_mean, qf, kt, vf, w, *links)
+        ctx.set_materialize_grads(False)
         ctx.args = (hq, hkv, eps, scale)
-        return out
+        return (out, *links)
 
     @staticmethod
     @_no_autocast
-    def backward(ctx, dout):
-        qkv, weights, cache, q_mean, k_mean, qf, kt, vf, w = ctx.saved_tensors
+    def backward(ctx, dout, *dlinks):
+        qkv, weights, cache, q_mean, k_mean, qf, kt, vf, w, *links = ctx.saved_tensors
         hq, hkv, eps, scale = ctx.args
         need = ctx.needs_input_grad
-        if _formula_backward(dout, qkv, weights):
-            with torch.enable_grad():
-                q_weight, k_weight = (_linked(p, c, v) for (p, v), c in zip(ctx.weights, weights))
-
+        if _formula_backward(dout, dlinks, qkv, weights):
             def formula(qkv, q_weight, k_weight):
-                return attention_formula(qkv, lambda a: rms_norm_formula(a, q_weight, eps),
-                                         lambda a: rms_norm_formula(a, k_weight, eps), cache, hq,
-                                         hkv, scale)
-            return (*_formula_grads(formula, (qkv, q_weight, k_weight), need[:3], dout), None, None,
-                    None, None, None)
+                return attention_formula(qkv, lambda a: rms_norm_formula(a, q_weight, eps, BF16),
+                                         lambda a: rms_norm_formula(a, k_weight, eps, BF16), cache,
+                                         hq, hkv, scale, dtype=BF16)
+            return (*_formula_grads(formula, (qkv.detach(), *weights), links, need, dout, dlinks),
+                    None, None, None, None, None)
         qkv, cache, q_mean, k_mean, w, dout = map(K._dense16, (qkv, cache, q_mean, k_mean, w, dout))
         b, t, width = qkv.shape
         dev, d = qkv.device, HEAD_DIM
@@ -363,3 +377,14 @@ class QkvAttention(torch.autograd.Function):
                          dn_k, dqkv[..., hq * d:])
         return (dqkv if need[0] else None, dqw if need[1] else None, dkw if need[2] else None, None,
                 None, None, None, None)
+
+
+class QkvAttention:
+    """``attention_formula`` with RMS norms of a packed bf16 qkv as an autograd
+    Function; the backward writes one packed ``d qkv``.  ``qkv`` itself is saved:
+    the program does not write to it."""
+
+    @staticmethod
+    def apply(qkv, q_weight, k_weight, cache, num_heads, num_kv_heads, eps, scale):
+        return _QkvAttention.apply(qkv, q_weight, k_weight, cache, num_heads, num_kv_heads, eps,
+                                   scale)[0]

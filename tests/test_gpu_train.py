@@ -417,3 +417,16 @@ def test_norm_weight_made_in_inference_mode(pkg, gpu):
     with torch.inference_mode():
         norm.weight = torch.nn.Parameter(norm.weight.clone(), requires_grad=False)
     assert torch.equal(torch.autograd.grad(norm(x).float().square().sum(), x)[0], want)
+
+
+def test_second_derivative_rounds_where_the_formula_does(pkg, T, gpu):
+    """Both parts of a norm's second derivative meet in fp32, as the formula's do:
+    the same bits."""
+    for fused, formula, inputs in _functions(pkg, T, gpu)[:1]:
+        out = []
+        for f in (fused, formula):
+            leaves = [t.detach().clone().requires_grad_() for t in inputs]
+            first = torch.autograd.grad(f(*leaves).float().pow(3).sum(), leaves, create_graph=True)
+            second = torch.autograd.grad(sum(g.float().square().sum() for g in first), leaves)
+            out.append([*first, *second])
+        assert all(torch.equal(a, b) for a, b in zip(*out))

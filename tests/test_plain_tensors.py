@@ -42,9 +42,9 @@ def _backward(T, name):
     x, w = torch.zeros(1, 5, 512, dtype=b16), torch.zeros(512, dtype=b16)
     f = torch.zeros(2, 5, 128)
     cls, saved, out, args = {
-        "norm": (T.RmsNorm, (x, w, torch.zeros(1, 5, 1)), x.shape, {"eps": 1e-6}),
+        "norm": (T._RmsNorm, (x, w, torch.zeros(1, 5, 1)), x.shape, {"eps": 1e-6}),
         "silu": (T.SiluMul, (x,), (1, 5, 256), {}),
-        "attention": (T.QkvAttention, (x, w[:256].view(2, 128), torch.zeros(5, 128), torch.zeros(1, 5, 2, 1),
+        "attention": (T._QkvAttention, (x, w[:256].view(2, 128), torch.zeros(5, 128), torch.zeros(1, 5, 2, 1),
                                        torch.zeros(1, 5, 1, 1), f, f.transpose(1, 2).contiguous(), f,
                                        torch.zeros(2, 5, 5)), (1, 5, 256), {"args": (2, 1, 1e-6, 0.1)}),
     }[name]
