@@ -242,7 +242,7 @@ class Qwen3Attention(nn.Module):
                 and T.attention_ok(qkv, qw, kw, cache, self.num_heads, self.num_kv_heads)):
             # The formula saves copies of qkv, which a hook may have kept and write to.
             proj = self.qkv_proj
-            if (type(proj) is not nn.Linear or proj._forward_hooks
+            if (type(proj) is not nn.Linear or proj._forward_hooks or "forward" in proj.__dict__
                     or nn.modules.module._has_any_global_hook()):
                 qkv = qkv.clone()
             o = T.QkvAttention.apply(qkv, qw, kw, cache, self.num_heads, self.num_kv_heads,
@@ -388,7 +388,8 @@ class Qwen3DecoderLayer(nn.Module):
         attn, mlp, n1, n2 = (sub.get(k) for k in ("self_attn", "mlp", "input_layernorm",
                                                   "post_attention_layernorm"))
         if (type(x) is not torch.Tensor or x.dim() != 2 or x.shape[0] > K.LINEAR_SMALL_ROWS
-                or type(attn) is not Qwen3Attention or type(mlp) is not Qwen3MLP or nn.modules.module._has_any_global_hook()
+                or type(attn) is not Qwen3Attention or type(mlp) is not Qwen3MLP
+                or nn.modules.module._has_any_global_hook()
                 or _decode_methods() != _DECODE_METHODS):
             return False
         for mod in (n1, n2):

@@ -430,3 +430,17 @@ def test_second_derivative_rounds_where_the_formula_does(pkg, T, gpu):
             second = torch.autograd.grad(sum(g.float().square().sum() for g in first), leaves)
             out.append([*first, *second])
         assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
+def test_projection_output_kept_by_its_own_forward(pkg, gpu):
+    """A forward set on the projection may keep what it returned and write to it."""
+    layer = _layer(pkg, gpu)
+    x = torch.randn(1, 9, 128, device=gpu).bfloat16().requires_grad_()
+    want = _grads(layer, layer(x), x)
+    proj, kept = layer.self_attn.qkv_proj, []
+    own = proj.forward
+    proj.forward = lambda z: kept.append(own(z)) or kept[-1]
+    y = layer(x)
+    with torch.no_grad():
+        kept[0].zero_()
+    assert all(torch.equal(a, b) for a, b in zip(_grads(layer, y, x), want))
